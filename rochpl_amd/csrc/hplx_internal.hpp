@@ -18,7 +18,19 @@ namespace hplx {
 // ---------------------------------------------------------------------------
 constexpr int kLeafMax     = 32;    // widest leaf the register-resident kernel takes
 constexpr int kLeafThreads = 512;   // threads per leaf workgroup
-constexpr int kLeafRPT     = 3;     // rows per thread in the leaf kernel
+constexpr int kLeafRPT     = 3;     // rows per thread of the tall leaves
+// Rows per thread of a leaf of R rows: one where at most 512 rows fit one
+// workgroup or 32 workgroups hold them, since the time per column falls with
+// the rows of a thread (500 rows 47 against 67 us, 4000 FP32 88 against 109,
+// 16000 FP64 114 against 119); three for 513 .. 1536 rows, which then need no
+// exchange between workgroups (1500 rows 70 against 78 us), and above 16384
+// rows, where the number of workgroups costs more (48000 rows 131 .. 139 us
+// either way, 131072 155 against 212).
+inline int leaf_rpt(int R) {
+  return R <= kLeafThreads || (R > kLeafThreads * kLeafRPT && R <= 32 * kLeafThreads)
+             ? 1
+             : kLeafRPT;
+}
 
 // Look-ahead: columns a step needs right of the next panel before it overlaps
 // the rest of the update with that panel (fewer go serially), and the CUs

@@ -9,12 +9,12 @@
 //   rows of the right part with the unit lower L11, update the rows below
 //   with one FP64 MFMA GEMM.  Leaves of <= 32 columns run as ONE cooperative
 //   kernel per leaf:
-//     - every workgroup keeps its slice of the leaf (up to 1024 rows x 32
+//     - every workgroup keeps its slice of the leaf (up to 1536 rows x 32
 //       columns) in registers for the whole leaf, so the leaf reads and writes
 //       HBM once;
-//     - the pivot search is a wave64 shuffle max-loc, then a workgroup
-//       max-loc through LDS, then one grid barrier per column after which every
-//       workgroup reduces the published per-workgroup candidates itself;
+//     - the pivot search is a wave64 DPP max-loc, then a workgroup max-loc
+//       through LDS, then one exchange per column after which every workgroup
+//       reduces the published per-workgroup candidates itself;
 //     - no host round-trip: the reference parks its leaf on a pinned-memory
 //       flag once per column and lets a host thread run HPL_pdmxswp
 //       (src/pfact/HPL_pdpanrlT_device.cpp:94-117,455-463);
@@ -214,19 +214,12 @@ __global__ __launch_bounds__(256) void swap_inverse_kernel(
 // ---------------------------------------------------------------------------
 
 template <typename V>
-const void* leaf_entry() {
-  if constexpr(sizeof(V) == 8)
-    return leaf_kernel_ptr<LeafKind::kF64>();
-  else
-    return leaf_kernel_ptr<LeafKind::kF32>();
-}
-
-template <typename V>
 hipError_t launch_leaf(Ctx& c, V* P, int lda, int m, int JB, int c0, int w,
                        int* ipiv, int row_offset, int info_base) {
-  constexpr int CH = kLeafThreads * kLeafRPT;
-  const int     R  = m - c0;
-  const int     G  = (R + CH - 1) / CH;
+  const int R   = m - c0;
+  const int rpt = leaf_rpt(R);
+  const int CH  = kLeafThreads * rpt;
+  const int G   = (R + CH - 1) / CH;
   if(G > kMaxLeafGrid || G < 1 || w < 1 || w > kLeafMax)
     return hipErrorInvalidValue;
   if(G > c.leaf_resident) return hipErrorInvalidValue;
@@ -254,7 +247,6 @@ hipError_t launch_leaf(Ctx& c, V* P, int lda, int m, int JB, int c0, int w,
   la.slots       = c.slots;
   la.seq_base    = c.leaf_launches << 6;
   la.err         = c.flags + 1;
-  la.rows_per_wg = CH;
   la.grid        = G;
   // A plain launch: every workgroup is resident at once because the grid is
   // capped by the occupancy of this kernel (one workgroup per CU) and the
@@ -263,7 +255,7 @@ hipError_t launch_leaf(Ctx& c, V* P, int lda, int m, int JB, int c0, int w,
   // API adds nothing here and refuses to launch while another process holds
   // the device.)
   void* args[] = {&la};
-  return hipLaunchKernel(leaf_entry<V>(), dim3(G), dim3(kLeafThreads), args,
+  return hipLaunchKernel(leaf_kernel_ptr<V>(rpt), dim3(G), dim3(kLeafThreads), args,
                          0, panel_stream(c));
 }
 
@@ -525,15 +517,15 @@ int panel_steps(const PanelAlgo& a0, int jb, int* out, int max_steps) {
 }
 
 hipError_t leaf_occupancy(int* blocks_per_cu) {
-  // the smaller of the FP64 and FP32 leaves' occupancies
-  int        b64 = 0, b32 = 0;
-  hipError_t e   = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &b64, leaf_kernel_ptr<LeafKind::kF64>(), kLeafThreads, 0);
-  if(e != hipSuccess) return e;
-  e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &b32, leaf_kernel_ptr<LeafKind::kF32>(), kLeafThreads, 0);
-  if(e != hipSuccess) return e;
-  *blocks_per_cu = b64 < b32 ? b64 : b32;
+  // the smallest of the leaves' occupancies
+  *blocks_per_cu = INT_MAX;
+  for(const void* f : {leaf_kernel_ptr<double>(1), leaf_kernel_ptr<double>(kLeafRPT),
+                       leaf_kernel_ptr<float>(1), leaf_kernel_ptr<float>(kLeafRPT)}) {
+    int        n = 0;
+    hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, kLeafThreads, 0);
+    if(e != hipSuccess) return e;
+    *blocks_per_cu = n < *blocks_per_cu ? n : *blocks_per_cu;
+  }
   return hipSuccess;
 }
 

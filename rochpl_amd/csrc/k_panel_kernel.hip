@@ -91,7 +91,7 @@ __device__ bool grid_sync(const PkArgs& a, unsigned target, int* ok_sh) {
 }
 
 __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
-  __shared__ leaf::LeafShared sh;
+  __shared__ leaf::LeafShared<double> sh;
   __shared__ double           tt[32][33];  // transpose tile
   __shared__ int              ok_sh;
   HPLX_USLOT(0) HPLX_USLOT(1) HPLX_USLOT(2) HPLX_USLOT(3)
@@ -130,9 +130,8 @@ __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
       la.slots       = a.slots;
       la.seq_base    = (a.leaf_base + leaf_i++) << 6;
       la.err         = a.err;
-      la.rows_per_wg = CH;
-      la.grid        = gl;
-      if(b < gl) leaf::leaf_run<double, double, kLeafRPT>(la, sh);
+          la.grid        = gl;
+      if(b < gl) leaf::leaf_run<double, double, kLeafThreads, kLeafRPT>(la, sh);
     } else if(o.kind == kPanelTrsm) {
       const double* T = a.P + o.ar + static_cast<size_t>(o.ac) * a.lda;
       for(int col = b; col < o.n; col += G)

@@ -4,29 +4,31 @@
 // type T, storage type S) pair: FP64 for the HPL solve, FP32 for the panels
 // of the mixed-precision factorisations.
 //
-// Every workgroup keeps its slice of the leaf (up to 512*RPT rows x 32
-// columns) in registers for the whole leaf.  Per column:
-//   1. each workgroup finds its candidate max |a| (DPP lane exchanges within
-//      a wave, then the 8 waves through LDS);
-//   2. the thread holding the candidate row stores it straight from its
-//      registers into the workgroup's slot (value, row index, 32-wide row);
-//      in workgroup 0 the thread holding the current top row stores it into
-//      the same slot; after a workgroup barrier one thread publishes a
-//      sequence number with release ordering;
-//   3. one wave of every workgroup polls all slots' sequence numbers (each
-//      lane its slots at once) and takes one acquire fence; then every thread
-//      loads a share of all candidate rows (16-byte loads, all in flight
-//      before the first LDS store) and the top row into LDS, and each wave
-//      reduces the candidates itself (no further barrier);
-//   4. registers are updated: row interchange, division by the pivot,
-//      rank-1 update of the remaining leaf columns.
+// Every workgroup keeps its slice of the leaf (NT threads, RPT rows of 32
+// columns each) in registers for the whole leaf.  A row never moves: each carries
+// a label, the row it stands for at the moment, and an interchange swaps two
+// labels.  At the end every row is stored where its label says.  Per column:
+//   1. each workgroup finds its candidate max |a|, ties to the lower label
+//      (DPP lane exchanges within a wave, then the waves through LDS);
+//   2. the wave holding the candidate row stores it into the workgroup's
+//      slot, every 32-bit half of a value in an 8-byte word whose other half
+//      is the column's sequence number, so that a word is complete as soon
+//      as its number is seen: no release, no acquire, no separate flag;
+//   3. the waves read all slots, polling the words themselves, into LDS;
+//      after one workgroup barrier every wave picks the pivot row;
+//   4. labels are swapped, the rows left are divided by the pivot and
+//      updated, the pivot row's values broadcast within the FMA (DPP).  The
+//      pivot row is finished: workgroup 0 keeps it in LDS for the end.
 // Slots are double-buffered by column parity, so a workgroup that runs ahead
 // never overwrites a slot another workgroup still reads.  A grid of one
-// workgroup skips the slots.  The reference instead parks its leaf on a
-// pinned host flag once per column and lets a host thread run HPL_pdmxswp
-// (:94-117,455-463).
+// workgroup passes the row through LDS only.  The reference instead parks
+// its leaf on a pinned host flag once per column and lets a host thread run
+// HPL_pdmxswp (:94-117,455-463).
 //
-// Each column's steps are instantiated per column (static register indices).
+// One column's code is looped over, with static register indices: the tile's
+// first 8 positions rotate by one per column, all 32 by 8 after 8 columns.
+// With all 32 columns instantiated the leaf was bound by instruction fetch
+// (300 KB of code, each instruction run once).
 //
 // Every wait is bounded: after kSpinLimit polls a workgroup raises *err and
 // all workgroups leave the kernel, so a grid that is not co-resident cannot
@@ -34,34 +36,25 @@
 #pragma once
 
 #include <climits>
+#include <type_traits>
 
 #include "hplx_internal.hpp"
+#include "lds_stream.hpp"
 
 namespace hplx {
 namespace leaf {
 
 constexpr uint32_t kSpinLimit = 1u << 22;
-constexpr int      kWaves     = kLeafThreads / 64;
-// slot layout (doubles): [0] |value|, [1] row, [2] sequence, [4..35] the
-// candidate row, [36..67] the top row (workgroup 0's slot only)
-constexpr int kSlotVal = 0, kSlotRow = 1, kSlotSeq = 2, kSlotData = 4,
-              kSlotTop = 36;
-static_assert(kSlotTop + kLeafMax <= kSlotStride, "slot too small");
-
-__device__ inline bool better(double v, int r, double bv, int br) {
-  return v > bv || (v == bv && r < br);
-}
-
-__device__ inline unsigned long long ld_seq(const double* p) {
-  return __hip_atomic_load(
-      reinterpret_cast<unsigned long long*>(const_cast<double*>(p)),
-      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline void st_seq(double* p, unsigned long long v) {
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), v,
-                     __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
+constexpr int      kTurn      = 8;  // columns per turn of the column loop
+// slot layout (8-byte words, sequence number in the upper half): [0..63] the
+// candidate row's 32-bit halves (FP32: [0..31] its values), [64..67] its
+// header: key (upper, lower half), label, the row it was loaded from
+constexpr int kSlotHead = 64;
+static_assert(kSlotHead + 4 <= kSlotStride, "slot too small");
+// Up to kNear workgroups every candidate row is read along with its header
+// (one memory round trip); with more the headers come first and then only
+// the pivot row.
+constexpr int kNear = 32;
 
 struct LeafArgs {
   void*    P;          // panel top-left (panel row 0), storage type S
@@ -74,31 +67,62 @@ struct LeafArgs {
   int      row_offset;
   int*     info;       // first exact zero pivot, 1-based global column
   int      info_base;  // global column of panel column 0
-  double*  slots;      // 2 x (kMaxGrid+1) x kSlotStride
+  double*  slots;      // 2 x (kMaxGrid+1) x kSlotStride 8-byte words
   uint32_t seq_base;   // unique per launch; column j publishes seq_base+j+1
   int*     err;
-  int      rows_per_wg;  // kLeafThreads * RPT
-  int      grid;         // workgroups taking part: 0 .. grid-1 (<= gridDim.x)
+  int      grid;       // workgroups taking part: 0 .. grid-1 (<= gridDim.x)
 };
 
-// Shared-memory scratch of the leaf kernel (the exchange works in double;
-// FP32 rows convert exactly).
+// Shared-memory scratch of the leaf kernel.
+template <typename T>
 struct LeafShared {
-  alignas(16) double cand[kMaxLeafGrid][kLeafMax];  // every workgroup's candidate row
-  double cv[kMaxLeafGrid];
-  int    cr[kMaxLeafGrid];
-  double top[kLeafMax];  // current top row
-  double wv[kWaves];
-  int    wr[kWaves];
-  int    ok;
-  int    piv[kLeafMax];
-  int    lab[kLeafMax];
-  int    ppos[kLeafMax];
-  int    plab[kLeafMax];
-  int    dst[2 * kLeafMax];
-  int    src[2 * kLeafMax];
-  int    np;
+  alignas(16) T cand[kNear][kLeafMax];    // the workgroups' candidate rows
+  alignas(16) T row[2][kLeafMax];         // this workgroup's, by column parity
+  alignas(16) T fin[kLeafMax][kLeafMax];  // workgroup 0: the finished top rows
+  alignas(16) uint32_t head[kNear][4];    // the candidates' headers
+  alignas(16) uint32_t wave[2][16][4];    // the waves' candidates, as headers
+  int sel[2];  // the pivot's label and the row it was loaded from
+  int ok;
 };
+
+// (a, b, c, d) = (b, c, d, a) in place.  In assembly because the compiler,
+// given the moves, keeps a second copy of the tile and spills it.
+__device__ inline void rotate4(double& a, double& b, double& c, double& d) {
+  double t;
+  asm volatile(
+      "v_mov_b64 %4, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2\n\t"
+      "v_mov_b64 %2, %3\n\tv_mov_b64 %3, %4"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "=&v"(t));
+}
+__device__ inline void rotate4(float& a, float& b, float& c, float& d) {
+  float t;
+  asm volatile(
+      "v_mov_b32 %4, %0\n\tv_mov_b32 %0, %1\n\tv_mov_b32 %1, %2\n\t"
+      "v_mov_b32 %2, %3\n\tv_mov_b32 %3, %4"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "=&v"(t));
+}
+
+// (a, ..., h) = (b, ..., h, a) in place.
+__device__ inline void rotate8(double& a, double& b, double& c, double& d, double& e, double& f, double& g,
+                               double& h) {
+  double t;
+  asm volatile(
+      "v_mov_b64 %8, %0\n\tv_mov_b64 %0, %1\n\tv_mov_b64 %1, %2\n\t"
+      "v_mov_b64 %2, %3\n\tv_mov_b64 %3, %4\n\tv_mov_b64 %4, %5\n\t"
+      "v_mov_b64 %5, %6\n\tv_mov_b64 %6, %7\n\tv_mov_b64 %7, %8"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h),
+        "=&v"(t));
+}
+__device__ inline void rotate8(float& a, float& b, float& c, float& d, float& e, float& f, float& g,
+                               float& h) {
+  float t;
+  asm volatile(
+      "v_mov_b32 %8, %0\n\tv_mov_b32 %0, %1\n\tv_mov_b32 %1, %2\n\t"
+      "v_mov_b32 %2, %3\n\tv_mov_b32 %3, %4\n\tv_mov_b32 %4, %5\n\t"
+      "v_mov_b32 %5, %6\n\tv_mov_b32 %6, %7\n\tv_mov_b32 %7, %8"
+      : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f), "+v"(g), "+v"(h),
+        "=&v"(t));
+}
 
 template <typename T, typename S>
 __device__ inline T load_s(const S* p) {
@@ -110,291 +134,667 @@ __device__ inline void store_s(S* p, T v) {
   *p = static_cast<S>(v);
 }
 
-// One step of a wave max-loc: combine (v, r) with the lane that the DPP
-// control CTRL selects (rows outside ROW_MASK keep their value).
+__device__ inline int readlane(int x, int l) {
+  return __builtin_amdgcn_readlane(x, l);
+}
+__device__ inline uint32_t readlane(uint32_t x, int l) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), l));
+}
+__device__ inline double readlane(double x, int l) {
+  return __hiloint2double(readlane(__double2hiint(x), l),
+                          readlane(__double2loint(x), l));
+}
+__device__ inline float readlane(float x, int l) {
+  return __int_as_float(readlane(__float_as_int(x), l));
+}
+
+// The order of the candidates is that of their keys, (upper, lower) half as
+// unsigned numbers, then of their labels, the smaller first.  A row's key is
+// the bit pattern of |a|, the upper half raised by kKeyBase; 0: no row; 1: a
+// NaN in the top row (taken if the column has no number at all, other NaNs
+// never).
+constexpr uint32_t kKeyBase = 2, kKeyTopNan = 1;
+
+__device__ inline uint32_t hi_bits(double x) {
+  return static_cast<uint32_t>(__double2hiint(x));
+}
+__device__ inline uint32_t lo_bits(double x) {
+  return static_cast<uint32_t>(__double2loint(x));
+}
+__device__ inline uint32_t hi_bits(float x) { return __float_as_uint(x); }
+__device__ inline uint32_t lo_bits(float) { return 0; }
+template <typename T>
+constexpr uint32_t kInfBits = sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u;
+
 template <int CTRL, int ROW_MASK>
-__device__ inline void maxloc_dpp(double& v, int& r) {
-  const long long b  = __double_as_longlong(v);
-  const int       lo = static_cast<int>(b), hi = static_cast<int>(b >> 32);
-  const int ol = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xF, false);
-  const int oh = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xF, false);
-  const int orr = __builtin_amdgcn_update_dpp(r, r, CTRL, ROW_MASK, 0xF, false);
-  const double ov = __longlong_as_double(
-      (static_cast<long long>(oh) << 32) | static_cast<unsigned int>(ol));
-  if(better(ov, orr, v, r)) {
-    v = ov;
-    r = orr;
-  }
+__device__ inline uint32_t max_dpp(uint32_t k) {
+  const uint32_t o = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(
+      0, static_cast<int>(k), CTRL, ROW_MASK, 0xF, false));
+  return o > k ? o : k;
 }
 
-// Wave max-loc of (v, r); every lane gets the result.  Within a row of 16
-// lanes: xor 1, xor 2 (quad permutes), half-row and row mirrors; across
-// rows: broadcasts of lane 15 (into rows 1, 3) and lane 31 (into rows 2,
-// 3), leaving the result in lane 63.
-__device__ inline void wave_maxloc(double& v, int& r) {
-  maxloc_dpp<0xB1, 0xF>(v, r);   // quad_perm [1,0,3,2]
-  maxloc_dpp<0x4E, 0xF>(v, r);   // quad_perm [2,3,0,1]
-  maxloc_dpp<0x141, 0xF>(v, r);  // row_half_mirror
-  maxloc_dpp<0x140, 0xF>(v, r);  // row_mirror
-  maxloc_dpp<0x142, 0xA>(v, r);  // row_bcast:15
-  maxloc_dpp<0x143, 0xC>(v, r);  // row_bcast:31
-  const long long b  = __double_as_longlong(v);
-  const int       lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
-  const int       hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), 63);
-  r                  = __builtin_amdgcn_readlane(r, 63);
-  v = __longlong_as_double((static_cast<long long>(hi) << 32) |
-                           static_cast<unsigned int>(lo));
+// Maximum over each row of 16 lanes, in each of them.
+__device__ inline uint32_t row_max(uint32_t k) {
+  k = max_dpp<0xB1, 0xF>(k);      // quad_perm [1,0,3,2]
+  k = max_dpp<0x4E, 0xF>(k);      // quad_perm [2,3,0,1]
+  k = max_dpp<0x141, 0xF>(k);     // row_half_mirror
+  return max_dpp<0x140, 0xF>(k);  // row_mirror
 }
 
-// Workgroup max-loc of (v, r); every thread gets the result.  sh.wv is next
-// written after further barriers of the same column, so none is needed here
-// after the read.
-__device__ inline void block_maxloc(double& v, int& r, LeafShared& sh) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  wave_maxloc(v, r);
-  if(lane == 0) {
-    sh.wv[wave] = v;
-    sh.wr[wave] = r;
-  }
-  __syncthreads();
-  v = sh.wv[0];
-  r = sh.wr[0];
-#pragma unroll
-  for(int k = 1; k < kWaves; ++k)
-    if(better(sh.wv[k], sh.wr[k], v, r)) {
-      v = sh.wv[k];
-      r = sh.wr[k];
+// Maximum over the wave: within a row of 16 lanes by quad permutes and
+// mirrors, across rows by broadcasts of lane 15 (into rows 1 and 3) and lane
+// 31 (into rows 2 and 3).
+__device__ inline uint32_t wave_max(uint32_t k) {
+  k = row_max(k);
+  k = max_dpp<0x142, 0xA>(k);  // row_bcast:15
+  k = max_dpp<0x143, 0xC>(k);  // row_bcast:31
+  return readlane(k, 63);
+}
+
+// Of the lanes in `mask` (not empty; equal upper halves) the first one in the
+// candidates' order, nearly always the only one; of empty candidates (upper
+// half 0) any.
+__device__ inline int first_of(unsigned long long mask, uint32_t hi,
+                               uint32_t lo, int lab) {
+  int best = __builtin_ctzll(mask);
+  mask &= mask - 1;
+  if(mask && hi) {
+    uint32_t bo = readlane(lo, best);
+    int      bl = readlane(lab, best);
+    for(; mask; mask &= mask - 1) {
+      const int      l = __builtin_ctzll(mask), x = readlane(lab, l);
+      const uint32_t o = readlane(lo, l);
+      if(o > bo || (o == bo && x < bl)) {
+        bo   = o;
+        bl   = x;
+        best = l;
+      }
     }
+  }
+  return best;
 }
 
-// Lane l of one wave waits for slots l, l+64, ... (< G) of `slots`, and for
-// `extra` if not null, to show sequence `want`.  All of a lane's slots are
-// read at once on every round, so the wait costs one memory latency once
-// they are published.  False on timeout or error.
-__device__ inline bool poll_slots(const double* slots, int G,
-                                  const double* extra, unsigned long long want,
-                                  int* err) {
-  constexpr int kPer = (kMaxGrid + 63) / 64;
+__device__ inline unsigned long long ld_word(const unsigned long long* p) {
+  return __hip_atomic_load(const_cast<unsigned long long*>(p), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_word(unsigned long long* p, uint32_t seq, uint32_t x) {
+  __hip_atomic_store(p, (static_cast<unsigned long long>(seq) << 32) | x,
+                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Word of a candidate row that a lane carries.
+template <typename T>
+__device__ inline int word_of(int lane) {
+  return sizeof(T) == 8 ? lane : lane & (kLeafMax - 1);
+}
+
+// A wait's poll failed: true when the grid has to stop.
+__device__ inline bool give_up(uint32_t& spins, int* err) {
+  ++spins;
+  if((spins & 255u) == 0 &&
+     __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    return true;
+  if(spins > kSpinLimit) {
+    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+  }
+  __builtin_amdgcn_s_sleep(1);
+  return false;
+}
+
+// Every workgroup's candidate of sequence `seq` into sh.cand / sh.head: wave
+// w of NW takes slots w, w + NW, ..., up to four at a time in flight.  False
+// on timeout or error.
+template <typename T, int NW>
+__device__ __forceinline__ bool gather_all(const LeafArgs& a,
+                                           const unsigned long long* slots,
+                                           uint32_t seq, LeafShared<T>& sh) {
+  constexpr int kBatch = 4;
+  constexpr int kRowWords = kLeafMax * sizeof(T) / 4;
   const int     lane = threadIdx.x & 63;
-  unsigned      pending = extra ? 1u << kPer : 0u;
+  const int     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  uint32_t*     cand = reinterpret_cast<uint32_t*>(&sh.cand[0][0]);
+  uint32_t      spins = 0;
+  for(int g0 = wave; g0 < a.grid; g0 += NW * kBatch) {
+    unsigned pending = 0;
 #pragma unroll
-  for(int q = 0; q < kPer; ++q)
-    if(lane + 64 * q < G) pending |= 1u << q;
-  uint32_t spins = 0;
-  while(pending) {
-    unsigned long long sv[kPer + 1];
+    for(int k = 0; k < kBatch; ++k)
+      if(g0 + k * NW < a.grid) pending |= 1u << k;
+    while(pending) {
+      unsigned long long rw[kBatch], hw[kBatch];
 #pragma unroll
-    for(int q = 0; q < kPer; ++q)
-      if(pending & (1u << q))
-        sv[q] = ld_seq(slots + (lane + 64 * q) * kSlotStride + kSlotSeq);
-    if(pending & (1u << kPer)) sv[kPer] = ld_seq(extra + kSlotSeq);
+      for(int k = 0; k < kBatch; ++k)
+        if(pending & (1u << k)) {
+          const unsigned long long* s = slots + (g0 + k * NW) * kSlotStride;
+          rw[k] = ld_word(s + word_of<T>(lane));
+          hw[k] = ld_word(s + kSlotHead + (lane & 3));
+        }
 #pragma unroll
-    for(int q = 0; q <= kPer; ++q)
-      if((pending & (1u << q)) && sv[q] == want) pending &= ~(1u << q);
-    if(!pending) break;
-    ++spins;
-    if((spins & 255u) == 0 &&
-       __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      return false;
-    if(spins > kSpinLimit) {
-      __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return false;
+      for(int k = 0; k < kBatch; ++k)
+        if(pending & (1u << k)) {
+          const bool in = static_cast<uint32_t>(rw[k] >> 32) == seq &&
+                          static_cast<uint32_t>(hw[k] >> 32) == seq;
+          if(__all(in)) {
+            const int g = g0 + k * NW;
+            cand[g * kRowWords + word_of<T>(lane)] = static_cast<uint32_t>(rw[k]);
+            if(lane < 4) sh.head[g][lane] = static_cast<uint32_t>(hw[k]);
+            pending &= ~(1u << k);
+          }
+        }
+      if(pending && give_up(spins, a.err)) return false;
     }
-    __builtin_amdgcn_s_sleep(1);
   }
   return true;
 }
 
-// Steps 2-3 of a column after the candidate row (and in workgroup 0 the
-// top row) has been stored into this workgroup's slot: publish, wait for
-// every workgroup, load all candidates and the top row, reduce.  Returns
-// the pivot row (sh.cand[its workgroup] holds its segment, sh.top the top
-// row), or -1 if the grid has to stop.
-__device__ __forceinline__ int exchange(const LeafArgs* ap, int jj,
-                                                  LeafShared* shp) {
-  const LeafArgs& a    = *ap;
-  LeafShared&     sh   = *shp;
-  const int       t    = threadIdx.x;
-  const int       lane = t & 63;
-  const int       b    = blockIdx.x;
-  const int       G    = a.grid;
-  const unsigned long long seq =
-      static_cast<unsigned long long>(a.seq_base) + jj + 1;
-  const double* slots = a.slots + static_cast<size_t>(jj & 1) * (kMaxGrid + 1) * kSlotStride;
-  // The workgroup barrier orders every wave's slot stores before thread 0's
-  // release store of the sequence number, so one release per slot (one L2
-  // write-back) publishes them all.
-  __syncthreads();
-  if(t == 0) st_seq(const_cast<double*>(slots) + b * kSlotStride + kSlotSeq, seq);
-  if(t < 64) {
-    const int ok = poll_slots(slots, G, nullptr, seq, a.err);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if(t == 0) sh.ok = ok;
-  }
-  __syncthreads();
-  if(!sh.ok) return -1;
-  if(t < G) {
-    sh.cv[t] = slots[t * kSlotStride + kSlotVal];
-    sh.cr[t] = static_cast<int>(slots[t * kSlotStride + kSlotRow]);
-  } else if(t >= kLeafThreads - kLeafMax) {
-    const int c = t - (kLeafThreads - kLeafMax);
-    sh.top[c]   = slots[kSlotTop + c];
-  }
-  // all candidate rows as 16-byte loads, issued four per thread before
-  // their LDS stores (one memory latency per 128 workgroups)
-  typedef double d2 __attribute__((ext_vector_type(2)));
-  constexpr int kHalf = kLeafMax / 2;
-  for(int i0 = t; i0 < G * kHalf; i0 += 4 * kLeafThreads) {
-    d2 rv[4];
+// The same for many workgroups, on one wave: lane l waits for the headers of
+// slots l, l + 64, ..., the wave picks the pivot and waits for its row
+// (sh.cand[0]; sh.sel its label and own row).
+template <typename T>
+__device__ __forceinline__ bool gather_pivot(const LeafArgs& a,
+                                             const unsigned long long* slots,
+                                             uint32_t seq, LeafShared<T>& sh) {
+  const int lane = threadIdx.x & 63;
+  uint32_t  kh = 0, kl = 0, spins = 0;
+  int       gl = INT_MAX, go = 0, gg = 0;
+  for(int g0 = 0; g0 < a.grid; g0 += 128) {
+    unsigned long long h[2][4];
+    bool               wait[2] = {g0 + lane < a.grid, g0 + 64 + lane < a.grid};
+    while(__any(wait[0] || wait[1])) {
 #pragma unroll
-    for(int k = 0; k < 4; ++k) {
-      const int i = i0 + k * kLeafThreads;
-      if(i < G * kHalf)
-        rv[k] = *reinterpret_cast<const d2*>(
-            &slots[(i / kHalf) * kSlotStride + kSlotData + 2 * (i % kHalf)]);
-    }
+      for(int k = 0; k < 2; ++k)
+        if(wait[k]) {
+          const unsigned long long* s =
+              slots + (g0 + 64 * k + lane) * kSlotStride + kSlotHead;
 #pragma unroll
-    for(int k = 0; k < 4; ++k) {
-      const int i = i0 + k * kLeafThreads;
-      if(i < G * kHalf)
-        *reinterpret_cast<d2*>(&sh.cand[i / kHalf][2 * (i % kHalf)]) = rv[k];
+          for(int i = 0; i < 4; ++i) h[k][i] = ld_word(s + i);
+        }
+      bool late = false;
+#pragma unroll
+      for(int k = 0; k < 2; ++k)
+        if(wait[k]) {
+          bool in = true;
+#pragma unroll
+          for(int i = 0; i < 4; ++i)
+            in = in && static_cast<uint32_t>(h[k][i] >> 32) == seq;
+          wait[k] = !in;
+          late    = late || !in;
+          if(in) {
+            const uint32_t hi = static_cast<uint32_t>(h[k][0]);
+            const uint32_t lo = static_cast<uint32_t>(h[k][1]);
+            const int      l  = static_cast<int>(h[k][2]);
+            if(hi > kh || (hi == kh && (lo > kl || (lo == kl && l < gl)))) {
+              kh = hi;
+              kl = lo;
+              gl = l;
+              go = static_cast<int>(h[k][3]);
+              gg = g0 + 64 * k + lane;
+            }
+          }
+        }
+      if(__any(late) && give_up(spins, a.err)) return false;
     }
   }
-  __syncthreads();
-  // every wave reduces the candidates itself
-  double cv = -1.0;
-  int    cr = INT_MAX;
-  for(int g = lane; g < G; g += 64)
-    if(better(sh.cv[g], sh.cr[g], cv, cr)) {
-      cv = sh.cv[g];
-      cr = sh.cr[g];
+  const uint32_t top = wave_max(kh);
+  const int      w   = first_of(__ballot(kh == top), top, kl, gl);
+  const int      g   = readlane(gg, w);
+  const int      lb = readlane(gl, w), org = readlane(go, w);
+  if(lane == 0) {
+    sh.sel[0] = lb;
+    sh.sel[1] = org;
+  }
+  const unsigned long long* s = slots + g * kSlotStride;
+  for(;;) {
+    const unsigned long long x = ld_word(s + word_of<T>(lane));
+    if(__all(static_cast<uint32_t>(x >> 32) == seq)) {
+      reinterpret_cast<uint32_t*>(&sh.cand[0][0])[word_of<T>(lane)] =
+          static_cast<uint32_t>(x);
+      return true;
     }
-  wave_maxloc(cv, cr);
-  return cr;
+    if(give_up(spins, a.err)) return false;
+  }
 }
 
-// One pivot step for compile-time column JJ: every register of the row tile
-// is addressed statically (no scratch spill).
-template <typename T, int RPT, int JJ>
-__device__ __forceinline__ void leaf_step(const LeafArgs& a,
-                                          T (&v)[RPT][kLeafMax],
-                                          const int (&rows)[RPT],
-                                          LeafShared& sh, bool& alive) {
-  const int t  = threadIdx.x;
-  const int b  = blockIdx.x;
-  const int gc = a.c0 + JJ;  // current top row == current column
-  // ---- step 1: workgroup candidate max |a(r, gc)| over rows r >= gc
-  double bv = -1.0;
-  int    br = INT_MAX;
+// v[POS + i][Q0 + q] += u[POS + i] * nl[Q0 + q] for i = 0 .. 7, q < 1 or 3,
+// u[N] the value that lane N mod 16 of each row of 16 lanes holds.  In assembly for
+// the DPP form of the FMA, which the compiler does not form; the wait states
+// cover a VALU write of u just before.  Every lane of the wave has to be
+// active.
+template <int POS, int Q0>
+__device__ __forceinline__ void fma_group1(double (&v)[kLeafMax][1], double u,
+                                           const double (&nl)[1]) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, %8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, %8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %4, %8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %5, %8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %6, %8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %7, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(v[POS + 0][Q0 + 0]), "+v"(v[POS + 1][Q0 + 0]), "+v"(v[POS + 2][Q0 + 0]), "+v"(v[POS + 3][Q0 + 0]), "+v"(v[POS + 4][Q0 + 0]), "+v"(v[POS + 5][Q0 + 0]), "+v"(v[POS + 6][Q0 + 0]), "+v"(v[POS + 7][Q0 + 0])
+      : "v"(u), "v"(nl[Q0 + 0]), "n"((POS + 0) & 15), "n"((POS + 1) & 15), "n"((POS + 2) & 15), "n"((POS + 3) & 15), "n"((POS + 4) & 15), "n"((POS + 5) & 15), "n"((POS + 6) & 15), "n"((POS + 7) & 15));
+}
+template <int POS, int Q0>
+__device__ __forceinline__ void fma_group1(float (&v)[kLeafMax][1], float u,
+                                           const float (&nl)[1]) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %8, %9 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %8, %9 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %2, %8, %9 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %8, %9 row_newbcast:%13 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %4, %8, %9 row_newbcast:%14 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %5, %8, %9 row_newbcast:%15 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %6, %8, %9 row_newbcast:%16 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %7, %8, %9 row_newbcast:%17 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(v[POS + 0][Q0 + 0]), "+v"(v[POS + 1][Q0 + 0]), "+v"(v[POS + 2][Q0 + 0]), "+v"(v[POS + 3][Q0 + 0]), "+v"(v[POS + 4][Q0 + 0]), "+v"(v[POS + 5][Q0 + 0]), "+v"(v[POS + 6][Q0 + 0]), "+v"(v[POS + 7][Q0 + 0])
+      : "v"(u), "v"(nl[Q0 + 0]), "n"((POS + 0) & 15), "n"((POS + 1) & 15), "n"((POS + 2) & 15), "n"((POS + 3) & 15), "n"((POS + 4) & 15), "n"((POS + 5) & 15), "n"((POS + 6) & 15), "n"((POS + 7) & 15));
+}
+template <int POS, int Q0>
+__device__ __forceinline__ void fma_group3(double (&v)[kLeafMax][3], double u,
+                                           const double (&nl)[3]) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %24, %25 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %24, %26 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, %24, %27 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %3, %24, %25 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %4, %24, %26 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %5, %24, %27 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %6, %24, %25 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %7, %24, %26 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %8, %24, %27 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %9, %24, %25 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %10, %24, %26 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %11, %24, %27 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %12, %24, %25 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %13, %24, %26 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %14, %24, %27 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %15, %24, %25 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %16, %24, %26 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %17, %24, %27 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %18, %24, %25 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %19, %24, %26 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %20, %24, %27 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %21, %24, %25 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %22, %24, %26 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %23, %24, %27 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(v[POS + 0][Q0 + 0]), "+v"(v[POS + 0][Q0 + 1]), "+v"(v[POS + 0][Q0 + 2]), "+v"(v[POS + 1][Q0 + 0]), "+v"(v[POS + 1][Q0 + 1]), "+v"(v[POS + 1][Q0 + 2]), "+v"(v[POS + 2][Q0 + 0]), "+v"(v[POS + 2][Q0 + 1]), "+v"(v[POS + 2][Q0 + 2]), "+v"(v[POS + 3][Q0 + 0]), "+v"(v[POS + 3][Q0 + 1]), "+v"(v[POS + 3][Q0 + 2]), "+v"(v[POS + 4][Q0 + 0]), "+v"(v[POS + 4][Q0 + 1]), "+v"(v[POS + 4][Q0 + 2]), "+v"(v[POS + 5][Q0 + 0]), "+v"(v[POS + 5][Q0 + 1]), "+v"(v[POS + 5][Q0 + 2]), "+v"(v[POS + 6][Q0 + 0]), "+v"(v[POS + 6][Q0 + 1]), "+v"(v[POS + 6][Q0 + 2]), "+v"(v[POS + 7][Q0 + 0]), "+v"(v[POS + 7][Q0 + 1]), "+v"(v[POS + 7][Q0 + 2])
+      : "v"(u), "v"(nl[Q0 + 0]), "v"(nl[Q0 + 1]), "v"(nl[Q0 + 2]), "n"((POS + 0) & 15), "n"((POS + 1) & 15), "n"((POS + 2) & 15), "n"((POS + 3) & 15), "n"((POS + 4) & 15), "n"((POS + 5) & 15), "n"((POS + 6) & 15), "n"((POS + 7) & 15));
+}
+template <int POS, int Q0>
+__device__ __forceinline__ void fma_group3(float (&v)[kLeafMax][3], float u,
+                                           const float (&nl)[3]) {
+  asm("s_nop 1\n\t"
+      "v_fmac_f32_dpp %0, %24, %25 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %24, %26 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %2, %24, %27 row_newbcast:%28 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %3, %24, %25 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %4, %24, %26 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %5, %24, %27 row_newbcast:%29 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %6, %24, %25 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %7, %24, %26 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %8, %24, %27 row_newbcast:%30 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %9, %24, %25 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %10, %24, %26 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %11, %24, %27 row_newbcast:%31 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %12, %24, %25 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %13, %24, %26 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %14, %24, %27 row_newbcast:%32 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %15, %24, %25 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %16, %24, %26 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %17, %24, %27 row_newbcast:%33 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %18, %24, %25 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %19, %24, %26 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %20, %24, %27 row_newbcast:%34 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %21, %24, %25 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %22, %24, %26 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %23, %24, %27 row_newbcast:%35 row_mask:0xf bank_mask:0xf\n\t"
+      : "+v"(v[POS + 0][Q0 + 0]), "+v"(v[POS + 0][Q0 + 1]), "+v"(v[POS + 0][Q0 + 2]), "+v"(v[POS + 1][Q0 + 0]), "+v"(v[POS + 1][Q0 + 1]), "+v"(v[POS + 1][Q0 + 2]), "+v"(v[POS + 2][Q0 + 0]), "+v"(v[POS + 2][Q0 + 1]), "+v"(v[POS + 2][Q0 + 2]), "+v"(v[POS + 3][Q0 + 0]), "+v"(v[POS + 3][Q0 + 1]), "+v"(v[POS + 3][Q0 + 2]), "+v"(v[POS + 4][Q0 + 0]), "+v"(v[POS + 4][Q0 + 1]), "+v"(v[POS + 4][Q0 + 2]), "+v"(v[POS + 5][Q0 + 0]), "+v"(v[POS + 5][Q0 + 1]), "+v"(v[POS + 5][Q0 + 2]), "+v"(v[POS + 6][Q0 + 0]), "+v"(v[POS + 6][Q0 + 1]), "+v"(v[POS + 6][Q0 + 2]), "+v"(v[POS + 7][Q0 + 0]), "+v"(v[POS + 7][Q0 + 1]), "+v"(v[POS + 7][Q0 + 2])
+      : "v"(u), "v"(nl[Q0 + 0]), "v"(nl[Q0 + 1]), "v"(nl[Q0 + 2]), "n"((POS + 0) & 15), "n"((POS + 1) & 15), "n"((POS + 2) & 15), "n"((POS + 3) & 15), "n"((POS + 4) & 15), "n"((POS + 5) & 15), "n"((POS + 6) & 15), "n"((POS + 7) & 15));
+}
+// The same for positions 1 .. 7 of the turn's 8 (u[N] for position N) at
+// step j: positions from 8 - j on hold finished columns and are left alone.
+template <int Q0>
+__device__ __forceinline__ void fma_turn1(double (&v)[kLeafMax][1], double u,
+                                          const double (&nl)[1], int j) {
+  asm("s_nop 1\n\t"
+      "s_cmp_gt_u32 %9, 6\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %0, %7, %8 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 5\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %1, %7, %8 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 4\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %2, %7, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 3\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %3, %7, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 2\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %4, %7, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 1\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %5, %7, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 0\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %6, %7, %8 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      ".Lleaf%=:"
+      : "+v"(v[1][Q0 + 0]), "+v"(v[2][Q0 + 0]), "+v"(v[3][Q0 + 0]), "+v"(v[4][Q0 + 0]), "+v"(v[5][Q0 + 0]), "+v"(v[6][Q0 + 0]), "+v"(v[7][Q0 + 0])
+      : "v"(u), "v"(nl[Q0 + 0]), "s"(j)
+      : "scc");
+}
+template <int Q0>
+__device__ __forceinline__ void fma_turn1(float (&v)[kLeafMax][1], float u,
+                                          const float (&nl)[1], int j) {
+  asm("s_nop 1\n\t"
+      "s_cmp_gt_u32 %9, 6\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %0, %7, %8 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 5\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %1, %7, %8 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 4\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %2, %7, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 3\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %3, %7, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 2\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %4, %7, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 1\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %5, %7, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %9, 0\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %6, %7, %8 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      ".Lleaf%=:"
+      : "+v"(v[1][Q0 + 0]), "+v"(v[2][Q0 + 0]), "+v"(v[3][Q0 + 0]), "+v"(v[4][Q0 + 0]), "+v"(v[5][Q0 + 0]), "+v"(v[6][Q0 + 0]), "+v"(v[7][Q0 + 0])
+      : "v"(u), "v"(nl[Q0 + 0]), "s"(j)
+      : "scc");
+}
+template <int Q0>
+__device__ __forceinline__ void fma_turn3(double (&v)[kLeafMax][3], double u,
+                                          const double (&nl)[3], int j) {
+  asm("s_nop 1\n\t"
+      "s_cmp_gt_u32 %25, 6\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %0, %21, %22 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %21, %23 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %2, %21, %24 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 5\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %3, %21, %22 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %4, %21, %23 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %5, %21, %24 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 4\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %6, %21, %22 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %7, %21, %23 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %8, %21, %24 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 3\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %9, %21, %22 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %10, %21, %23 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %11, %21, %24 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 2\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %12, %21, %22 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %13, %21, %23 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %14, %21, %24 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 1\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %15, %21, %22 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %16, %21, %23 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %17, %21, %24 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 0\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f64_dpp %18, %21, %22 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %19, %21, %23 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %20, %21, %24 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      ".Lleaf%=:"
+      : "+v"(v[1][Q0 + 0]), "+v"(v[1][Q0 + 1]), "+v"(v[1][Q0 + 2]), "+v"(v[2][Q0 + 0]), "+v"(v[2][Q0 + 1]), "+v"(v[2][Q0 + 2]), "+v"(v[3][Q0 + 0]), "+v"(v[3][Q0 + 1]), "+v"(v[3][Q0 + 2]), "+v"(v[4][Q0 + 0]), "+v"(v[4][Q0 + 1]), "+v"(v[4][Q0 + 2]), "+v"(v[5][Q0 + 0]), "+v"(v[5][Q0 + 1]), "+v"(v[5][Q0 + 2]), "+v"(v[6][Q0 + 0]), "+v"(v[6][Q0 + 1]), "+v"(v[6][Q0 + 2]), "+v"(v[7][Q0 + 0]), "+v"(v[7][Q0 + 1]), "+v"(v[7][Q0 + 2])
+      : "v"(u), "v"(nl[Q0 + 0]), "v"(nl[Q0 + 1]), "v"(nl[Q0 + 2]), "s"(j)
+      : "scc");
+}
+template <int Q0>
+__device__ __forceinline__ void fma_turn3(float (&v)[kLeafMax][3], float u,
+                                          const float (&nl)[3], int j) {
+  asm("s_nop 1\n\t"
+      "s_cmp_gt_u32 %25, 6\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %0, %21, %22 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %1, %21, %23 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %2, %21, %24 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 5\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %3, %21, %22 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %4, %21, %23 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %5, %21, %24 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 4\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %6, %21, %22 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %7, %21, %23 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %8, %21, %24 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 3\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %9, %21, %22 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %10, %21, %23 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %11, %21, %24 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 2\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %12, %21, %22 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %13, %21, %23 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %14, %21, %24 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 1\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %15, %21, %22 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %16, %21, %23 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %17, %21, %24 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+      "s_cmp_gt_u32 %25, 0\n\ts_cbranch_scc1 .Lleaf%=\n\t"
+      "v_fmac_f32_dpp %18, %21, %22 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %19, %21, %23 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f32_dpp %20, %21, %24 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+      ".Lleaf%=:"
+      : "+v"(v[1][Q0 + 0]), "+v"(v[1][Q0 + 1]), "+v"(v[1][Q0 + 2]), "+v"(v[2][Q0 + 0]), "+v"(v[2][Q0 + 1]), "+v"(v[2][Q0 + 2]), "+v"(v[3][Q0 + 0]), "+v"(v[3][Q0 + 1]), "+v"(v[3][Q0 + 2]), "+v"(v[4][Q0 + 0]), "+v"(v[4][Q0 + 1]), "+v"(v[4][Q0 + 2]), "+v"(v[5][Q0 + 0]), "+v"(v[5][Q0 + 1]), "+v"(v[5][Q0 + 2]), "+v"(v[6][Q0 + 0]), "+v"(v[6][Q0 + 1]), "+v"(v[6][Q0 + 2]), "+v"(v[7][Q0 + 0]), "+v"(v[7][Q0 + 1]), "+v"(v[7][Q0 + 2])
+      : "v"(u), "v"(nl[Q0 + 0]), "v"(nl[Q0 + 1]), "v"(nl[Q0 + 2]), "s"(j)
+      : "scc");
+}
+
+// Column jb0 + j of the leaf, held in tile position 0 (every register of the
+// tile is addressed statically).  Positions [0, 8 - j) hold the columns from
+// there on and [8 - j, 8) the j columns finished in this turn; [8, act) hold
+// the unfinished columns of the next turns.  lab: the labels of the thread's
+// rows, -1 for a row that is finished or outside the panel, whose registers
+// may then hold anything; msk: 0x7fffffff, 0 for those rows.  dst: lane
+// i >= 32 the label of the row loaded from row c0 + i - 32 (-1 once it is a
+// pivot row); src: lane i < 32 the row that the pivot row of column i was
+// loaded from; piv: lane i < 32 its label then.  False if the grid has to
+// stop.
+struct LeafMoves {
+  int piv, dst, src;
+};
+
+template <typename T, int NT, int RPT>
+__device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RPT],
+                                          int (&lab)[RPT], uint32_t (&msk)[RPT],
+                                          LeafShared<T>& sh, LeafMoves& mv,
+                                          int& zero, int jb0, int j, int act) {
+  constexpr int NW   = NT / 64;
+  const int     t    = threadIdx.x;
+  const int     lane = t & 63;
+  const int     wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int     b    = blockIdx.x;
+  const int     jj   = jb0 + j, par = j & 1;
+  const int     gc   = a.c0 + jj;  // current top row == current column
+  // ---- step 1: candidate max |a(r, gc)| over the labels left, first by the
+  // upper halves alone
+  uint32_t k[RPT], top = 0;
 #pragma unroll
   for(int q = 0; q < RPT; ++q) {
-    if(rows[q] >= gc && rows[q] < a.m) {
-      const double x = fabs(static_cast<double>(v[q][JJ]));
-      if(better(x, rows[q], bv, br)) {
-        bv = x;
-        br = rows[q];
-      }
-    }
+    k[q] = hi_bits(v[0][q]) & msk[q];
+    top  = k[q] > top ? k[q] : top;
   }
-  block_maxloc(bv, br, sh);
-  // ---- steps 2-3
-  int           p;
-  const double* u;
-  if(a.grid == 1) {
+  top = wave_max(top);
+  uint32_t kl = 0;
+  int      kb = INT_MAX, kq = 0, hits = 0;
+  unsigned long long at = 0;
 #pragma unroll
-    for(int q = 0; q < RPT; ++q)
-      if(rows[q] == br) {
-#pragma unroll
-        for(int c = 0; c < kLeafMax; ++c) sh.cand[0][c] = static_cast<double>(v[q][c]);
-      }
-    if(t == JJ) {  // the top row c0 + JJ: workgroup 0, first row set
-#pragma unroll
-      for(int c = 0; c < kLeafMax; ++c) sh.top[c] = static_cast<double>(v[0][c]);
-    }
-    __syncthreads();
-    p = br;
-    u = sh.cand[0];
+  for(int q = RPT - 1; q >= 0; --q) {
+    const bool               is = k[q] == top;
+    const unsigned long long w  = __ballot(is);
+    hits += __builtin_popcountll(w);
+    at |= w;
+    kl = is ? lo_bits(v[0][q]) : kl;
+    kb = is ? lab[q] : kb;
+    kq = is ? q : kq;
+  }
+  int owner;
+  top += kKeyBase;
+  if(hits == 1 && top < kInfBits<T> + kKeyBase) {
+    owner = __builtin_ctzll(at);
   } else {
-    double* slot = a.slots + (static_cast<size_t>(JJ & 1) * (kMaxGrid + 1) + b) * kSlotStride;
+    // ties, an infinity, a NaN, a zero column or no row: the exact order
+    uint32_t kh = 0;
+    kl          = 0;
+    kb          = INT_MAX;
+    kq          = 0;
+#pragma unroll
+    for(int q = 0; q < RPT; ++q) {
+      const T    x   = v[0][q];
+      const bool nan = !(x == x);
+      uint32_t   h   = (hi_bits(x) & 0x7fffffffu) + kKeyBase, l = lo_bits(x);
+      if(nan) {
+        h = lab[q] == gc ? kKeyTopNan : 0;
+        l = 0;
+      }
+      if(lab[q] >= 0 && h > 0 &&
+         (h > kh || (h == kh && (l > kl || (l == kl && lab[q] < kb))))) {
+        kh = h;
+        kl = l;
+        kb = lab[q];
+        kq = q;
+      }
+    }
+    top   = wave_max(kh);
+    owner = first_of(__ballot(kh == top), top, kl, kb);
+  }
+  const uint32_t wlo = readlane(kl, owner);
+  const int      wlb = readlane(kb, owner);
+  kq                 = readlane(kq, owner);
+  if(lane == 0) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<u4*>(sh.wave[par][wave]) =
+        u4{top, wlo, static_cast<uint32_t>(wlb), 0u};
+  }
+  __syncthreads();
+  // sh.wave of this parity is written again two barriers on
+  const uint32_t ch = sh.wave[par][lane & (NW - 1)][0];
+  const uint32_t cl = sh.wave[par][lane & (NW - 1)][1];
+  const int      cb = static_cast<int>(sh.wave[par][lane & (NW - 1)][2]);
+  top               = readlane(row_max(ch), 0);
+  const int ww = first_of(__ballot(ch == top) & ((1u << NW) - 1), top, cl, cb);
+  const int lb = readlane(cb, ww);
+  // the row that workgroup candidate was loaded from
+  const int CH  = NT * RPT;
+  int       org = a.c0 + b * CH + kq * NT + wave * 64 + owner;
+  // ---- the candidate row, by its wave
+  if(wave == ww && lb != INT_MAX && lane == owner) {
 #pragma unroll
     for(int q = 0; q < RPT; ++q)
-      if(rows[q] == br) {
+      if(kq == q) {
 #pragma unroll
-        for(int c = 0; c < kLeafMax; ++c) slot[kSlotData + c] = static_cast<double>(v[q][c]);
+        for(int c = 0; c < kLeafMax; ++c) sh.row[par][c] = v[c][q];
+        // keeps the cases apart: merged, they would index the tile by kq
+        asm volatile("; row %0" : : "n"(q));
       }
-    if(t == 0) {
-      slot[kSlotVal] = bv;
-      slot[kSlotRow] = static_cast<double>(br);
+    if(a.grid == 1) {
+      sh.sel[0] = lb;
+      sh.sel[1] = org;
     }
-    if(b == 0 && t == JJ) {  // the top row c0 + JJ
-#pragma unroll
-      for(int c = 0; c < kLeafMax; ++c) slot[kSlotTop + c] = static_cast<double>(v[0][c]);
-    }
-    p = exchange(&a, JJ, &sh);
-    if(p < 0) {
-      alive = false;
-      return;
-    }
-    u = sh.cand[(p - a.c0) / a.rows_per_wg];
   }
-  if(t == 0) sh.piv[JJ] = p;
-  const T piv = static_cast<T>(u[JJ]);
-  if(b == 0 && t == 0) {
-    a.ipiv[gc] = p + a.row_offset;
-    if(piv == T(0) && *a.info == 0) *a.info = a.info_base + gc + 1;
+  int      p, po;  // the pivot's label, the row it was loaded from
+  const T* urow;
+  if(a.grid == 1) {
+    __syncthreads();
+    p    = sh.sel[0];
+    po   = sh.sel[1];
+    urow = sh.row[par];
+  } else {
+    // ---- steps 2-3.  A workgroup without rows left publishes an empty
+    // candidate (key 0, label INT_MAX).
+    const uint32_t      seq  = a.seq_base + jj + 1;
+    unsigned long long* slots =
+        reinterpret_cast<unsigned long long*>(a.slots) +
+        static_cast<size_t>(par) * (kMaxGrid + 1) * kSlotStride;
+    unsigned long long* mine = slots + b * kSlotStride;
+    if(wave == ww) {
+      // the wave's lanes see its own LDS stores in order
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const uint32_t* half = reinterpret_cast<const uint32_t*>(sh.row[par]);
+      st_word(mine + word_of<T>(lane), seq, half[word_of<T>(lane)]);
+      if(lane < 4)
+        st_word(mine + kSlotHead + lane, seq,
+                lane == 0   ? top
+                : lane == 1 ? wlo
+                            : static_cast<uint32_t>(lane == 2 ? lb : org));
+    }
+    const bool near = a.grid <= kNear;
+    if(near ? !gather_all<T, NW>(a, slots, seq, sh)
+            : wave == 0 && !gather_pivot<T>(a, slots, seq, sh))
+      sh.ok = 0;
+    __syncthreads();
+    if(!sh.ok) return false;
+    if(near) {  // every wave picks the pivot itself
+      uint32_t gh = 0, go = 0;
+      int      gl = INT_MAX;
+      if(lane < a.grid) {
+        gh = sh.head[lane][0];
+        go = sh.head[lane][1];
+        gl = static_cast<int>(sh.head[lane][2]);
+      }
+      top         = wave_max(gh);
+      const int g = first_of(__ballot(gh == top) & ((1ull << a.grid) - 1), top, go, gl);
+      p           = readlane(gl, g);
+      po          = static_cast<int>(sh.head[g][3]);
+      urow        = sh.cand[g];
+    } else {
+      p    = sh.sel[0];
+      po   = sh.sel[1];
+      urow = sh.cand[0];
+    }
   }
-  // ---- step 4: interchange rows gc and p, scale, rank-1 update
+  p  = __builtin_amdgcn_readfirstlane(p);
+  po = __builtin_amdgcn_readfirstlane(po);
+  // u0 / u1: the pivot row's positions 0..15 / 16..31, in every 16 lanes
+  const T u0 = urow[lane & 15], u1 = urow[16 + (lane & 15)];
+  const T piv = readlane(u0, 0);
+  if(b == 0 && t < kLeafMax)
+    sh.fin[jj][t < kTurn ? jb0 + ((t + j) & (kTurn - 1))
+                         : (t + jb0) & (kLeafMax - 1)] = urow[t];
+  if(piv == T(0) && zero < 0) zero = jj;
+  // ---- step 4: interchange rows gc and p (the pivot row is finished),
+  // scale, rank-1 update
+  mv.piv = lane == jj ? p : mv.piv;
+  mv.src = lane == jj ? po : mv.src;
+  mv.dst = mv.dst == p ? -1 : mv.dst == gc ? p : mv.dst;
+  T nl[RPT];
 #pragma unroll
   for(int q = 0; q < RPT; ++q) {
-    if(rows[q] == gc) {
-#pragma unroll
-      for(int c = 0; c < kLeafMax; ++c) v[q][c] = static_cast<T>(u[c]);
-    } else if(rows[q] == p) {
-#pragma unroll
-      for(int c = 0; c < kLeafMax; ++c) v[q][c] = static_cast<T>(sh.top[c]);
-    }
+    if(lab[q] == p) msk[q] = 0;
+    lab[q] = lab[q] == p ? -1 : lab[q] == gc ? p : lab[q];
+    if(piv != T(0)) v[0][q] = v[0][q] / piv;
+    nl[q] = -v[0][q];
   }
-#pragma unroll
-  for(int q = 0; q < RPT; ++q) {
-    if(rows[q] > gc && rows[q] < a.m) {
-      T l = v[q][JJ];
-      if(piv != T(0)) l = l / piv;
-      v[q][JJ] = l;
-#pragma unroll
-      for(int c = JJ + 1; c < kLeafMax; ++c)
-        v[q][c] = fma(-l, static_cast<T>(u[c]), v[q][c]);
-    }
+  if constexpr(RPT == 1) {
+    fma_turn1<0>(v, u0, nl, j);
+    if(act > 8) fma_group1<8, 0>(v, u0, nl);
+    if(act > 16) fma_group1<16, 0>(v, u1, nl);
+    if(act > 24) fma_group1<24, 0>(v, u1, nl);
+  } else {
+    fma_turn3<0>(v, u0, nl, j);
+    if(act > 8) fma_group3<8, 0>(v, u0, nl);
+    if(act > 16) fma_group3<16, 0>(v, u1, nl);
+    if(act > 24) fma_group3<24, 0>(v, u1, nl);
   }
-  // sh.cand / sh.top are rewritten next column only after the barrier in
-  // its block_maxloc, which every wave reaches after this update
+  // sh.cand / sh.row are rewritten only after later barriers, which every
+  // wave reaches after its reads here
+  return true;
 }
 
-template <typename T, int RPT, int JJ>
-struct LeafSteps {
-  __device__ __forceinline__ static void run(const LeafArgs& a,
-                                             T (&v)[RPT][kLeafMax],
-                                             const int (&rows)[RPT],
-                                             LeafShared& sh, bool& alive) {
-    if(JJ < a.w && alive) leaf_step<T, RPT, JJ>(a, v, rows, sh, alive);
-    LeafSteps<T, RPT, JJ + 1>::run(a, v, rows, sh, alive);
-  }
-};
-
+// The turn's positions 0 .. 7 rotated by one.
 template <typename T, int RPT>
-struct LeafSteps<T, RPT, kLeafMax> {
-  __device__ __forceinline__ static void run(const LeafArgs&,
-                                             T (&)[RPT][kLeafMax],
-                                             const int (&)[RPT], LeafShared&,
-                                             bool&) {}
-};
+__device__ __forceinline__ void rotate_turn(T (&v)[kLeafMax][RPT]) {
+#pragma unroll
+  for(int q = 0; q < RPT; ++q)
+    rotate8(v[0][q], v[1][q], v[2][q], v[3][q], v[4][q],
+            v[5][q], v[6][q], v[7][q]);
+}
 
-// One leaf on workgroups 0 .. a.grid-1: the body of leaf_kernel, also run
-// by the persistent panel kernel (k_panel_kernel.hip) once per leaf.
-// Workgroups whose rows all lie at or below a.m take part in every exchange
-// with an empty candidate.
-template <typename T, typename S, int RPT>
-__device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared& sh) {
-  constexpr int CH   = kLeafThreads * RPT;  // rows per workgroup
+// One leaf on workgroups 0 .. a.grid-1 of NT threads, RPT rows each: the
+// body of leaf_kernel, also run by the persistent panel kernel
+// (k_panel_kernel.hip) once per leaf.  Workgroups whose rows all lie at or
+// below a.m take part in every exchange with an empty candidate.
+template <typename T, typename S, int NT, int RPT>
+__device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared<T>& sh) {
+  constexpr int NW   = NT / 64;
+  constexpr int CH   = NT * RPT;  // rows per workgroup
   const int     t    = threadIdx.x;
   const int     lane = t & 63;
   const int     wave = t >> 6;
@@ -402,93 +802,94 @@ __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared& sh) {
   const int     G    = a.grid;
   S*            P    = static_cast<S*>(a.P);
 
-  int rows[RPT];
-  T   v[RPT][kLeafMax];
+  int          lab[RPT];  // the row each slot stands for; -1: none
+  uint32_t     msk[RPT];
+  T            v[kLeafMax][RPT];
 #pragma unroll
-  for(int q = 0; q < RPT; ++q) rows[q] = a.c0 + b * CH + q * kLeafThreads + t;
+  for(int q = 0; q < RPT; ++q) {
+    const int row = a.c0 + b * CH + q * NT + t;
+    lab[q]        = row < a.m ? row : -1;
+    msk[q]        = row < a.m ? 0x7fffffffu : 0u;
+  }
 #pragma unroll
   for(int c = 0; c < kLeafMax; ++c) {
     const S* col = P + static_cast<size_t>(a.c0 + c) * a.lda;
 #pragma unroll
     for(int q = 0; q < RPT; ++q)
-      v[q][c] = (c < a.w && rows[q] < a.m) ? load_s<T, S>(col + rows[q]) : T(0);
+      v[c][q] = (c < a.w && lab[q] >= 0)
+                       ? load_s<T, S>(col + static_cast<unsigned>(lab[q]))
+                       : T(0);
   }
+  if(t == 0) sh.ok = 1;
+  // every row has been read before any candidate of it is published, and so
+  // before any workgroup stores a row
+  wait_vm<0>();
 
-  bool alive = true;
-  LeafSteps<T, RPT, 0>::run(a, v, rows, sh, alive);
-  if(!alive) return;
-
-  // ---- write the leaf back
+  LeafMoves mv;
+  mv.piv   = 0;
+  mv.src   = a.c0 + (lane & (kLeafMax - 1));
+  mv.dst   = lane < kLeafMax ? -2 : mv.src;
+  int zero = -1;  // the first column with a zero pivot
+  int jb0  = 0;
+#pragma unroll 1
+  for(; jb0 < a.w; jb0 += kTurn) {
+    const int act  = (a.w + kTurn - 1) / kTurn * kTurn - jb0;
+    const int turn = a.w - jb0 < kTurn ? a.w - jb0 : kTurn;
+#pragma unroll 1
+    for(int j = 0; j < kTurn; ++j) {
+      if(j < turn && !leaf_step<T, NT, RPT>(a, v, lab, msk, sh, mv, zero, jb0, j, act))
+        return;
+      rotate_turn(v);
+    }
+    // the next columns come to the front, the finished ones go to the end
 #pragma unroll
-  for(int c = 0; c < kLeafMax; ++c) {
-    if(c < a.w) {
-      S* col = P + static_cast<size_t>(a.c0 + c) * a.lda;
+    for(int i = 0; i < kTurn; ++i)
 #pragma unroll
       for(int q = 0; q < RPT; ++q)
-        if(rows[q] < a.m) store_s<T, S>(col + rows[q], v[q][c]);
-    }
+        rotate4(v[i][q], v[i + 8][q], v[i + 16][q], v[i + 24][q]);
   }
 
-  // ---- compose the w interchanges and apply them to the other panel columns
-  if(t == 0) {
-    const int top_end = a.c0 + a.w;
-    int       nout    = 0;
-    for(int i = 0; i < a.w; ++i) sh.lab[i] = a.c0 + i;
-    for(int jj = 0; jj < a.w; ++jj) {
-      const int p = sh.piv[jj];
-      if(p < top_end) {
-        const int x      = sh.lab[jj];
-        sh.lab[jj]       = sh.lab[p - a.c0];
-        sh.lab[p - a.c0] = x;
-      } else {
-        int s = -1;
-        for(int k = 0; k < nout; ++k)
-          if(sh.ppos[k] == p) {
-            s = k;
-            break;
-          }
-        if(s < 0) {
-          s          = nout++;
-          sh.ppos[s] = p;
-          sh.plab[s] = p;
-        }
-        const int x = sh.lab[jj];
-        sh.lab[jj]  = sh.plab[s];
-        sh.plab[s]  = x;
-      }
+  // ---- write the leaf back: the rows below where their labels say, the
+  // finished top rows by workgroup 0
+#pragma unroll
+  for(int c = 0; c < kLeafMax; ++c) {
+    const int cc = (c + jb0) & (kLeafMax - 1);  // the column position c holds
+    if(cc < a.w) {
+      S* col = P + static_cast<size_t>(a.c0 + cc) * a.lda;
+#pragma unroll
+      for(int q = 0; q < RPT; ++q)
+        if(lab[q] >= 0)
+          store_s<T, S>(col + static_cast<unsigned>(lab[q]), v[c][q]);
     }
-    int np = 0;
-    for(int i = 0; i < a.w; ++i)
-      if(sh.lab[i] != a.c0 + i) {
-        sh.dst[np] = a.c0 + i;
-        sh.src[np] = sh.lab[i];
-        ++np;
-      }
-    for(int k = 0; k < nout; ++k)
-      if(sh.plab[k] != sh.ppos[k]) {
-        sh.dst[np] = sh.ppos[k];
-        sh.src[np] = sh.plab[k];
-        ++np;
-      }
-    sh.np = np;
   }
-  __syncthreads();
-  const int np     = sh.np;
+  if(b == 0) {
+    __syncthreads();  // sh.fin
+    const int r = t & (kLeafMax - 1);
+    if(r < a.w)
+      for(int c = t / kLeafMax; c < a.w; c += NT / kLeafMax)
+        store_s<T, S>(P + a.c0 + r + static_cast<size_t>(a.c0 + c) * a.lda,
+                      sh.fin[r][c]);
+    if(t < a.w) a.ipiv[a.c0 + t] = mv.piv + a.row_offset;
+    if(t == 0 && zero >= 0 && *a.info == 0)
+      *a.info = a.info_base + a.c0 + zero + 1;
+  }
+
+  // ---- apply the leaf's moves to the other panel columns
   const int others = a.JB - a.w;
-  if(np > 0 && lane < np) {
+  const int dst    = lane < kLeafMax ? a.c0 + lane : mv.dst;
+  if(dst >= 0 && dst != mv.src) {
     // a wave takes columns idx, idx + stride, ...; each column's sources are
     // all loaded (one instruction) before any of its destinations is stored,
     // and kBatch columns are in flight at once
     constexpr int kBatch = 8;
-    const int     stride = G * kWaves;
-    const int     src = sh.src[lane], dst = sh.dst[lane];
-    for(int idx0 = b * kWaves + wave; idx0 < others; idx0 += kBatch * stride) {
+    const int     stride = G * NW;
+    for(int idx0 = b * NW + wave; idx0 < others; idx0 += kBatch * stride) {
       S x[kBatch];
 #pragma unroll
       for(int u = 0; u < kBatch; ++u) {
         const int idx = idx0 + u * stride;
         const int c   = idx < a.c0 ? idx : idx + a.w;
-        if(idx < others) x[u] = P[src + static_cast<size_t>(c) * a.lda];
+        if(idx < others) x[u] = P[mv.src + static_cast<size_t>(c) * a.lda];
       }
 #pragma unroll
       for(int u = 0; u < kBatch; ++u) {
@@ -500,19 +901,26 @@ __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared& sh) {
   }
 }
 
-template <typename T, typename S, int RPT>
-__global__ __launch_bounds__(kLeafThreads) void leaf_kernel(LeafArgs a) {
-  __shared__ LeafShared sh;
+// Bound by latency: per column one workgroup-wide and one grid-wide exchange
+// and the issue of about 150 (one row per thread) or 290 instructions; HBM
+// traffic is one read and one write of the leaf.  Time of a 32-column leaf of
+// m rows, FP64 (FP32), before this form and now:
+//   m = 500 131 (128) -> 47 (42) us, 1500 160 (158) -> 70 (62),
+//   4000 222 (216) -> 102 (88), 16000 246 (239) -> 114 (105),
+//   65000 276 (270) -> 134 (127), 131072 318 (320) -> 155 (150).
+template <typename T, typename S, int NT, int RPT>
+__global__ __launch_bounds__(NT) void leaf_kernel(LeafArgs a) {
+  __shared__ LeafShared<T> sh;
   if(__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     return;
-  leaf_run<T, S, RPT>(a, sh);
+  leaf_run<T, S, NT, RPT>(a, sh);
 }
 
 }  // namespace leaf
 
-// Kernel entry of one variant (defined in k_leaf*.hip): FP64, or FP32.
-enum class LeafKind { kF64, kF32 };
-template <LeafKind K>
-const void* leaf_kernel_ptr();
+// Kernel entry of the FP64 or FP32 leaf with rpt (1 or kLeafRPT) rows per
+// thread (defined in k_leaf*.hip).
+template <typename T>
+const void* leaf_kernel_ptr(int rpt);
 
 }  // namespace hplx
