@@ -200,9 +200,9 @@ int hplx_pdgetrf(hplx_ctx* ctx, const hplx_palg* palg, hplx_pmat* mat);
  * solves A X = B, trans = 1 solves A^T X = B, for nrhs columns of B (device,
  * ldb >= n) in place.  The L solve applies each panel's interchanges the way
  * HPL_pdgesv carries b through the factorisation (HPL's L is left unpivoted
- * by later panels); the U solve is HPL_pdtrsv's.  No allocation: the
- * transposed solve keeps split-K partial sums in the context's own panel
- * buffers, so calls on one context must not overlap. */
+ * by later panels).  No allocation: the exchange buffers and
+ * partial sums live in the context's own panel buffers, so calls on one
+ * context must not overlap. */
 int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
                  double* B, int ldb);
 
@@ -212,11 +212,11 @@ int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
  * hplx_pdgetrs, queued on `stream` (a hipStream_t of the current device;
  * NULL = its null stream) in the same order, so the result is bit-identical;
  * nothing is allocated and nothing is synchronised (the caller waits on the
- * stream).  Scratch: one file-scope device array of 8 MiB + 8 KiB per
+ * stream).  Scratch: one file-scope device array of 16 MiB + 136 KiB per
  * device, reserved when the library's code object loads and held until the
  * process ends; every call on a device shares it, so calls that overlap on
  * one device (on different streams, or from several threads) race.
- * mat->nb above 1024 (the scratch's pivot slots) returns
+ * mat->nb above 1024 (what the scratch is laid out for) returns
  * HPLX_ERR_UNSUPPORTED; bad arguments HPLX_ERR_INVALID; a launch failure
  * HPLX_ERR_HIP (no error string: there is no context to hold one). */
 int hplx_pdgetrs_noalloc(const hplx_pmat* mat, int trans, int nrhs, double* B,

@@ -87,90 +87,17 @@ int cu_sets(Ctx& c, int* census_dev) {
 
 }  // namespace
 
-namespace hplx {
+namespace {
 
-// The solve with the factors of a pmat (hplx_pdgetrs), queued on s with the
-// given scratch: permU (2 kMaxNB ints) and the split-K partial products of
-// the transposed solve (work_doubles doubles; fewer only means fewer
-// splits).  No synchronisation, no allocation.
-hipError_t getrs_enqueue(hipStream_t s, const double* A, int N, int nb,
-                         int lda, const int* ipiv, int trans, int nrhs,
-                         double* B, int ldb, int* permU, double* work,
-                         size_t work_doubles) {
-#define HCHK(expr)                    \
-  do {                                \
-    const hipError_t e_ = (expr);     \
-    if(e_ != hipSuccess) return e_;   \
-  } while(0)
-  const int    np = (N + nb - 1) / nb;
-  // C (m x nrhs, ldb) -= Ablk (m x jb, lda) * Y (jb x nrhs, ldb) on FP64 MFMA
-  auto sub_product = [&](int m, int jb, const double* Ablk, const double* Y,
-                         double* Cblk) -> hipError_t {
-    return hplx::launch_nn_sub(s, jb, m, nrhs, Ablk, lda, Y, ldb, Cblk, ldb);
-  };
-  if(!trans) {
-    // L solve with the panel-by-panel interchanges, as b is carried through
-    // the factorisation (HPL_pdgesv), then U x = y (HPL_pdtrsv)
-    for(int p = 0; p < np; ++p) {
-      const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb;
-      HCHK(hplx::launch_pipid(s, jb, ipiv + j, j, permU));
-      HCHK(hplx::launch_swap_inplace(s, jb, nrhs, B + j, ldb, permU));
-      HCHK(hplx::launch_tri_solve(s, true, false, true, jb, nrhs,
-                                  A + j + static_cast<size_t>(j) * lda,
-                                  lda, B + j, ldb));
-      if(N - j - jb > 0)
-        HCHK(sub_product(N - j - jb, jb,
-                              A + j + jb + static_cast<size_t>(j) * lda, B + j,
-                              B + j + jb));
-    }
-    for(int p = np - 1; p >= 0; --p) {
-      const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb;
-      HCHK(hplx::launch_tri_solve(s, false, false, false, jb, nrhs,
-                                  A + j + static_cast<size_t>(j) * lda,
-                                  lda, B + j, ldb));
-      if(j > 0)
-        HCHK(sub_product(j, jb, A + static_cast<size_t>(j) * lda, B + j,
-                              B));
-    }
-  } else {
-    // A = P0^T L0 P1^T L1 ... U  =>  A^T z = g  is solved as
-    // w = U^{-T} g, then for panels from the last: z_p -= L21^T z_below,
-    // z_p = L11^{-T} z_p, z = P_p^T z.
-    for(int p = 0; p < np; ++p) {
-      const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb, e = j + jb;
-      HCHK(hplx::launch_tri_solve(s, true, true, false, jb, nrhs,
-                                  A + j + static_cast<size_t>(j) * lda,
-                                  lda, B + j, ldb));
-      // z_below -= U12^T z_p (U12 = rows j..e of the columns right of the
-      // panel)
-      if(e < N)
-        HCHK(hplx::launch_tn_sub(s, jb, N - e, nrhs,
-                                 A + j + static_cast<size_t>(e) * lda,
-                                 lda, B + j, ldb, B + e, ldb, work,
-                                 work_doubles));
-    }
-    // z_p -= L21^T z_below reduces over all N - e rows below the panel for
-    // a jb x nrhs result: split over K, the partials in the work buffer,
-    // while they fit
-    for(int p = np - 1; p >= 0; --p) {
-      const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb, e = j + jb;
-      if(e < N)
-        HCHK(hplx::launch_tn_sub(s, N - e, jb, nrhs,
-                                 A + e + static_cast<size_t>(j) * lda,
-                                 lda, B + e, ldb, B + j, ldb, work,
-                                 work_doubles));
-      HCHK(hplx::launch_tri_solve(s, false, true, true, jb, nrhs,
-                                  A + j + static_cast<size_t>(j) * lda,
-                                  lda, B + j, ldb));
-      HCHK(hplx::launch_pipid(s, jb, ipiv + j, j, permU));
-      HCHK(hplx::launch_swap_inverse(s, jb, nrhs, B + j, ldb, permU));
-    }
-  }
-#undef HCHK
-  return hipSuccess;
+// The context's buffers as the solves' scratch (the L11^{-1} buffers are idle
+// outside the panel loops).
+hplx::FlowScratch flow_scratch(const Ctx& c) {
+  return {c.flow_x, c.Linv,
+          static_cast<size_t>(hplx::kMaxNB) * hplx::kMaxNB, c.flow_perm,
+          c.flow_flags};
 }
 
-}  // namespace hplx
+}  // namespace
 
 extern "C" {
 
@@ -243,7 +170,10 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   size_t off_dout   = off_flags + 256;
   size_t off_linv2  = align_up(off_dout + 256, 256);
   size_t off_perm2  = align_up(off_linv2 + nLinv, 256);
-  size_t off_claim  = align_up(off_perm2 + nperm, 256);
+  size_t off_fperm  = align_up(off_perm2 + nperm, 256);
+  size_t off_fx     = align_up(off_fperm + hplx::kFlowPerm * sizeof(int), 256);
+  size_t off_fflags = align_up(off_fx + hplx::kFlowX * sizeof(double), 256);
+  size_t off_claim  = align_up(off_fflags + hplx::kFlowFlags * sizeof(int), 256);
   size_t off_stop   = align_up(off_claim + 2 * hplx::kClaimInts * sizeof(int), 256);
   size_t off_vacate = off_stop + 256;
   size_t off_census = align_up(off_vacate + hplx::kVacateSets * 8 * 8, 256);
@@ -271,6 +201,9 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   c.dout    = reinterpret_cast<double*>(b + off_dout);
   c.Linv2   = reinterpret_cast<double*>(b + off_linv2);
   c.permU2  = reinterpret_cast<int*>(b + off_perm2);
+  c.flow_perm  = reinterpret_cast<int*>(b + off_fperm);
+  c.flow_flags = reinterpret_cast<int*>(b + off_fflags);
+  c.flow_x     = reinterpret_cast<unsigned long long*>(b + off_fx);
   c.claim   = reinterpret_cast<int*>(b + off_claim);
   c.stop    = reinterpret_cast<int*>(b + off_stop);
   c.vacate  = reinterpret_cast<unsigned long long*>(b + off_vacate);
@@ -772,7 +705,7 @@ int hplx_pdgesv(hplx_ctx* ctx, const hplx_palg* palg, hplx_pmat* mat) {
   HIPCHK(c, hipMemcpyAsync(mat->X, mat->A + static_cast<size_t>(N) * mat->ld,
                            static_cast<size_t>(N) * sizeof(double),
                            hipMemcpyDeviceToDevice, s));
-  HIPCHK(c, hplx::launch_trsv(s, N, mat->nb, mat->A, mat->ld, mat->X));
+  HIPCHK(c, hplx::launch_trsv(s, N, mat->A, mat->ld, mat->X, flow_scratch(c)));
   HIPCHK(c, hipStreamSynchronize(s));
   return HPLX_SUCCESS;
 }
@@ -793,8 +726,7 @@ int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
     return fail(c, HPLX_ERR_INVALID, "pdgetrs: bad arguments");
   if(nrhs == 0) return HPLX_SUCCESS;
   HIPCHK(c, hplx::getrs_enqueue(c.stream, mat->A, mat->n, mat->nb, mat->ld,
-                                mat->ipiv, trans, nrhs, B, ldb, c.permU, c.Linv,
-                                static_cast<size_t>(hplx::kMaxNB) * hplx::kMaxNB));
+                                mat->ipiv, trans, nrhs, B, ldb, flow_scratch(c)));
   HIPCHK(c, hipStreamSynchronize(c.stream));
   return HPLX_SUCCESS;
 }
@@ -960,7 +892,7 @@ int hplx_pdtrsv(hplx_ctx* ctx, int n, int nb, const double* A, int lda,
   HIPCHK(c, hipMemcpyAsync(x, A + static_cast<size_t>(n) * lda,
                            static_cast<size_t>(n) * sizeof(double),
                            hipMemcpyDeviceToDevice, c.stream));
-  HIPCHK(c, hplx::launch_trsv(c.stream, n, nb, A, lda, x));
+  HIPCHK(c, hplx::launch_trsv(c.stream, n, A, lda, x, flow_scratch(c)));
   HIPCHK(c, hipStreamSynchronize(c.stream));
   return HPLX_SUCCESS;
 }

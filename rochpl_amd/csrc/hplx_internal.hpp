@@ -93,6 +93,9 @@ struct Ctx {
   // those of panel k
   double*   Linv2      = nullptr;
   int*      permU2     = nullptr;
+  int*      flow_perm  = nullptr;    // kFlowPerm
+  int*      flow_flags = nullptr;    // kFlowFlags
+  unsigned long long* flow_x = nullptr;  // kFlowX
   int*      claim      = nullptr;    // 2 sets of kClaimInts update-claim counters
   int*      stop       = nullptr;    // 2 flags: claims of update k stop
   unsigned long long* vacate = nullptr;  // kVacateSets x 8 words (see cu_sets)
@@ -260,6 +263,11 @@ hipError_t launch_panel_kernel(Ctx& c, int slot, double* P, int lda, int m,
 
 hipError_t launch_pipid(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
                         int* permU);
+// The same for np consecutive panels of nb rows (the last one of what is left
+// of `rows`): panel p's interchanges ipiv + p nb, relative to base + p nb,
+// into permU + 2 p nb.
+hipError_t launch_pipid_panels(hipStream_t s, int np, int nb, int rows,
+                               const int* ipiv, int base, int* permU);
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, double* A,
                               int lda, const int* permU, double* W, int ldw);
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, float* A, int lda,
@@ -274,14 +282,7 @@ hipError_t launch_linv(hipStream_t s, int jb, const double* L, int ldl,
                        double* Linv, int ldi);
 hipError_t launch_linv(hipStream_t s, int jb, const float* L, int ldl,
                        float* Linv, int ldi);
-// op(T) x = b for nrhs columns of X; op(T) lower or upper as `lower` says
-// (T itself is upper when lower && trans, lower when !lower && trans).
-hipError_t launch_tri_solve(hipStream_t s, bool lower, bool trans, bool unit,
-                            int k, int nrhs, const double* T, int ldt,
-                            double* X, int ldx);
-hipError_t launch_tri_solve(hipStream_t s, bool lower, bool trans, bool unit,
-                            int k, int nrhs, const float* T, int ldt, float* X,
-                            int ldx);
+// B (k x n) = L^{-1} B, L unit lower.
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const double* L,
                                 int ldl, double* B, int ldb);
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const float* L,
@@ -373,18 +374,34 @@ hipError_t launch_nn_sub(hipStream_t s, int K, int m, int n, const double* A,
 hipError_t launch_outer_neg(hipStream_t s, int K, int m, int n,
                             const double* A, int lda, const double* B, int ldb,
                             double* C, int ldc);
-hipError_t launch_trsv(hipStream_t s, int n, int nb, const double* A, int lda,
-                       double* x);
+// Scratch of the triangular solves (k_flow.hip): the exchange buffer of the
+// solved blocks (128 values per right-hand side of a slice, and a flag per
+// block and slice; at least a panel's blocks with the most slices), the
+// split-K partial products of the transposed solve (work_doubles of them;
+// fewer only mean fewer splits) and the composed interchanges of the panels
+// prepared at once.  None needs to start in a particular state.
+constexpr int    kFlowBlocks = 128;
+constexpr int    kFlowCols   = 1024;  // right-hand sides at once
+constexpr int    kFlowFlags  = kMaxNB * kFlowCols / (128 * 4);
+constexpr size_t kFlowX      = static_cast<size_t>(kMaxNB) * kFlowCols;
+constexpr int    kFlowPerm   = 2 * 128 * kFlowBlocks;  // ints
+struct FlowScratch {
+  unsigned long long* x;     // kFlowX
+  double*             work;  // work_doubles
+  size_t              work_doubles;
+  int*                perm;   // kFlowPerm
+  int*                flags;  // kFlowFlags
+};
+
+// The back-solve U x = b (HPL_pdtrsv), x in place.
+hipError_t launch_trsv(hipStream_t s, int n, const double* A, int lda,
+                       double* x, const FlowScratch& w);
 
 // The solve with the factors of hplx_pdgetrf / hplx_pdgesv (hplx_pdgetrs)
-// queued on s: permU is 2 kMaxNB ints of scratch, work holds the split-K
-// partial products of the transposed solve (work_doubles doubles; a smaller
-// buffer only means fewer splits).  Neither needs to start zeroed.  No
-// allocation and no synchronisation.
+// queued on s.  No allocation and no synchronisation.
 hipError_t getrs_enqueue(hipStream_t s, const double* A, int N, int nb,
                          int lda, const int* ipiv, int trans, int nrhs,
-                         double* B, int ldb, int* permU, double* work,
-                         size_t work_doubles);
+                         double* B, int ldb, const FlowScratch& w);
 
 size_t     check_part_len(int n);  // doubles of scratch launch_check needs
 hipError_t launch_check(hipStream_t s, int n, int seed, double diag_shift,

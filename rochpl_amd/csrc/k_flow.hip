@@ -1,0 +1,692 @@
+// Triangular solves with a whole matrix of right-hand sides, as a dataflow of
+// 128-row blocks: one launch per panel of L (whose interchanges separate the
+// panels) and one per up to kFlowBlocks blocks of U, instead of a solve of
+// every diagonal block by one workgroup per right-hand side and a product
+// after it (HPL_pdtrsv, src/pgesv/HPL_pdtrsv_device.cpp:169-332, and the
+// solves hplx_pdgetrs and hplx_pdgesv_adjoint add).
+//
+// A workgroup owns a block of 128 rows and a slice of 16 or 4 right-hand
+// sides.  It keeps its block of B in MFMA accumulators, subtracts op(T)_ij x_j
+// for the solved 64-row halves j in dependency order as they appear
+// (V_MFMA_F64_16X16X4_F64 or _4X4X4_4B_F64, T straight from memory into the operand
+// registers, one half ahead), and, if the block lies on the diagonal, solves
+// its two 64 x 64 triangles by substitution, with the product between them,
+// and publishes x_i.  (Products with the triangles' inverses take about as
+// long, but their errors grow with the triangles' condition: the factors of a
+// Gaussian kernel matrix of order 1000 gave a backward error of 8e-6 with
+// them, 1.4e-16 with the substitution.)
+//
+// Progress.  A workgroup waits only for blocks of smaller index, and the
+// dispatcher hands out workgroups in index order on every XCD, so the
+// unfinished workgroup of the smallest index never waits: the grid need not
+// be resident at once.  The waits are bounded all the same; past the limit a
+// workgroup goes on with NaNs.
+//
+// x_i travels through an exchange buffer that the call fills with a NaN of a
+// payload of its own first (fill_kernel), and then a flag is raised.  The
+// next block of the chain polls the values themselves, by device-scope
+// accesses, until none is that NaN: a step needs one store-to-load trip
+// through memory and no cache write-back or invalidation.  The blocks
+// further on are not in a hurry: they poll the flag at leisure and then read
+// x_i through their L2 (U of N = 16384 with 64 right-hand sides in 64-row
+// blocks: 2243 us with all of them polling the values, 1220 us so).  Nothing
+// outlives the call, so the launches can be captured and replayed.
+//
+// Bound by latency: a step of the chain is two substitutions of 64 rows (each
+// 64 dependent FMAs on broadcast values), two products of 64 columns and that
+// trip, 4.6 us in all for narrow slices, 8.7 for wide ones.  128-row blocks
+// rather than 64-row ones: half the trips (that U 1115 us).
+//
+// hplx_pdgetrs, before and now: N = 16384, NB = 512, 64 right-hand sides 9.50
+// -> 2.78 ms (transposed 8.92 -> 3.51), one 9.27 -> 1.69, 512 15.2 -> 9.9;
+// N = 5000, NB = 128, one 2.87 -> 0.77 ms.  The floor is one read of the
+// factors (2.1 GB, 0.4 ms).
+#include <utility>
+
+#include "hplx_internal.hpp"
+#include "lds_stream.hpp"
+
+namespace hplx {
+namespace {
+
+typedef double ud4 __attribute__((ext_vector_type(4)));
+// two neighbouring doubles at any 8-byte address
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+constexpr int kFB  = 128;  // rows of a block
+constexpr int kFH  = 64;   // and of its halves
+constexpr int kFLd = 66;   // LDS pitch of a right-hand side of a half
+constexpr int kNext = 1;   // blocks ahead in the chain that poll the values
+constexpr uint32_t kFlowSpinLimit = 1u << 22;
+// Narrow slices (4 right-hand sides) while at most this many workgroups come
+// of it, 2 per CU: a step takes 4.6 instead of 8.7 us, but every slice reads
+// all of T (N = 16384: 16 right-hand sides 2.04 against 2.21 ms, 24 2.31
+// against 2.21).
+constexpr int kNarrowGrid = 512;
+// From this many right-hand sides on the rows off the diagonal blocks of
+// kSplitRows rows are updated by the GEMM of k_trsv.hip, which reads T once
+// per 64 of them.
+constexpr int kSplitRhs = 192, kSplitRows = 512;
+// A half's triangle in LDS holds, of its columns in pairs, the positions from
+// 16 (c / 16) on (positions: rows in the order they are solved); the index of
+// the entry at position p is tri_col(c) + 2 p.
+__host__ __device__ constexpr int tri_col(int c) {
+  const int b = c / 16;  // 16 columns of 64, of 48, of 32, of 16 entries
+  return 16 * (64 * b - 8 * b * (b - 1)) + (c - 16 * b) / 2 * 2 * (64 - 16 * b) -
+         32 * b + (c & 1);
+}
+constexpr int kTri = 16 * (64 + 48 + 32 + 16);
+
+// y -= x_J m for a column J of a half's triangle: x_J is lane J's of each 16
+// (4 right-hand sides side by side), m is -T(., J).  One asm per column, the
+// rows further on first: s_nop covers the VALU write of x just before.  Every
+// lane has to be active.
+#define HPLX_FMA(y, x, m, j) \
+  "v_fmac_f64_dpp %" #y ", %" #x ", %" #m " row_newbcast:%" #j " row_mask:0xf bank_mask:0xf\n\t"
+template <int S, int J>
+__device__ __forceinline__ void tri_column(double (&x)[4], const double (&m)[4]) {
+  if constexpr(S == 0)
+    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 5, 8) HPLX_FMA(2, 0, 6, 8) HPLX_FMA(3, 0, 7, 8)
+            HPLX_FMA(0, 0, 4, 8)
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+        : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "n"(J));
+  if constexpr(S == 1)
+    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 4, 6) HPLX_FMA(2, 0, 5, 6) HPLX_FMA(0, 0, 3, 6)
+        : "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
+        : "v"(m[1]), "v"(m[2]), "v"(m[3]), "n"(J));
+  if constexpr(S == 2)
+    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 3, 4) HPLX_FMA(0, 0, 2, 4)
+        : "+v"(x[2]), "+v"(x[3])
+        : "v"(m[2]), "v"(m[3]), "n"(J));
+  if constexpr(S == 3)
+    asm("s_nop 1\n\t" HPLX_FMA(0, 0, 1, 2) : "+v"(x[3]) : "v"(m[3]), "n"(J));
+}
+#undef HPLX_FMA
+
+// Columns 16 S + 2 J2 and the next; p: the triangle + 2 (lane % 16).
+typedef double d2a __attribute__((ext_vector_type(2)));
+template <int S, int J2>
+__device__ __forceinline__ void tri_pair(double (&x)[4], const double* p) {
+  constexpr int c = tri_col(16 * S + 2 * J2);
+  double        m0[4], m1[4];
+#pragma unroll
+  for(int s = S; s < 4; ++s) {
+    const d2a v = *reinterpret_cast<const d2a*>(p + c + 32 * s);
+    m0[s]       = v.x;
+    m1[s]       = v.y;
+  }
+  tri_column<S, 2 * J2>(x, m0);
+  tri_column<S, 2 * J2 + 1>(x, m1);
+}
+template <int S, int... J2>
+__device__ __forceinline__ void tri_columns(double (&x)[4], const double* p,
+                                            std::integer_sequence<int, J2...>) {
+  (tri_pair<S, J2>(x, p), ...);
+}
+
+struct FlowArgs {
+  const double* T;
+  int           ldt;
+  double*       B;
+  int           ldb, nrhs;
+  int           d0, d1;  // rows of the diagonal blocks
+  int           o0, o1;  // rows of the others, updated only
+  int           nd, nt;  // blocks on the diagonal, in all
+  int           ns;      // slices of 16 right-hand sides
+  unsigned long long* x;      // nd x ns blocks of 2 halves of 16 x 64 values
+  int*                flags;  // nd x ns
+};
+
+// The exchange buffer's filling: a NaN no computed value has (those that
+// would be published are replaced by the plain quiet NaN).
+constexpr unsigned long long kEmpty = 0x7ff8b10cffffb10cull;
+
+__global__ __launch_bounds__(256) void fill_kernel(unsigned long long* p, int n,
+                                                   int* flags, int nf) {
+  const int i0 = blockIdx.x * 256 + threadIdx.x;
+  for(int i = i0; i < n; i += gridDim.x * 256) p[i] = kEmpty;
+  if(i0 < nf) flags[i0] = 0;
+}
+
+// A wave's 16 rows x 64 columns of op(T): lane (m, g) holds T(row0 + m,
+// col0 + 16 g + s), s = 0 .. 15 (the MFMA's k index is 4 s' + g in any
+// order, as long as both operands agree).  nr / nc: rows and columns inside;
+// the others are zero and read nothing.
+template <bool TRANS>
+__device__ __forceinline__ void load_block(const double* __restrict__ T, int ldt,
+                                           int row0, int nr, int col0, int nc,
+                                           double (&t)[16]) {
+  const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+  if(nr >= 16 && nc >= kFH) {
+    if(TRANS) {
+      const double* p = T + col0 + 16 * g + static_cast<size_t>(row0 + m) * ldt;
+#pragma unroll
+      for(int s = 0; s < 16; s += 2) {
+        const d2u v = *reinterpret_cast<const d2u*>(p + s);
+        t[s]     = v.x;
+        t[s + 1] = v.y;
+      }
+    } else {
+      // uniform column starts plus one 32-bit offset per lane
+      const double*  p   = T + row0 + static_cast<size_t>(col0) * ldt;
+      const uint32_t off = static_cast<uint32_t>(m + 16 * g * ldt);
+#pragma unroll
+      for(int s = 0; s < 16; ++s) t[s] = (p + static_cast<size_t>(s) * ldt)[off];
+    }
+    return;
+  }
+  if(nr <= 0 || nc <= 0) {
+#pragma unroll
+    for(int s = 0; s < 16; ++s) t[s] = 0.0;
+    return;
+  }
+  // an edge: clamped addresses, then zeros
+  const double* p  = T + (TRANS ? col0 + static_cast<size_t>(row0) * ldt
+                                : row0 + static_cast<size_t>(col0) * ldt);
+  const int     mr = m < nr ? m : nr - 1;
+#pragma unroll
+  for(int s = 0; s < 16; ++s) {
+    const int c  = 16 * g + s, cr = c < nc ? c : nc - 1;
+    const double v = p[static_cast<uint32_t>(TRANS ? cr + mr * ldt : mr + cr * ldt)];
+    t[s] = m < nr && c < nc ? v : 0.0;
+  }
+}
+
+// T x for the wave's 16 rows and a slice of right-hand sides (xs: [column]
+// [row], 64 rows).  Wide: 16 columns, V_MFMA_F64_16X16X4_F64; narrow: 4
+// columns, V_MFMA_F64_4X4X4_4B_F64 (its four blocks four rows each), a
+// quarter of the time.  A lane holds kE values: row(e), col().
+template <bool WIDE>
+struct Product;
+template <>
+struct Product<true> {
+  static constexpr int kR = 16, kE = 4;
+  typedef ud4          Acc;
+  __device__ static int row(int e) { return 4 * e + ((threadIdx.x & 63) >> 4); }
+  __device__ static int col() { return threadIdx.x & 15; }
+  __device__ static ud4 zero() { return ud4{0.0, 0.0, 0.0, 0.0}; }
+  __device__ static ud4 mfma(double t, double x, ud4 acc) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(t, x, acc, 0, 0, 0);
+  }
+};
+typedef double ud1 __attribute__((ext_vector_type(1)));
+template <>
+struct Product<false> {
+  static constexpr int kR = 4, kE = 1;
+  typedef ud1          Acc;
+  __device__ static int row(int) {
+    return 4 * ((threadIdx.x >> 2) & 3) + ((threadIdx.x & 63) >> 4);
+  }
+  __device__ static int col() { return threadIdx.x & 3; }
+  __device__ static ud1 zero() { return ud1{0.0}; }
+  __device__ static ud1 mfma(double t, double x, ud1 acc) {
+    return ud1{__builtin_amdgcn_mfma_f64_4x4x4f64(t, x, acc.x, 0, 0, 0)};
+  }
+};
+
+template <bool WIDE>
+__device__ __forceinline__ typename Product<WIDE>::Acc block_product(
+    const double (&t)[16], const double* xs) {
+  typedef Product<WIDE> P;
+  const double* x = xs + P::col() * kFLd + 16 * ((threadIdx.x & 63) >> 4);
+  double        xf[16];
+#pragma unroll
+  for(int s = 0; s < 16; ++s) xf[s] = x[s];
+  typename P::Acc acc = P::zero();
+#pragma unroll
+  for(int s = 0; s < 16; ++s) acc = P::mfma(t[s], xf[s], acc);
+  return acc;
+}
+
+constexpr double kHuge = 1.7976931348623157e308;
+
+// The triangles of a diagonal block's two halves, in the order they are
+// solved, as tri_columns takes them: divided by the diagonal and negated,
+// zero up to the diagonal.  scale: the diagonal's reciprocals.  rare is set
+// if one of them is not an ordinary number.  t: the block's first entry, w
+// its rows.  L (its unit diagonal is not read) is what is solved forward as it
+// lies or backward transposed.
+template <bool TRANS, bool BACK>
+__device__ __forceinline__ void stage_triangle(const double* __restrict__ t, int ldt, int w,
+                                               double* tri, double* scale, int* rare) {
+  constexpr bool UNIT = TRANS == BACK;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int h = wave >> 2, r0 = kFH * (BACK ? 1 - h : h);
+  auto row = [&](int p) { return r0 + (BACK ? kFH - 1 - p : p); };
+  auto at  = [&](int i, int j) {  // of a row and a column inside
+    i = min(i, w - 1), j = min(j, w - 1);
+    return t[TRANS ? j + static_cast<size_t>(i) * ldt : i + static_cast<size_t>(j) * ldt];
+  };
+  // a line of op(T) along memory per wave: a column, or a row of the
+  // transposed
+  double v[16];
+#pragma unroll
+  for(int q = 0; q < 16; ++q) {
+    const int k = 4 * q + (wave & 3);
+    v[q]        = TRANS ? at(row(k), row(lane)) : at(row(lane), row(k));
+  }
+  const int    mr = row(lane);
+  const double d  = UNIT || mr >= w ? 1.0 : at(mr, mr);
+  if((wave & 3) == 0) {
+    scale[kFH * h + lane] = 1.0 / d;
+    if(!(fabs(d) >= 0x1p-1000 && fabs(d) <= 0x1p1000)) *rare = 1;
+  }
+#pragma unroll
+  for(int q = 0; q < 16; ++q) {
+    const int    k = 4 * q + (wave & 3);
+    const int    p = TRANS ? k : lane, c = TRANS ? lane : k;
+    const double e = UNIT ? v[q] : v[q] / (TRANS ? __shfl(d, k) : d);
+    if(p >= (c & ~15))
+      tri[h * kTri + tri_col(c) + 2 * p] = p > c && row(p) < w && row(c) < w ? -e : 0.0;
+  }
+}
+
+// A half by plain substitution, for what tri_columns cannot take: a diagonal
+// whose reciprocal is not an ordinary number, or values that are not finite
+// (whose products with its zeros are not zero).
+template <bool TRANS, bool BACK>
+__device__ __forceinline__ void solve_half(const double* __restrict__ t, int ldt, int r0,
+                                        int left, const double* xc, double (&v)[4]) {
+  constexpr bool UNIT = TRANS == BACK;
+  const int lane = threadIdx.x & 63, m = lane & 15;
+#pragma unroll
+  for(int s = 0; s < 4; ++s) v[s] = xc[BACK ? kFH - 1 - (16 * s + m) : 16 * s + m];
+  for(int p = 0; p < kFH; ++p) {
+    const int j = BACK ? kFH - 1 - p : p;
+    if(j >= left) continue;
+    const double* tj = t + r0 + static_cast<size_t>(r0) * ldt;
+    double        xj = 0.0;
+#pragma unroll
+    for(int s = 0; s < 4; ++s)
+      if((p >> 4) == s) {
+        xj = __shfl(v[s], p & 15, 16);
+        if(!UNIT) xj = xj / tj[j + static_cast<size_t>(j) * ldt];
+        if(m == (p & 15)) v[s] = xj;
+      }
+#pragma unroll
+    for(int s = 0; s < 4; ++s) {
+      const int q = 16 * s + m, i = BACK ? kFH - 1 - q : q;
+      if(q > p && i < left)
+        v[s] = fma(-tj[TRANS ? j + static_cast<size_t>(i) * ldt
+                             : i + static_cast<size_t>(j) * ldt],
+                   xj, v[s]);
+    }
+  }
+}
+
+// TRANS: op(T) = T^T.  BACK: the diagonal blocks are solved from the last.
+template <bool TRANS, bool BACK, bool WIDE>
+__global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
+  typedef Product<WIDE> P;
+  constexpr int         R = P::kR, E = P::kE, W = (R + 7) / 8;
+  constexpr bool        UNIT = TRANS == BACK;
+  __shared__ __attribute__((aligned(16))) double xs[2][R * kFLd];
+  __shared__ __attribute__((aligned(16))) double tri[2 * kTri];
+  __shared__ double scale[2 * kFH];
+  __shared__ int    rare;
+  // the slices of a block on one XCD (they read the same rows of T), blocks
+  // in index order
+  const int per = 8 * a.ns, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
+  const int sl = br / 8, i = bg * 8 + (br & 7);
+  if(i >= a.nt) return;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int ac = P::col();  // this lane's right-hand side
+  const int c0 = sl * R, nc = min(R, a.nrhs - c0);
+  auto diag_row = [&](int k) { return a.d0 + kFB * (BACK ? a.nd - 1 - k : k); };
+  const bool diag = i < a.nd;
+  const int  r = diag ? diag_row(i) : a.o0 + kFB * (i - a.nd);
+  const int  w = min(kFB, (diag ? a.d1 : a.o1) - r);
+  const int  r0 = r + 16 * wave, nr = w - 16 * wave;  // this wave's rows
+  // the solved halves in the order they appear: half h of block k is rows
+  // [half_row, + 64)
+  const int steps = 2 * (diag ? i : a.nd);
+  auto half_row = [&](int st) {
+    return diag_row(st >> 1) + kFH * (BACK ? 1 - (st & 1) : st & 1);
+  };
+
+  double*         Bc = a.B + r0 + static_cast<size_t>(c0 + ac) * a.ldb;
+  // the products are summed by themselves and added to B at the end
+  typename P::Acc acc = P::zero(), b = P::zero();
+#pragma unroll
+  for(int e = 0; e < E; ++e)
+    if(P::row(e) < nr && ac < nc) b[e] = Bc[P::row(e)];
+  double tv[16], tn[16];
+  if(diag) {
+    if(t == 0) rare = 0;
+    __syncthreads();
+    stage_triangle<TRANS, BACK>(a.T + r + static_cast<size_t>(r) * a.ldt, a.ldt, w, tri,
+                                scale, &rare);
+  }
+  // the second half of a block on the diagonal has one more product to form,
+  // with its own first half
+  const bool second = diag && (BACK ? wave < 4 : wave >= 4);
+  const int  mine   = steps + (second ? 1 : 0);
+  if(mine > 0) {
+    const int cj = half_row(0);
+    load_block<TRANS>(a.T, a.ldt, r0, nr, cj, min(kFH, a.d1 - cj), tn);
+  }
+  uint32_t spins = 0;
+  bool     dead  = false;
+  for(int st = 0; st < steps; ++st) {
+#pragma unroll
+    for(int s = 0; s < 16; ++s) tv[s] = tn[s];
+    // x of this half into LDS: wave w columns w, w + 8
+    const int           j  = st >> 1;
+    unsigned long long* xj = a.x + (static_cast<size_t>(2 * j + (st & 1)) * a.ns + sl) *
+                                       (R * kFH) + kFH * wave + lane;
+    unsigned long long  xv[W];
+    if(wave < R) {
+      if(diag && j + kNext >= i) {
+        __builtin_amdgcn_s_setprio(3);
+        for(;;) {
+          bool in = true;
+#pragma unroll
+          for(int q = 0; q < W; ++q)
+            xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+          for(int q = 0; q < W; ++q) in = in && xv[q] != kEmpty;
+          if(__all(in) || dead) break;
+          dead = ++spins > kFlowSpinLimit;
+        }
+      } else {
+        const int* flag = a.flags + j * a.ns + sl;
+        while(!dead && !__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+          dead = ++spins > kFlowSpinLimit;
+          __builtin_amdgcn_s_sleep(8);
+        }
+        asm volatile("" : : : "memory");  // the values are read after the flag
+#pragma unroll
+        for(int q = 0; q < W; ++q) xv[q] = xj[8 * kFH * q];
+      }
+      if(dead) {
+#pragma unroll
+        for(int q = 0; q < W; ++q) xv[q] = 0x7ff8000000000000ull;
+      }
+    }
+    if(st + 1 < mine) {
+      const int cn = half_row(st + 1);
+      load_block<TRANS>(a.T, a.ldt, r0, nr, cn, min(kFH, a.d1 - cn), tn);
+    }
+    double* x = xs[st & 1];
+    if(wave < R) {
+#pragma unroll
+      for(int q = 0; q < W; ++q)
+        x[(wave + 8 * q) * kFLd + lane] =
+            -__longlong_as_double(static_cast<long long>(xv[q]));
+    }
+    __syncthreads();  // this buffer is written again two barriers on
+    // a half's sum is formed by itself: N / 64 roundings at the magnitude of
+    // the whole instead of N
+    acc += block_product<WIDE>(tv, x);
+  }
+  if(!diag) {
+#pragma unroll
+    for(int e = 0; e < E; ++e)
+      if(P::row(e) < nr && ac < nc) Bc[P::row(e)] = b[e] + acc[e];
+    return;
+  }
+  for(int h = 0; h < 2; ++h) {
+    // the half's right-hand sides into LDS, in the order of their positions
+    const int half = BACK ? 1 - h : h, left = w - kFH * half;
+    double*   x    = xs[0];
+    __syncthreads();  // the last products have read xs
+    if((wave >> 2) == half)
+#pragma unroll
+      for(int e = 0; e < E; ++e) x[ac * kFLd + 16 * (wave & 3) + P::row(e)] = b[e] + acc[e];
+    __syncthreads();
+    // 4 right-hand sides a wave, lane (m, g): rows m, 16 + m, ... in solving
+    // order of the g-th
+    if(wave < R / 4) {
+      const int     m = lane & 15, c = 4 * wave + (lane >> 4);
+      const double* p = tri + h * kTri + 2 * m;
+      double        v[4];
+      double*       xc = x + c * kFLd;
+#pragma unroll
+      for(int s = 0; s < 4; ++s) {
+        const int q = 16 * s + m;
+        v[s]        = xc[BACK ? kFH - 1 - q : q] * (UNIT ? 1.0 : scale[kFH * h + q]);
+      }
+      typedef std::make_integer_sequence<int, 8> Pairs;
+      tri_columns<0>(v, p, Pairs());
+      tri_columns<1>(v, p, Pairs());
+      tri_columns<2>(v, p, Pairs());
+      tri_columns<3>(v, p, Pairs());
+      const bool fine = fabs(v[0]) <= kHuge && fabs(v[1]) <= kHuge && fabs(v[2]) <= kHuge &&
+                        fabs(v[3]) <= kHuge;
+      // which path a right-hand side takes does not depend on the others
+      const unsigned long long bad = __ballot(rare || !fine);
+      if(bad) {
+        double u[4];
+        solve_half<TRANS, BACK>(a.T + r + static_cast<size_t>(r) * a.ldt, a.ldt, kFH * half,
+                                left, xc, u);
+        if((bad >> (lane & 48)) & 0xffff)
+#pragma unroll
+          for(int s = 0; s < 4; ++s) v[s] = u[s];
+      }
+      unsigned long long* xi =
+          a.x + (static_cast<size_t>(2 * i + h) * a.ns + sl) * (R * kFH) + c * kFH;
+#pragma unroll
+      for(int s = 0; s < 4; ++s) {
+        const int q = BACK ? kFH - 1 - (16 * s + m) : 16 * s + m;
+        __hip_atomic_store(
+            xi + q,
+            v[s] == v[s] ? static_cast<unsigned long long>(__double_as_longlong(v[s]))
+                         : 0x7ff8000000000000ull,
+            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for(int s = 0; s < 4; ++s) {
+        const int q = BACK ? kFH - 1 - (16 * s + m) : 16 * s + m;
+        xc[q]       = -v[s];
+        if(q < left && c < nc) a.B[r + kFH * half + q + static_cast<size_t>(c0 + c) * a.ldb] = v[s];
+      }
+      wait_vm<0>();  // the values have reached the device's memory
+    }
+    __syncthreads();
+    if(h == 0 && second) acc += block_product<WIDE>(tn, x);
+  }
+  if(t == 0)
+    __hip_atomic_store(a.flags + i * a.ns + sl, 1, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The solves of one call on a stream, for at most kFlowCols right-hand sides.
+struct Flow {
+  hipStream_t        s;
+  const double*      T;
+  int                ldt;
+  double*            B;
+  int                ldb, nrhs, rows;  // rows: of T
+  const FlowScratch& w;
+
+  bool wide() const {
+    return static_cast<long>((rows + kFB - 1) / kFB) * ((nrhs + 3) / 4) > kNarrowGrid;
+  }
+  bool split() const { return nrhs >= kSplitRhs; }
+  int  group() const { return wide() ? Product<true>::kR : Product<false>::kR; }
+  int slices() const { return (nrhs + group() - 1) / group(); }
+  // blocks whose x fit the exchange buffer
+  int blocks() const {
+    const size_t b = kFlowX / x_panel(1);
+    return b < static_cast<size_t>(kFlowBlocks) ? static_cast<int>(b) : kFlowBlocks;
+  }
+  size_t x_panel(int bpp) const {
+    return static_cast<size_t>(bpp) * slices() * group() * kFB;
+  }
+
+  // np panels' (of bpp blocks) x marked as not there yet
+  hipError_t prepare(int np, int bpp) {
+    if(np * bpp > blocks()) return hipErrorInvalidValue;
+    const int n = static_cast<int>(x_panel(bpp)) * np;
+    hipLaunchKernelGGL(fill_kernel, dim3(n < 256 * 1024 ? (n + 255) / 256 : 1024),
+                       dim3(256), 0, s, w.x, n, w.flags, np * bpp * slices());
+    return hipGetLastError();
+  }
+
+  template <bool WIDE>
+  void launch(bool trans, bool back, dim3 g, dim3 b, const FlowArgs& a) {
+    if(trans && back)
+      hipLaunchKernelGGL((flow_kernel<true, true, WIDE>), g, b, 0, s, a);
+    else if(trans)
+      hipLaunchKernelGGL((flow_kernel<true, false, WIDE>), g, b, 0, s, a);
+    else if(back)
+      hipLaunchKernelGGL((flow_kernel<false, true, WIDE>), g, b, 0, s, a);
+    else
+      hipLaunchKernelGGL((flow_kernel<false, false, WIDE>), g, b, 0, s, a);
+  }
+
+  // op(T) on rows [d0, d1) solved, then applied to rows [o0, o1); block: the
+  // index of the first of these blocks among the prepared ones.
+  hipError_t solve(bool trans, bool back, int d0, int d1, int o0, int o1,
+                   int block) {
+    if(!split()) return flow(trans, back, d0, d1, o0, o1, block);
+    const int n = (d1 - d0 + kSplitRows - 1) / kSplitRows;
+    for(int k = 0; k < n; ++k) {
+      const int q  = back ? n - 1 - k : k;
+      const int s0 = d0 + q * kSplitRows;
+      const int s1 = s0 + kSplitRows < d1 ? s0 + kSplitRows : d1;
+      hipError_t e = flow(trans, back, s0, s1, s0, s0, block + q * (kSplitRows / kFB));
+      // the rows of the diagonal range still to be solved, then the others
+      if(e == hipSuccess) e = back ? update(trans, s0, s1, d0, s0) : update(trans, s0, s1, s1, d1);
+      if(e == hipSuccess) e = update(trans, s0, s1, o0, o1);
+      if(e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+
+  // rows [o0, o1) -= op(T) x for the solved rows [s0, s1)
+  hipError_t update(bool trans, int s0, int s1, int o0, int o1) {
+    if(o1 <= o0) return hipSuccess;
+    if(trans)
+      return launch_tn_sub(s, s1 - s0, o1 - o0, nrhs,
+                           T + s0 + static_cast<size_t>(o0) * ldt, ldt, B + s0, ldb,
+                           B + o0, ldb, w.work, w.work_doubles);
+    return launch_nn_sub(s, s1 - s0, o1 - o0, nrhs,
+                         T + o0 + static_cast<size_t>(s0) * ldt, ldt, B + s0, ldb,
+                         B + o0, ldb);
+  }
+
+  hipError_t flow(bool trans, bool back, int d0, int d1, int o0, int o1, int block) {
+    FlowArgs a;
+    a.T     = T;
+    a.ldt   = ldt;
+    a.x     = w.x + x_panel(block);
+    a.flags = w.flags + block * slices();
+    a.B     = B;
+    a.ldb   = ldb;
+    a.nrhs  = nrhs;
+    a.ns    = slices();
+    a.d0    = d0;
+    a.d1    = d1;
+    a.o0    = o0;
+    a.o1    = o1;
+    a.nd    = (d1 - d0 + kFB - 1) / kFB;
+    a.nt    = a.nd + (o1 - o0 + kFB - 1) / kFB;
+    const long grid = (a.nt + 7L) / 8 * 8 * a.ns;
+    if(block + a.nd > blocks() || grid > 0x7fffffffL) return hipErrorInvalidValue;
+    const dim3 g(static_cast<unsigned>(grid)), b(512);
+    if(wide())
+      launch<true>(trans, back, g, b, a);
+    else
+      launch<false>(trans, back, g, b, a);
+    return hipGetLastError();
+  }
+
+  // U x = b over rows [0, n): chunks from the bottom
+  hipError_t upper(int n) {
+    const int c = blocks() * kFB;
+    for(int d0 = (n - 1) / c * c; d0 >= 0; d0 -= c) {
+      const int  d1 = d0 + c < n ? d0 + c : n;
+      hipError_t e  = prepare(1, (d1 - d0 + kFB - 1) / kFB);
+      if(e == hipSuccess) e = solve(false, true, d0, d1, 0, d0, 0);
+      if(e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+
+  // U^T x = b over rows [0, n)
+  hipError_t upper_trans(int n) {
+    const int c = blocks() * kFB;
+    for(int d0 = 0; d0 < n; d0 += c) {
+      const int  d1 = d0 + c < n ? d0 + c : n;
+      hipError_t e  = prepare(1, (d1 - d0 + kFB - 1) / kFB);
+      if(e == hipSuccess) e = solve(true, false, d0, d1, d1, n, 0);
+      if(e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+};
+
+}  // namespace
+
+hipError_t launch_trsv(hipStream_t s, int n, const double* A, int lda, double* x,
+                       const FlowScratch& w) {
+  if(n <= 0) return hipSuccess;
+  return Flow{s, A, lda, x, n, 1, n, w}.upper(n);
+}
+
+#define HCHK(expr)                  \
+  do {                              \
+    const hipError_t e_ = (expr);   \
+    if(e_ != hipSuccess) return e_; \
+  } while(0)
+
+// At most kFlowCols right-hand sides.
+static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
+                               int lda, const int* ipiv, int trans, int nrhs,
+                               double* B, int ldb, const FlowScratch& w) {
+  Flow f{s, A, lda, B, ldb, nrhs, N, w};
+  const int np  = (N + nb - 1) / nb;
+  const int bpp = (nb + kFB - 1) / kFB;
+  const int pc  = f.blocks() / bpp;  // panels prepared at once
+  // panels [p0, p0 + pc): their exchange buffers, and the interchanges composed
+  auto prepare = [&](int p0) -> hipError_t {
+    const int p1 = p0 + pc < np ? p0 + pc : np;
+    HCHK(f.prepare(p1 - p0, bpp));
+    return launch_pipid_panels(s, p1 - p0, nb, N - p0 * nb, ipiv + p0 * nb,
+                               p0 * nb, w.perm);
+  };
+  if(!trans) {
+    // L solve with the panel-by-panel interchanges, as b is carried through
+    // the factorisation (HPL_pdgesv), then U x = y (HPL_pdtrsv)
+    for(int p = 0; p < np; ++p) {
+      const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb, pi = p % pc;
+      if(pi == 0) HCHK(prepare(p));
+      HCHK(launch_swap_inplace(s, jb, nrhs, B + j, ldb, w.perm + pi * 2 * nb));
+      HCHK(f.solve(false, false, j, j + jb, j + jb, N, pi * bpp));
+    }
+    return f.upper(N);
+  }
+  // A = P0^T L0 P1^T L1 ... U  =>  A^T z = g  is solved as
+  // w = U^{-T} g, then for panels from the last: z_p -= L21^T z_below,
+  // z_p = L11^{-T} z_p, z = P_p^T z.
+  HCHK(f.upper_trans(N));
+  for(int p = np - 1; p >= 0; --p) {
+    const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb, e = j + jb, pi = p % pc;
+    if(p == np - 1 || pi == pc - 1) HCHK(prepare(p - pi));
+    // z_p -= L21^T z_below reduces over all N - e rows below the panel for a
+    // jb x nrhs result: split over K, the partials in the work buffer, while
+    // they fit
+    if(e < N)
+      HCHK(launch_tn_sub(s, N - e, jb, nrhs, A + e + static_cast<size_t>(j) * lda,
+                         lda, B + e, ldb, B + j, ldb, w.work, w.work_doubles));
+    HCHK(f.solve(true, true, j, e, e, e, pi * bpp));
+    HCHK(launch_swap_inverse(s, jb, nrhs, B + j, ldb, w.perm + pi * 2 * nb));
+  }
+  return hipSuccess;
+}
+
+hipError_t getrs_enqueue(hipStream_t s, const double* A, int N, int nb, int lda,
+                         const int* ipiv, int trans, int nrhs, double* B,
+                         int ldb, const FlowScratch& w) {
+  for(int c = 0; c < nrhs; c += kFlowCols)
+    HCHK(getrs_slices(s, A, N, nb, lda, ipiv, trans,
+                      nrhs - c < kFlowCols ? nrhs - c : kFlowCols,
+                      B + static_cast<size_t>(c) * ldb, ldb, w));
+  return hipSuccess;
+}
+#undef HCHK
+
+}  // namespace hplx

@@ -63,15 +63,21 @@ __global__ void reset_kernel(int* info, int* err) {
 //                  p_i if none
 //     a position q >= jb ends with g(last i with p_i = q).
 //   Chains of g only go to smaller indices and are followed per thread.
+// One workgroup per panel (several for the solves with stored factors).
 __global__ __launch_bounds__(1024) void pipid_kernel(
-    int jb, const int* __restrict__ ipiv, int base, int* __restrict__ permU) {
+    int nb, int rows, const int* __restrict__ ipiv, int base,
+    int* __restrict__ permU) {
   __shared__ int sp[kMaxNB];
   __shared__ int sprev[kMaxNB];   // last i' < i with p_i' == p_i, or -1
   __shared__ int sto[kMaxNB];     // last i' < i with p_i' == i, or -1
   __shared__ int slast[kMaxNB];   // 1 if no later step targets p_i
   __shared__ int sg[kMaxNB];
   __shared__ int sout[2 * kMaxNB];
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, p0 = blockIdx.x * nb;
+  const int jb = min(nb, rows - p0);
+  ipiv += p0;
+  base += p0;
+  permU += 2 * static_cast<size_t>(p0);
   // an interchange must target a row at or below its own; anything else is
   // treated as no interchange so that every LDS index stays in range
   for(int i = t; i < jb; i += blockDim.x) {
@@ -549,8 +555,17 @@ hipError_t launch_pipid(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
                         int* permU) {
   if(jb <= 0) return hipSuccess;
   if(jb > kMaxNB) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(pipid_kernel, dim3(1), dim3(1024), 0, s, jb, ipiv,
+  hipLaunchKernelGGL(pipid_kernel, dim3(1), dim3(1024), 0, s, jb, jb, ipiv,
                      ipiv_base, permU);
+  return hipGetLastError();
+}
+
+hipError_t launch_pipid_panels(hipStream_t s, int np, int nb, int rows,
+                               const int* ipiv, int base, int* permU) {
+  if(np <= 0) return hipSuccess;
+  if(nb < 1 || nb > kMaxNB || rows <= (np - 1) * nb) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(pipid_kernel, dim3(np), dim3(1024), 0, s, nb, rows, ipiv,
+                     base, permU);
   return hipGetLastError();
 }
 

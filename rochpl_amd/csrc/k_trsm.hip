@@ -3,11 +3,9 @@
 //
 // Used for the unit-lower L11 solves of the panel recursion and of the
 // trailing update (rocblas_dtrsm at src/pfact/HPL_pdrpanrlT.cpp:124-135 and
-// src/pgesv/HPL_pdupdateTT.cpp:95-106), for the explicit inverse of L11, for
-// the diagonal blocks of the back-solve (rocblas_dtrsv at
-// src/pgesv/HPL_pdtrsv_device.cpp:170-178,279-287), for the transposed
-// solves of the adjoint, and (diag_inv_kernel) for the FP32 or FP64
-// inverses of the diagonal blocks of the mixed-precision factors.
+// src/pgesv/HPL_pdupdateTT.cpp:95-106), for the explicit inverse of L11, and
+// (diag_inv_kernel) for the FP32 or FP64 inverses of the diagonal blocks of
+// the mixed-precision factors.
 //
 // x lives in LDS.  The block is processed in 64-row chunks along the sweep
 // direction: wave 0 solves the chunk's 64 x 64 triangle with the chunk's rows
@@ -49,21 +47,12 @@ __global__ __launch_bounds__(256) void diag_inv_kernel(int kb,
 }
 
 template <typename V>
-hipError_t tri_solve_t(hipStream_t s, bool lower, bool trans, bool unit, int k,
-                       int nrhs, const V* T, int ldt, V* X, int ldx) {
-  if(k <= 0 || nrhs <= 0) return hipSuccess;
+hipError_t trsm_t(hipStream_t s, int k, int n, const V* L, int ldl, V* B,
+                  int ldb) {
+  if(k <= 0 || n <= 0) return hipSuccess;
   if(k > kMaxNB) return hipErrorInvalidValue;
-  const dim3 g(nrhs), b(256);
-  if(lower && !trans && unit)
-    hipLaunchKernelGGL((tri_solve_kernel<V, V, true, false, true, false>), g, b, 0, s, k, T, ldt, X, ldx);
-  else if(!lower && !trans && !unit)
-    hipLaunchKernelGGL((tri_solve_kernel<V, V, false, false, false, false>), g, b, 0, s, k, T, ldt, X, ldx);
-  else if(lower && trans && !unit)  // U^T: U stored upper
-    hipLaunchKernelGGL((tri_solve_kernel<V, V, true, true, false, false>), g, b, 0, s, k, T, ldt, X, ldx);
-  else if(!lower && trans && unit)  // L^T: L stored unit lower
-    hipLaunchKernelGGL((tri_solve_kernel<V, V, false, true, true, false>), g, b, 0, s, k, T, ldt, X, ldx);
-  else
-    return hipErrorInvalidValue;
+  hipLaunchKernelGGL((tri_solve_kernel<V, V, true, false, true, false>), dim3(n),
+                     dim3(256), 0, s, k, L, ldl, B, ldb);
   return hipGetLastError();
 }
 
@@ -78,18 +67,6 @@ hipError_t linv_t(hipStream_t s, int jb, const V* L, int ldl, V* Linv,
 }
 
 }  // namespace
-
-hipError_t launch_tri_solve(hipStream_t s, bool lower, bool trans, bool unit,
-                            int k, int nrhs, const double* T, int ldt,
-                            double* X, int ldx) {
-  return tri_solve_t(s, lower, trans, unit, k, nrhs, T, ldt, X, ldx);
-}
-
-hipError_t launch_tri_solve(hipStream_t s, bool lower, bool trans, bool unit,
-                            int k, int nrhs, const float* T, int ldt, float* X,
-                            int ldx) {
-  return tri_solve_t(s, lower, trans, unit, k, nrhs, T, ldt, X, ldx);
-}
 
 hipError_t launch_linv(hipStream_t s, int jb, const double* L, int ldl,
                        double* Linv, int ldi) {
@@ -136,12 +113,12 @@ hipError_t launch_diag_inverse(hipStream_t s, bool lower, int nblk, int kb,
 
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const double* L,
                                 int ldl, double* B, int ldb) {
-  return launch_tri_solve(s, true, false, true, k, n, L, ldl, B, ldb);
+  return trsm_t(s, k, n, L, ldl, B, ldb);
 }
 
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const float* L,
                                 int ldl, float* B, int ldb) {
-  return launch_tri_solve(s, true, false, true, k, n, L, ldl, B, ldb);
+  return trsm_t(s, k, n, L, ldl, B, ldb);
 }
 
 }  // namespace hplx

@@ -1,13 +1,6 @@
-// Back-solve U x = b' (HPL_pdtrsv at P=Q=1, src/pgesv/HPL_pdtrsv_device.cpp:29-346).
-//
-// The reference walks the NB-blocks from the bottom with rocblas_dtrsv on the
-// diagonal block and two rocblas_dgemv calls for the rows above
-// (:169-180,195-332).  Here each block is one single-workgroup blocked solve
-// of the diagonal block (k_trsm.hip) followed by one HBM-bound GEMV over all
-// rows above,
-// with the block's columns split across the 4 waves of a workgroup so that
-// enough loads are in flight.  Every element of the upper triangle is read
-// exactly once.
+// Products of the solves: the GEMVs of the mixed-precision solves (rocblas_dgemv
+// at src/pgesv/HPL_pdtrsv_device.cpp:195-332), and the products with many
+// right-hand sides of the FP64 solves and the adjoint.
 #include "mxp.hpp"
 
 namespace hplx {
@@ -260,12 +253,6 @@ hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const __half* M,
   return gemv_sub_t(s, m, k, M, ldm, x, y, xback);
 }
 
-hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const double* M,
-                           int ldm, const double* x, double* y,
-                           double* xback) {
-  return gemv_sub_t(s, m, k, M, ldm, x, y, xback);
-}
-
 template <typename V>
 hipError_t inv_gemv_t(hipStream_t s, int k, const V* Inv, const V* x, V* y) {
   if(k <= 0) return hipSuccess;
@@ -339,27 +326,6 @@ hipError_t launch_outer_neg(hipStream_t s, int K, int m, int n,
   hipLaunchKernelGGL((tn_kernel<true, false, true, true>),
                      dim3(static_cast<unsigned>(tiles)), dim3(256), 0, s, K, m,
                      n, K, A, lda, B, ldb, C, ldc, tiles_m, tiles_n);
-  return hipGetLastError();
-}
-
-hipError_t launch_trsv(hipStream_t s, int n, int nb, const double* A, int lda,
-                       double* x) {
-  if(n <= 0) return hipSuccess;
-  if(nb <= 0 || nb > kMaxNB) nb = nb <= 0 ? 1 : kMaxNB;
-  const int nblk = (n + nb - 1) / nb;
-  for(int J = nblk - 1; J >= 0; --J) {
-    const int s0 = J * nb;
-    const int kb = (n - s0) < nb ? (n - s0) : nb;
-    hipError_t e = launch_tri_solve(s, false, false, false, kb, 1,
-                                    A + s0 + static_cast<size_t>(s0) * lda,
-                                    lda, x + s0, n);
-    if(e != hipSuccess) return e;
-    if(s0 > 0)
-      hipLaunchKernelGGL((gemv_sub_kernel<double, double>), dim3((s0 + 63) / 64),
-                         dim3(256), 0, s, s0, kb,
-                         A + static_cast<size_t>(s0) * lda, lda, x + s0, x,
-                         nullptr);
-  }
   return hipGetLastError();
 }
 

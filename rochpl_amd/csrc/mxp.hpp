@@ -85,9 +85,6 @@ hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const float* M,
 hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const __half* M,
                            int ldm, const double* x, double* y,
                            double* xback = nullptr);
-hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const double* M,
-                           int ldm, const double* x, double* y,
-                           double* xback = nullptr);
 hipError_t launch_gemv_sub(hipStream_t s, int m, int k, const float* M,
                            int ldm, const float* x, float* y,
                            float* xback = nullptr);

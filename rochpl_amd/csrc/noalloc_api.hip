@@ -10,13 +10,15 @@
 
 namespace {
 
-// Scratch of every call on one device: the composed pivots of a panel
-// (2 kMaxNB ints) and the split-K partial products of the transposed solve
-// (kMaxNB^2 doubles, the size hplx_pdgetrs gives them, so both entry points
-// split alike and return the same bits).  8 MiB + 8 KiB per device.
+// Scratch of every call on one device (hplx::FlowScratch): the split-K
+// partial products of the transposed solve (kMaxNB^2 doubles, the size
+// hplx_pdgetrs gives them, so both entry points split alike and return the
+// same bits), the exchange buffer and the composed interchanges and flags.
+// 16 MiB + 136 KiB per device.
 constexpr size_t kWorkDoubles = static_cast<size_t>(hplx::kMaxNB) * hplx::kMaxNB;
-constexpr size_t kPermInts    = 2 * static_cast<size_t>(hplx::kMaxNB);
-constexpr size_t kScratchBytes = kWorkDoubles * sizeof(double) + kPermInts * sizeof(int);
+constexpr size_t kScratchBytes =
+    (kWorkDoubles + hplx::kFlowX) * sizeof(double) +
+    (hplx::kFlowPerm + hplx::kFlowFlags) * sizeof(int);
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -54,17 +56,20 @@ int hplx_pdgetrs_noalloc(const hplx_pmat* mat, int trans, int nrhs, double* B,
      mat->ld < mat->n || nrhs < 0 || (nrhs > 0 && (!B || ldb < mat->n)) ||
      (trans != 0 && trans != 1))
     return HPLX_ERR_INVALID;
-  // the scratch holds the composed pivots of one panel of at most kMaxNB
+  // the scratch holds the composed interchanges of panels of at most kMaxNB
   if(mat->nb > hplx::kMaxNB) return HPLX_ERR_UNSUPPORTED;
   if(nrhs == 0 || mat->n == 0) return HPLX_SUCCESS;
   hipError_t e   = hipSuccess;
   void*      ptr = scratch_on_current_device(&e);
   if(!ptr) return HPLX_ERR_HIP;
-  double* work  = static_cast<double*>(ptr);
-  int*    permU = reinterpret_cast<int*>(work + kWorkDoubles);
+  hplx::FlowScratch w;
+  w.work         = static_cast<double*>(ptr);
+  w.work_doubles = kWorkDoubles;
+  w.x            = reinterpret_cast<unsigned long long*>(w.work + kWorkDoubles);
+  w.perm         = reinterpret_cast<int*>(w.x + hplx::kFlowX);
+  w.flags        = w.perm + hplx::kFlowPerm;
   e = hplx::getrs_enqueue(static_cast<hipStream_t>(stream), mat->A, mat->n,
-                          mat->nb, mat->ld, mat->ipiv, trans, nrhs, B, ldb,
-                          permU, work, kWorkDoubles);
+                          mat->nb, mat->ld, mat->ipiv, trans, nrhs, B, ldb, w);
   return e == hipSuccess ? HPLX_SUCCESS : HPLX_ERR_HIP;
 }
 
