@@ -446,8 +446,9 @@ struct Fp64Loop {
   // Columns [c0, c0 + n) right of panel k (c0 relative to the first column
   // after the panel): row swaps into W, U12 = L11^{-1} W over A12, and (when
   // the rows below exist and the streamed update takes the shape) U12^T
-  // into W.  Returns in *fast whether the streamed update applies.
-  int prepare(int k, int c0, int n, hipStream_t s, bool* fast) {
+  // into W.  Returns in *fast whether the streamed update applies (split: a
+  // claimed update follows, which only it can be).
+  int prepare(int k, int c0, int n, hipStream_t s, bool split, bool* fast) {
     const int j = k * nb, jb = width(k), m = N - j;
     double*   P   = A + j + static_cast<size_t>(j) * lda;
     double*   A12 = A + j + static_cast<size_t>(j + jb + c0) * lda;
@@ -467,7 +468,8 @@ struct Fp64Loop {
     *fast = false;
     if(m - jb > 0) {
       const int ldu = hplx::ut_ld(n);
-      *fast = hplx::update_fast_ok(m - jb, n, jb, P + jb, lda, ws->W, ldu,
+      *fast = (split || hplx::update_pays(m - jb, n)) &&
+              hplx::update_fast_ok(m - jb, n, jb, P + jb, lda, ws->W, ldu,
                                    lda - j - jb, ldu);
       if(*fast) HIPCHK(c, hplx::launch_transpose(s, jb, n, A12, lda, ws->W, ldu));
     }
@@ -584,7 +586,7 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
       // columns of panel k+1 first (all of them if there is no next panel)
       const int la_cols = jb1 > 0 ? jb1 : nt;
       const int rest    = nt - la_cols;
-      if((r = L.prepare(k, 0, la_cols, U, &fast)) ||
+      if((r = L.prepare(k, 0, la_cols, U, false, &fast)) ||
          (r = L.gemm(k, 0, la_cols, U, fast)))
         return r;
       // the CUs the next panel's leaves need
@@ -592,7 +594,7 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
       const bool overlap = la && jb1 > 0 && rest >= kMinOverlapCols &&
                            rR <= c.cus_per_xcd && rR < 28;
       if(overlap) {
-        if((r = L.prepare(k, la_cols, rest, U, &fast))) return r;
+        if((r = L.prepare(k, la_cols, rest, U, true, &fast))) return r;
         int* claim = c.claim + (k & 1) * hplx::kClaimInts;
         int* stop  = c.stop + (k & 1) * 32;
         HIPCHK(c, hplx::launch_zero_ints(U, claim, hplx::kClaimInts));
@@ -658,7 +660,7 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
         }
       } else {
         if(jb1 > 0 && (r = L.panel(k + 1, U))) return r;
-        if(rest > 0 && ((r = L.prepare(k, la_cols, rest, U, &fast)) ||
+        if(rest > 0 && ((r = L.prepare(k, la_cols, rest, U, false, &fast)) ||
                         (r = L.gemm(k, la_cols, rest, U, fast))))
           return r;
       }
@@ -851,7 +853,8 @@ int hplx_pdupdate(hplx_ctx* ctx, double* A, int lda, int m, int jb, int n,
     // the same two paths as the panel loop: U12^T into W and the streamed
     // update, or the general GEMM
     const int ldu = hplx::ut_ld(n);
-    if(hplx::update_fast_ok(m - jb, n, jb, A + jb, lda, W, ldu, lda - jb, ldu)) {
+    if(hplx::update_pays(m - jb, n) &&
+       hplx::update_fast_ok(m - jb, n, jb, A + jb, lda, W, ldu, lda - jb, ldu)) {
       HIPCHK(c, hplx::launch_transpose(s, jb, n, A12, lda, W, ldu));
       HIPCHK(c, hplx::launch_update(s, m - jb, n, jb, A + jb, lda, W, ldu,
                                     A12 + jb, lda, lda - jb, ldu));

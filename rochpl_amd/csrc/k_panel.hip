@@ -266,9 +266,8 @@ hipError_t launch_leaf(Ctx& c, V* P, int lda, int m, int JB, int c0, int w,
 }
 
 // C (m x n) -= A (m x k) B (k x n) inside the panel recursion
-// (rocblas_dgemm at src/pfact/HPL_pdrpanrlT.cpp:142-154).  FP64 products at
-// least one 128-column tile wide go through the streamed trailing-update
-// kernel with B transposed into the context's L11^{-1} buffer, which is idle
+// (rocblas_dgemm at src/pfact/HPL_pdrpanrlT.cpp:142-154).  Large FP64
+// products go through the streamed trailing-update kernel with B transposed into the context's L11^{-1} buffer, which is idle
 // while a panel is factored; the others, and FP32, through the generic GEMM.
 inline hipError_t panel_gemm(Ctx& c, int m, int n, int k, const double* A,
                              int lda, const double* B, int ldb, double* C,
@@ -281,7 +280,7 @@ inline hipError_t panel_gemm(Ctx& c, int m, int n, int k, const double* A,
   // of them is followed by a further column of the panel (B's first
   // column), so the extra element lies inside the panel's storage.
   const int a_rows = (m + 1) & ~1;
-  if(n >= 128 && static_cast<size_t>(k) * ldt <= static_cast<size_t>(kMaxNB) * kMaxNB &&
+  if(update_pays(m, n) && static_cast<size_t>(k) * ldt <= static_cast<size_t>(kMaxNB) * kMaxNB &&
      update_fast_ok(m, n, k, A, lda, Bt, ldt, a_rows, ldt)) {
     hipError_t e = launch_transpose(s, k, n, B, ldb, Bt, ldt);
     if(e != hipSuccess) return e;

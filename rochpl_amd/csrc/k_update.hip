@@ -48,6 +48,8 @@ namespace {
 
 using namespace upd;
 
+constexpr long kPaysTiles = 192;
+
 // kPanel marks the panel products (HPL_pdrpanrlT's GEMMs) so that kernel
 // traces tell them from the trailing update; the code is the same.
 template <bool kPanel>
@@ -156,6 +158,16 @@ __global__ __launch_bounds__(256) void transpose_kernel(
 }
 
 }  // namespace
+
+// The streamed update needs a transposed copy of U and 128 x 128 tiles to
+// share; where these leave CUs idle the small tiles of k_gemm.hip are faster
+// (3840 x 256 x 256, 60 tiles: 17 us against 38 + 5 for the copy; 8617 x 384 x
+// 384, 204 tiles, about 65 both; whole solves with N = 4096: 17.97 ms with
+// this update always, 15.6 with it from 96 tiles on, 15.6 from 192; N = 9001:
+// 46.9, 41.8, 41.1; the factorisation with N = 32768, NB = 896: 478, 472, 469).
+bool update_pays(int m, int n) {
+  return ((m + 127L) / 128) * ((n + 127L) / 128) >= kPaysTiles;
+}
 
 bool update_fast_ok(int m, int n, int k, const double* A, int lda,
                     const double* Bt, int ldb, int a_rows, int b_cols) {
