@@ -92,7 +92,7 @@ namespace {
 // The context's buffers as the solves' scratch (the L11^{-1} buffers are idle
 // outside the panel loops).
 hplx::FlowScratch flow_scratch(const Ctx& c) {
-  return {c.flow_x, c.Linv,
+  return {reinterpret_cast<unsigned long long*>(c.Linv2), c.Linv,
           static_cast<size_t>(hplx::kMaxNB) * hplx::kMaxNB, c.flow_perm,
           c.flow_flags};
 }
@@ -171,8 +171,7 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   size_t off_linv2  = align_up(off_dout + 256, 256);
   size_t off_perm2  = align_up(off_linv2 + nLinv, 256);
   size_t off_fperm  = align_up(off_perm2 + nperm, 256);
-  size_t off_fx     = align_up(off_fperm + hplx::kFlowPerm * sizeof(int), 256);
-  size_t off_fflags = align_up(off_fx + hplx::kFlowX * sizeof(double), 256);
+  size_t off_fflags = align_up(off_fperm + hplx::kFlowPerm * sizeof(int), 256);
   size_t off_claim  = align_up(off_fflags + hplx::kFlowFlags * sizeof(int), 256);
   size_t off_stop   = align_up(off_claim + 2 * hplx::kClaimInts * sizeof(int), 256);
   size_t off_vacate = off_stop + 256;
@@ -203,7 +202,6 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   c.permU2  = reinterpret_cast<int*>(b + off_perm2);
   c.flow_perm  = reinterpret_cast<int*>(b + off_fperm);
   c.flow_flags = reinterpret_cast<int*>(b + off_fflags);
-  c.flow_x     = reinterpret_cast<unsigned long long*>(b + off_fx);
   c.claim   = reinterpret_cast<int*>(b + off_claim);
   c.stop    = reinterpret_cast<int*>(b + off_stop);
   c.vacate  = reinterpret_cast<unsigned long long*>(b + off_vacate);

@@ -95,7 +95,6 @@ struct Ctx {
   int*      permU2     = nullptr;
   int*      flow_perm  = nullptr;    // kFlowPerm
   int*      flow_flags = nullptr;    // kFlowFlags
-  unsigned long long* flow_x = nullptr;  // kFlowX
   int*      claim      = nullptr;    // 2 sets of kClaimInts update-claim counters
   int*      stop       = nullptr;    // 2 flags: claims of update k stop
   unsigned long long* vacate = nullptr;  // kVacateSets x 8 words (see cu_sets)

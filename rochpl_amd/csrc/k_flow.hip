@@ -41,13 +41,14 @@
 // -> 2.78 ms (transposed 8.92 -> 3.51), one 9.27 -> 1.69, 512 15.2 -> 9.9;
 // N = 5000, NB = 128, one 2.87 -> 0.77 ms.  The floor is one read of the
 // factors (2.1 GB, 0.4 ms).
-#include <utility>
-
 #include "hplx_internal.hpp"
 #include "lds_stream.hpp"
+#include "tri_chain.hpp"
 
 namespace hplx {
 namespace {
+
+using namespace tri;
 
 typedef double ud4 __attribute__((ext_vector_type(4)));
 // two neighbouring doubles at any 8-byte address
@@ -67,63 +68,6 @@ constexpr int kNarrowGrid = 512;
 // kSplitRows rows are updated by the GEMM of k_trsv.hip, which reads T once
 // per 64 of them.
 constexpr int kSplitRhs = 192, kSplitRows = 512;
-// A half's triangle in LDS holds, of its columns in pairs, the positions from
-// 16 (c / 16) on (positions: rows in the order they are solved); the index of
-// the entry at position p is tri_col(c) + 2 p.
-__host__ __device__ constexpr int tri_col(int c) {
-  const int b = c / 16;  // 16 columns of 64, of 48, of 32, of 16 entries
-  return 16 * (64 * b - 8 * b * (b - 1)) + (c - 16 * b) / 2 * 2 * (64 - 16 * b) -
-         32 * b + (c & 1);
-}
-constexpr int kTri = 16 * (64 + 48 + 32 + 16);
-
-// y -= x_J m for a column J of a half's triangle: x_J is lane J's of each 16
-// (4 right-hand sides side by side), m is -T(., J).  One asm per column, the
-// rows further on first: s_nop covers the VALU write of x just before.  Every
-// lane has to be active.
-#define HPLX_FMA(y, x, m, j) \
-  "v_fmac_f64_dpp %" #y ", %" #x ", %" #m " row_newbcast:%" #j " row_mask:0xf bank_mask:0xf\n\t"
-template <int S, int J>
-__device__ __forceinline__ void tri_column(double (&x)[4], const double (&m)[4]) {
-  if constexpr(S == 0)
-    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 5, 8) HPLX_FMA(2, 0, 6, 8) HPLX_FMA(3, 0, 7, 8)
-            HPLX_FMA(0, 0, 4, 8)
-        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
-        : "v"(m[0]), "v"(m[1]), "v"(m[2]), "v"(m[3]), "n"(J));
-  if constexpr(S == 1)
-    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 4, 6) HPLX_FMA(2, 0, 5, 6) HPLX_FMA(0, 0, 3, 6)
-        : "+v"(x[1]), "+v"(x[2]), "+v"(x[3])
-        : "v"(m[1]), "v"(m[2]), "v"(m[3]), "n"(J));
-  if constexpr(S == 2)
-    asm("s_nop 1\n\t" HPLX_FMA(1, 0, 3, 4) HPLX_FMA(0, 0, 2, 4)
-        : "+v"(x[2]), "+v"(x[3])
-        : "v"(m[2]), "v"(m[3]), "n"(J));
-  if constexpr(S == 3)
-    asm("s_nop 1\n\t" HPLX_FMA(0, 0, 1, 2) : "+v"(x[3]) : "v"(m[3]), "n"(J));
-}
-#undef HPLX_FMA
-
-// Columns 16 S + 2 J2 and the next; p: the triangle + 2 (lane % 16).
-typedef double d2a __attribute__((ext_vector_type(2)));
-template <int S, int J2>
-__device__ __forceinline__ void tri_pair(double (&x)[4], const double* p) {
-  constexpr int c = tri_col(16 * S + 2 * J2);
-  double        m0[4], m1[4];
-#pragma unroll
-  for(int s = S; s < 4; ++s) {
-    const d2a v = *reinterpret_cast<const d2a*>(p + c + 32 * s);
-    m0[s]       = v.x;
-    m1[s]       = v.y;
-  }
-  tri_column<S, 2 * J2>(x, m0);
-  tri_column<S, 2 * J2 + 1>(x, m1);
-}
-template <int S, int... J2>
-__device__ __forceinline__ void tri_columns(double (&x)[4], const double* p,
-                                            std::integer_sequence<int, J2...>) {
-  (tri_pair<S, J2>(x, p), ...);
-}
-
 struct FlowArgs {
   const double* T;
   int           ldt;
@@ -448,11 +392,10 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         const int q = 16 * s + m;
         v[s]        = xc[BACK ? kFH - 1 - q : q] * (UNIT ? 1.0 : scale[kFH * h + q]);
       }
-      typedef std::make_integer_sequence<int, 8> Pairs;
-      tri_columns<0>(v, p, Pairs());
-      tri_columns<1>(v, p, Pairs());
-      tri_columns<2>(v, p, Pairs());
-      tri_columns<3>(v, p, Pairs());
+      tri_columns<0>(v, p);
+      tri_columns<1>(v, p);
+      tri_columns<2>(v, p);
+      tri_columns<3>(v, p);
       const bool fine = fabs(v[0]) <= kHuge && fabs(v[1]) <= kHuge && fabs(v[2]) <= kHuge &&
                         fabs(v[3]) <= kHuge;
       // which path a right-hand side takes does not depend on the others

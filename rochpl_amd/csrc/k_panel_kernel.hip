@@ -11,8 +11,8 @@
 //     pivot exchange through the same candidate slots, one sequence number
 //     per leaf;
 //   - a triangular solve gives each workgroup right-hand-side columns
-//     b, b + G, ... (tri_solve.hpp, the same per-column routine as
-//     tri_solve_kernel);
+//     b, b + G, ... (tri_solve.hpp, one at a time, with the order of
+//     operations of k_trsm.hip);
 //   - a product first transposes its U block into the scratch buffer (32 x 32
 //     tiles through LDS), passes a barrier, then runs the streamed update's
 //     128 x 128 tiles b, b + G, ... (update_tile.hpp, the routine of the
@@ -135,9 +135,8 @@ __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
     } else if(o.kind == kPanelTrsm) {
       const double* T = a.P + o.ar + static_cast<size_t>(o.ac) * a.lda;
       for(int col = b; col < o.n; col += G)
-        trs::tri_solve_col<double, double, true, false, true, false>(
-            o.k, T, a.lda, a.P + o.br + static_cast<size_t>(o.bc + col) * a.lda,
-            col);
+        trs::tri_solve_col(o.k, T, a.lda,
+                           a.P + o.br + static_cast<size_t>(o.bc + col) * a.lda);
     } else {
       const int rows = o.m_fix >= 0 ? o.m_fix : a.m - o.m_sub;
       if(rows <= 0) continue;  // uniform over the grid: no barrier owed

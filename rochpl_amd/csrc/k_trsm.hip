@@ -1,68 +1,223 @@
-// Triangular solves on one diagonal block (k <= 1024), one workgroup per
-// right-hand-side column:  op(T) x = b in place, op(T) = T or T^T.
+// Triangular solves on one diagonal block (k <= 1024), 16 right-hand sides per
+// workgroup:  T x = b in place.
 //
 // Used for the unit-lower L11 solves of the panel recursion and of the
 // trailing update (rocblas_dtrsm at src/pfact/HPL_pdrpanrlT.cpp:124-135 and
 // src/pgesv/HPL_pdupdateTT.cpp:95-106), for the explicit inverse of L11, and
-// (diag_inv_kernel) for the FP32 or FP64 inverses of the diagonal blocks of
-// the mixed-precision factors.
+// for the FP32 or FP64 inverses of the diagonal blocks of the mixed-precision
+// factors.
 //
 // x lives in LDS.  The block is processed in 64-row chunks along the sweep
-// direction: wave 0 solves the chunk's 64 x 64 triangle with the chunk's rows
-// of op(T) in registers (one row per lane) and x broadcast by lane shuffles;
-// then every thread applies the chunk's 64 columns to the rows still to be
-// solved, with all 64 loads of a row issued before the first product (the
-// block is latency bound: one workgroup per column).  One workgroup barrier
-// per 64 rows.
+// direction: 4 of the waves solve the chunk's triangle for 4 right-hand sides
+// each (tri_chain.hpp), then all apply the chunk's 64 columns to the
+// rows still to be solved, 16 rows at a time, by 16 x 16 x 4 MFMAs, T straight
+// from memory into the operand registers.  An MFMA's result is the chain of
+// its four FMAs in order, so a row's sum over a chunk has the bits of the plain
+// loop over the 64 columns.  Two workgroup barriers per 64 rows; the next
+// triangle and the first rows' operands are loaded while a triangle is solved.
+//
+// Bound by latency: a chunk costs a substitution, a product and the barriers,
+// 6 us with 1024 rows.  With one workgroup per right-hand side each of them
+// read all of T; us then and now: the inverse of 1024 x 1024 in FP32 357, 97;
+// FP64 256 x 256 35, 20; FP64 896 x 896 on the CUs beside an update 462, 138;
+// a solve with 32 x 32 and 32 right-hand sides 9.5, 6; all inverses for the
+// correction solves of N = 32768 with FP16 factors 8490, 1460.
 #include "mxp.hpp"
-#include "tri_solve.hpp"
+#include "tri_chain.hpp"
 
 namespace hplx {
 namespace {
 
-using namespace trs;
+using namespace tri;
 
-template <typename MT, typename V, bool LOWER, bool TRANS, bool UNIT,
-          bool IDENTITY>
-__global__ __launch_bounds__(256) void tri_solve_kernel(
-    int k, const MT* __restrict__ T, int ldt, V* __restrict__ X, int ldx) {
-  tri_solve_col<MT, V, LOWER, TRANS, UNIT, IDENTITY>(
-      k, T, ldt, X + static_cast<size_t>(blockIdx.x) * ldx, blockIdx.x);
+template <typename V>
+using vec4_t = V __attribute__((ext_vector_type(4)));
+
+template <typename V>
+__device__ inline vec4_t<V> mfma16x16x4(V a, V b, vec4_t<V> c) {
+  if constexpr(sizeof(V) == 8)
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Inverses (in V: FP64 or FP32) of consecutive kb x kb diagonal blocks of T:
-// block J (blockIdx.y) starts at T[J kb, J kb]; column blockIdx.x of its
-// inverse goes to Inv + (J kb + col) kb (each inverse column-major with
-// leading dimension kb).  LOWER: unit lower triangle; else the upper
-// triangle.
-template <typename MT, typename V, bool LOWER>
-__global__ __launch_bounds__(256) void diag_inv_kernel(int kb,
-                                                       const MT* __restrict__ T,
-                                                       int ldt,
-                                                       V* __restrict__ Inv) {
-  const size_t J = blockIdx.y;
-  tri_solve_col<MT, V, LOWER, false, LOWER, true>(
-      kb, T + J * kb * (1 + static_cast<size_t>(ldt)), ldt,
-      Inv + (J * kb + blockIdx.x) * kb, blockIdx.x);
+template <typename V, typename MT>
+__device__ inline V to_v(MT x) {
+  if constexpr(sizeof(MT) == 2)
+    return static_cast<V>(__half2float(x));
+  else
+    return static_cast<V>(x);
 }
 
 template <typename V>
-hipError_t trsm_t(hipStream_t s, int k, int n, const V* L, int ldl, V* B,
-                  int ldb) {
-  if(k <= 0 || n <= 0) return hipSuccess;
-  if(k > kMaxNB) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((tri_solve_kernel<V, V, true, false, true, false>), dim3(n),
-                     dim3(256), 0, s, k, L, ldl, B, ldb);
-  return hipGetLastError();
+constexpr V kLargest = sizeof(V) == 8 ? V(1.7976931348623157e308) : V(3.40282347e38);
+
+constexpr int kTriThreads = 512;
+
+// 16 columns of X per workgroup, of problem blockIdx.y (T and X advance by
+// t_step and x_step).  LOWER: unit lower triangle, forward; else upper,
+// backward.  IDENTITY: the right-hand sides are the identity's columns (X is
+// only written).  V: element type of X and of the arithmetic; MT: of T.  KM:
+// the largest k.
+template <typename MT, typename V, bool LOWER, bool IDENTITY, int KM>
+__global__ __launch_bounds__(kTriThreads) void tri_kernel(int k, int n, const MT* __restrict__ T,
+                                                  int ldt, size_t t_step,
+                                                  V* __restrict__ X, int ldx,
+                                                  size_t x_step) {
+  constexpr int LX = KM + 1, NC = 16, NW = kTriThreads / 64;
+  __shared__ __attribute__((aligned(16))) V tri[kTri];
+  __shared__ V sx[NC * LX];
+  __shared__ V sd[64];
+  T += blockIdx.y * t_step;
+  X += blockIdx.y * x_step;
+  const int t = threadIdx.x, lane = t & 63, m = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int col0 = blockIdx.x * NC, nc = min(NC, n - col0);
+  const int nchunk = (k + 63) / 64;
+  // with the identity, the rows before its columns in sweep order stay zero
+  const int first =
+      IDENTITY ? (LOWER ? col0 / 64 : nchunk - 1 - min(col0 + NC - 1, k - 1) / 64) : 0;
+  auto chunk_row = [&](int s) { return 64 * (LOWER ? s : nchunk - 1 - s); };
+  auto row       = [&](int p) { return LOWER ? p : 63 - p; };
+  // a chunk's triangle: lane = position, the wave's columns NW q + wave (clamped
+  // into the block), and its diagonal
+  constexpr int QT = 64 / NW;
+  MT   tr[QT], td;
+  auto load_triangle = [&](int c0) {
+    const int i = min(c0 + row(lane), k - 1);
+#pragma unroll
+    for(int q = 0; q < QT; ++q)
+      tr[q] = T[i + static_cast<size_t>(min(c0 + row(NW * q + wave), k - 1)) * ldt];
+    if(!LOWER) td = T[i + static_cast<size_t>(i) * ldt];
+  };
+  // rows [r, r + 16) of the chunk's columns as an MFMA operand
+  auto load_rows = [&](int r, int c0, MT(&a)[16]) {
+    const int i = min(r + m, k - 1);
+#pragma unroll
+    for(int q = 0; q < 16; ++q)
+      a[q] = T[i + static_cast<size_t>(min(c0 + 4 * q + g, k - 1)) * ldt];
+  };
+  load_triangle(chunk_row(first));
+  for(int c = wave; c < NC; c += NW)
+    for(int i = lane; i < k; i += 64)
+      sx[c * LX + i] = IDENTITY   ? (i == col0 + c ? V(1) : V(0))
+                       : c < nc ? X[i + static_cast<size_t>(col0 + c) * ldx]
+                                : V(0);
+  for(int s = first; s < nchunk; ++s) {
+    const int c0 = chunk_row(s), w = min(64, k - c0);
+#pragma unroll
+    for(int q = 0; q < QT; ++q) {
+      const int c = NW * q + wave;  // column and row of the triangle: positions
+      if(lane >= (c & ~15))
+        tri[tri_col(c) + 2 * lane] =
+            lane > c && row(lane) < w && row(c) < w ? -to_v<V>(tr[q]) : V(0);
+    }
+    if(!LOWER && wave == 0) sd[lane] = row(lane) < w ? to_v<V>(td) : V(1);
+    __syncthreads();
+    if(s + 1 < nchunk) load_triangle(chunk_row(s + 1));
+    const int r0 = LOWER ? c0 + w : 0, r1 = LOWER ? k : c0;
+    MT        a[16], an[16];
+    if(r0 + 16 * wave < r1) load_rows(r0 + 16 * wave, c0, an);
+    if(wave < 4) {
+      V*       xc = sx + (4 * wave + g) * LX + c0;
+      const V* p  = tri + 2 * m;
+      V        v[4], d[4];
+#pragma unroll
+      for(int q = 0; q < 4; ++q) {
+        const int i = row(16 * q + m);
+        v[q]        = i < w ? xc[i] : V(0);
+        d[q]        = LOWER ? V(1) : sd[16 * q + m];
+      }
+      tri_columns<0, LOWER>(v, p, d[0]);
+      if(!LOWER || w > 16) tri_columns<1, LOWER>(v, p, d[1]);
+      if(!LOWER || w > 32) tri_columns<2, LOWER>(v, p, d[2]);
+      if(!LOWER || w > 48) tri_columns<3, LOWER>(v, p, d[3]);
+      bool fine = true;
+#pragma unroll
+      for(int q = 0; q < 4; ++q) fine = fine && fabs(v[q]) <= kLargest<V>;
+      const unsigned long long bad = __ballot(!fine);
+      if((bad >> (lane & 48)) & 0xffff) {
+        // values that are not finite, whose products with the triangle's zeros
+        // are not zero: the substitution as it is written
+        V u[4];
+#pragma unroll
+        for(int q = 0; q < 4; ++q) {
+          const int i = row(16 * q + m);
+          u[q]        = i < w ? xc[i] : V(0);
+        }
+        for(int pj = 0; pj < 64; ++pj) {
+          const int j = row(pj);
+          if(j >= w) continue;
+          V xj = V(0);
+#pragma unroll
+          for(int q = 0; q < 4; ++q)
+            if((pj >> 4) == q) {
+              xj = __shfl(u[q], pj & 15, 16);
+              if(!LOWER) xj = xj / sd[pj];
+              if(m == (pj & 15)) u[q] = xj;
+            }
+#pragma unroll
+          for(int q = 0; q < 4; ++q) {
+            const int pi = 16 * q + m, i = row(pi);
+            if(pi > pj && i < w)
+              u[q] = fma(-to_v<V>(T[c0 + i + static_cast<size_t>(c0 + j) * ldt]), xj, u[q]);
+          }
+        }
+#pragma unroll
+        for(int q = 0; q < 4; ++q) v[q] = u[q];
+      }
+#pragma unroll
+      for(int q = 0; q < 4; ++q) {
+        const int i = row(16 * q + m);
+        if(i < w) xc[i] = v[q];
+      }
+    }
+    __syncthreads();
+    // the chunk's columns times x, off the rows still to be solved
+    if(r0 + 16 * wave < r1) {
+      V xb[16];
+#pragma unroll
+      for(int q = 0; q < 16; ++q)
+        xb[q] = 4 * q + g < w ? sx[m * LX + c0 + 4 * q + g] : V(0);
+      for(int r = r0 + 16 * wave; r < r1; r += 16 * NW) {
+#pragma unroll
+        for(int q = 0; q < 16; ++q) a[q] = an[q];
+        if(r + 16 * NW < r1) load_rows(r + 16 * NW, c0, an);
+        vec4_t<V> acc{0, 0, 0, 0};
+#pragma unroll
+        for(int q = 0; q < 16; ++q)
+          acc = mfma16x16x4<V>(4 * q + g < w ? to_v<V>(a[q]) : V(0), xb[q], acc);
+#pragma unroll
+        for(int e = 0; e < 4; ++e) {
+          const int i = r + (sizeof(V) == 8 ? 4 * e + g : 4 * g + e);
+          if(i < r1) sx[m * LX + i] -= acc[e];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for(int c = wave; c < nc; c += NW)
+    for(int i = lane; i < k; i += 64)
+      X[i + static_cast<size_t>(col0 + c) * ldx] = sx[c * LX + i];
 }
 
-template <typename V>
-hipError_t linv_t(hipStream_t s, int jb, const V* L, int ldl, V* Linv,
-                  int ldi) {
-  if(jb <= 0) return hipSuccess;
-  if(jb > kMaxNB) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((tri_solve_kernel<V, V, true, false, true, true>), dim3(jb),
-                     dim3(256), 0, s, jb, L, ldl, Linv, ldi);
+// The instance with the least LDS: more workgroups to a CU.
+template <bool LOWER, bool IDENTITY, typename MT, typename V>
+hipError_t tri_solve(hipStream_t s, int k, int n, int blocks, const MT* T, int ldt,
+                     size_t t_step, V* X, int ldx, size_t x_step) {
+  if(k <= 0 || n <= 0 || blocks <= 0) return hipSuccess;
+  if(k > kMaxNB || blocks > 65535) return hipErrorInvalidValue;
+  const dim3 g((n + 15) / 16, blocks), b(kTriThreads);
+  static_assert(kMaxNB <= 1024, "tri_kernel's largest instance");
+  if(k <= 128)
+    hipLaunchKernelGGL((tri_kernel<MT, V, LOWER, IDENTITY, 128>), g, b, 0, s, k, n, T, ldt,
+                       t_step, X, ldx, x_step);
+  else if(k <= 512)
+    hipLaunchKernelGGL((tri_kernel<MT, V, LOWER, IDENTITY, 512>), g, b, 0, s, k, n, T, ldt,
+                       t_step, X, ldx, x_step);
+  else
+    hipLaunchKernelGGL((tri_kernel<MT, V, LOWER, IDENTITY, 1024>), g, b, 0, s, k, n, T, ldt,
+                       t_step, X, ldx, x_step);
   return hipGetLastError();
 }
 
@@ -70,55 +225,54 @@ hipError_t linv_t(hipStream_t s, int jb, const V* L, int ldl, V* Linv,
 
 hipError_t launch_linv(hipStream_t s, int jb, const double* L, int ldl,
                        double* Linv, int ldi) {
-  return linv_t(s, jb, L, ldl, Linv, ldi);
+  return tri_solve<true, true>(s, jb, jb, 1, L, ldl, 0, Linv, ldi, 0);
 }
 
 hipError_t launch_linv(hipStream_t s, int jb, const float* L, int ldl,
                        float* Linv, int ldi) {
-  return linv_t(s, jb, L, ldl, Linv, ldi);
+  return tri_solve<true, true>(s, jb, jb, 1, L, ldl, 0, Linv, ldi, 0);
 }
 
+// Block J starts at T[J kb, J kb], its inverse (leading dimension kb) at Inv +
+// J kb kb.
 template <typename MT, typename V>
-hipError_t diag_inverse_t(hipStream_t s, bool lower, int nblk, int kb,
-                          const MT* T, int ldt, V* Inv) {
+static hipError_t diag_inverse(hipStream_t s, bool lower, int nblk, int kb, const MT* T,
+                               int ldt, V* Inv) {
   if(nblk <= 0 || kb <= 0) return hipSuccess;
-  if(kb > kMaxNB || nblk > 65535) return hipErrorInvalidValue;
-  const dim3 g(kb, nblk);
-  if(lower)
-    hipLaunchKernelGGL((diag_inv_kernel<MT, V, true>), g, dim3(256), 0, s, kb, T, ldt, Inv);
-  else
-    hipLaunchKernelGGL((diag_inv_kernel<MT, V, false>), g, dim3(256), 0, s, kb, T, ldt, Inv);
-  return hipGetLastError();
+  const size_t t_step = kb * (1 + static_cast<size_t>(ldt));
+  const size_t x_step = kb * static_cast<size_t>(kb);
+  return lower ? tri_solve<true, true>(s, kb, kb, nblk, T, ldt, t_step, Inv, kb, x_step)
+               : tri_solve<false, true>(s, kb, kb, nblk, T, ldt, t_step, Inv, kb, x_step);
 }
 
 hipError_t launch_diag_inverse(hipStream_t s, bool lower, int nblk, int kb,
                                const float* T, int ldt, double* Inv) {
-  return diag_inverse_t(s, lower, nblk, kb, T, ldt, Inv);
+  return diag_inverse(s, lower, nblk, kb, T, ldt, Inv);
 }
 
 hipError_t launch_diag_inverse(hipStream_t s, bool lower, int nblk, int kb,
                                const __half* T, int ldt, double* Inv) {
-  return diag_inverse_t(s, lower, nblk, kb, T, ldt, Inv);
+  return diag_inverse(s, lower, nblk, kb, T, ldt, Inv);
 }
 
 hipError_t launch_diag_inverse(hipStream_t s, bool lower, int nblk, int kb,
                                const float* T, int ldt, float* Inv) {
-  return diag_inverse_t(s, lower, nblk, kb, T, ldt, Inv);
+  return diag_inverse(s, lower, nblk, kb, T, ldt, Inv);
 }
 
 hipError_t launch_diag_inverse(hipStream_t s, bool lower, int nblk, int kb,
                                const __half* T, int ldt, float* Inv) {
-  return diag_inverse_t(s, lower, nblk, kb, T, ldt, Inv);
+  return diag_inverse(s, lower, nblk, kb, T, ldt, Inv);
 }
 
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const double* L,
                                 int ldl, double* B, int ldb) {
-  return trsm_t(s, k, n, L, ldl, B, ldb);
+  return tri_solve<true, false>(s, k, n, 1, L, ldl, 0, B, ldb, 0);
 }
 
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const float* L,
                                 int ldl, float* B, int ldb) {
-  return trsm_t(s, k, n, L, ldl, B, ldb);
+  return tri_solve<true, false>(s, k, n, 1, L, ldl, 0, B, ldb, 0);
 }
 
 }  // namespace hplx
