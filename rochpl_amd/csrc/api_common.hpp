@@ -50,6 +50,37 @@ inline int sync_event(Ctx& c, size_t i, hipEvent_t* e) {
   return HPLX_SUCCESS;
 }
 
+// Room for the times of a factorisation of `panels` panels.
+inline int reserve_stamps(Ctx& c, int panels) {
+  if(panels <= c.stamp_panels) return HPLX_SUCCESS;
+  if(c.stamps) (void)hipFree(c.stamps);
+  c.stamps       = nullptr;
+  c.stamp_panels = 0;
+  HIPCHK(c, hipMalloc(&c.stamps, sizeof(long long) * 2 * kStampPairs * panels));
+  c.stamp_panels = panels;
+  return HPLX_SUCCESS;
+}
+
+// Pair i of the updates (kind 0), the interchanges (1) or the panels (2).
+inline long long* stamp_at(const Ctx& c, int kind, int i) {
+  constexpr int first[3] = {0, 3, 5};
+  return c.stamps + 2 * (static_cast<size_t>(first[kind]) * c.stamp_panels + i);
+}
+
+// The durations (ms) of the first n pairs of a kind.
+inline int stamp_times(Ctx& c, int kind, int n, std::vector<double>* ms) {
+  ms->assign(n, 0.0);
+  if(n == 0) return HPLX_SUCCESS;
+  int khz = 0;
+  HIPCHK(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
+  std::vector<long long> t(2 * static_cast<size_t>(n));
+  HIPCHK(c, hipMemcpy(t.data(), stamp_at(c, kind, 0), sizeof(long long) * t.size(),
+                      hipMemcpyDeviceToHost));
+  for(int i = 0; i < n; ++i)
+    (*ms)[i] = static_cast<double>(t[2 * i + 1] - t[2 * i]) / khz;
+  return HPLX_SUCCESS;
+}
+
 inline int use(hplx_ctx* ctx) {
   if(!ctx) return HPLX_ERR_INVALID;
   hipError_t e = hipSetDevice(ctx->c.device);

@@ -25,6 +25,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <numeric>
 
 #include "api_common.hpp"
 
@@ -229,11 +230,9 @@ int hplx_ctx_destroy(hplx_ctx* ctx) {
   (void)hipStreamSynchronize(c.stream);
   if(c.ustream) (void)hipStreamSynchronize(c.ustream);
   if(c.pstream) (void)hipStreamSynchronize(c.pstream);
-  for(hipEvent_t e : c.ev) (void)hipEventDestroy(e);
   for(hipEvent_t e : c.ev_prog) (void)hipEventDestroy(e);
   for(hipEvent_t e : c.ev_sync) (void)hipEventDestroy(e);
-  for(hipEvent_t e : c.ev_swap) (void)hipEventDestroy(e);
-  for(hipEvent_t e : c.ev_panel) (void)hipEventDestroy(e);
+  if(c.stamps) (void)hipFree(c.stamps);
   if(c.small_base) (void)hipFree(c.small_base);
   if(c.ustream) (void)hipStreamDestroy(c.ustream);
   if(c.pstream) (void)hipStreamDestroy(c.pstream);
@@ -410,6 +409,16 @@ struct Fp64Loop {
   int          N, nb, lda;
   hplx::PanelAlgo algo;
 
+  // where the end of the last update goes: noted by the next kernel that notes
+  // a time on the same stream
+  long long*  end        = nullptr;
+  hipStream_t end_stream = nullptr;
+  long long*  take_end(hipStream_t s) {
+    long long* t = s == end_stream ? end : nullptr;
+    if(t) end = nullptr;
+    return t;
+  }
+
   double* Linv(int k) const { return (k & 1) ? c.Linv2 : c.Linv; }
   int*    permU(int k) const { return (k & 1) ? c.permU2 : c.permU; }
   int     width(int k) const { return (N - k * nb) < nb ? (N - k * nb) : nb; }
@@ -421,23 +430,17 @@ struct Fp64Loop {
     double*   P = A + j + static_cast<size_t>(j) * lda;
     c.panel_stream_  = s;
     c.panel_scratch_ = Linv(k);
-    // the factorisation, timed by its own event pair
-    while(static_cast<int>(c.ev_panel.size()) < 2 * (c.panel_pairs + 1)) {
-      hipEvent_t ev;
-      HIPCHK(c, hipEventCreate(&ev));
-      c.ev_panel.push_back(ev);
-    }
-    HIPCHK(c, hipEventRecord(c.ev_panel[2 * c.panel_pairs], s));
+    // the factorisation, timed by its own pair
+    long long* t = hplx::stamp_at(c, 2, c.panel_pairs++);
+    HIPCHK(c, hplx::launch_stamp(s, {t, take_end(s)}));
     const hipError_t e = hplx::panel_factor(c, algo, P, lda, N - j, jb,
                                             mat->ipiv + j, j);
     c.panel_stream_  = nullptr;
     c.panel_scratch_ = nullptr;
     HIPCHK(c, e);
-    HIPCHK(c, hipEventRecord(c.ev_panel[2 * c.panel_pairs + 1], s));
-    ++c.panel_pairs;
     c.panel_bytes += 16.0 * (N - j) * static_cast<double>(jb);
-    HIPCHK(c, hplx::launch_pipid(s, jb, mat->ipiv + j, j, permU(k)));
-    HIPCHK(c, hplx::launch_linv(s, jb, P, lda, Linv(k), nb));
+    HIPCHK(c, hplx::launch_panel_tail(s, jb, mat->ipiv + j, j, permU(k), P, lda, Linv(k),
+                                      nb, {t + 1, nullptr}));
     return HPLX_SUCCESS;
   }
 
@@ -450,19 +453,14 @@ struct Fp64Loop {
     const int j = k * nb, jb = width(k), m = N - j;
     double*   P   = A + j + static_cast<size_t>(j) * lda;
     double*   A12 = A + j + static_cast<size_t>(j + jb + c0) * lda;
-    // the interchanges, timed by their own event pair
-    while(static_cast<int>(c.ev_swap.size()) < 2 * (c.swap_pairs + 1)) {
-      hipEvent_t e;
-      HIPCHK(c, hipEventCreate(&e));
-      c.ev_swap.push_back(e);
-    }
-    HIPCHK(c, hipEventRecord(c.ev_swap[2 * c.swap_pairs], s));
-    HIPCHK(c, hplx::launch_swap_gather(s, jb, n, A12, lda, permU(k), ws->W, nb));
-    HIPCHK(c, hipEventRecord(c.ev_swap[2 * c.swap_pairs + 1], s));
-    ++c.swap_pairs;
+    // the interchanges, timed by their own pair
+    long long* t = hplx::stamp_at(c, 1, c.swap_pairs++);
+    HIPCHK(c, hplx::launch_swap_gather(s, jb, n, A12, lda, permU(k), ws->W, nb,
+                                       {t, take_end(s)}));
     c.swap_bytes += 4.0 * 8.0 * jb * static_cast<double>(n);
     HIPCHK(c, hplx::launch_dgemm(s, jb, n, jb, 1.0, Linv(k), nb, ws->W, nb,
-                                 0.0, A12, lda, true));
+                                 0.0, A12, lda, true, 0, false, false,
+                                 {t + 1, nullptr}));
     *fast = false;
     if(m - jb > 0) {
       const int ldu = hplx::ut_ld(n);
@@ -474,22 +472,24 @@ struct Fp64Loop {
     return HPLX_SUCCESS;
   }
 
-  // A22 -= L21 U12 on those columns in one launch, timed by an event pair.
+  // A22 -= L21 U12 on those columns in one launch, timed by a pair.
   int gemm(int k, int c0, int n, hipStream_t s, bool fast) {
     const int j = k * nb, jb = width(k), m = N - j;
     if(m - jb <= 0) return HPLX_SUCCESS;
     double* P   = A + j + static_cast<size_t>(j) * lda;
     double* A12 = A + j + static_cast<size_t>(j + jb + c0) * lda;
-    hipEvent_t e0 = c.ev[2 * c.ev_pairs], e1 = c.ev[2 * c.ev_pairs + 1];
-    HIPCHK(c, hipEventRecord(e0, s));
+    long long* t = hplx::stamp_at(c, 0, c.ev_pairs);
     if(fast)
       HIPCHK(c, hplx::launch_update(s, m - jb, n, jb, P + jb, lda, ws->W,
                                     hplx::ut_ld(n), A12 + jb, lda,
-                                    lda - j - jb, hplx::ut_ld(n)));
+                                    lda - j - jb, hplx::ut_ld(n), false,
+                                    {t, nullptr}));
     else
       HIPCHK(c, hplx::launch_dgemm(s, m - jb, n, jb, -1.0, P + jb, lda, A12,
-                                   lda, 1.0, A12 + jb, lda, false, 1));
-    HIPCHK(c, hipEventRecord(e1, s));
+                                   lda, 1.0, A12 + jb, lda, false, 1, false, false,
+                                   {t, nullptr}));
+    end = t + 1;
+    end_stream = s;
     c.ev_kind[c.ev_pairs]  = 1;
     c.ev_flops[c.ev_pairs] = 2.0 * (m - jb) * static_cast<double>(n) * jb;
     c.gemm_flops += c.ev_flops[c.ev_pairs];
@@ -535,11 +535,7 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
   Fp64Loop L{c, mat, static_cast<hplx::MatWs*>(mat->ws), mat->A, N, nb, lda,
              hplx::panel_algo(*palg)};
   const int npanels = (N + nb - 1) / nb;
-  while(static_cast<int>(c.ev.size()) < 6 * npanels) {
-    hipEvent_t e;
-    HIPCHK(c, hipEventCreate(&e));
-    c.ev.push_back(e);
-  }
+  if((r = hplx::reserve_stamps(c, npanels))) return r;
   c.ev_pairs   = 0;
   c.gemm_flops = 0.0;
   c.swap_pairs = 0;
@@ -581,22 +577,22 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
     const int jb1 = k + 1 < npanels ? L.width(k + 1) : 0;
     bool      fast;
     if(nt > 0) {
-      // columns of panel k+1 first (all of them if there is no next panel)
       const int la_cols = jb1 > 0 ? jb1 : nt;
       const int rest    = nt - la_cols;
-      if((r = L.prepare(k, 0, la_cols, U, false, &fast)) ||
-         (r = L.gemm(k, 0, la_cols, U, fast)))
-        return r;
       // the CUs the next panel's leaves need
       const int rR = hplx::vacate_set_size(N - j - jb);
       const bool overlap = la && jb1 > 0 && rest >= kMinOverlapCols &&
-                           rR <= c.cus_per_xcd && rR < 28;
+                           rR <= c.cus_per_xcd && rR < 28 &&
+                           static_cast<double>(N - j - jb) * rest * jb >= hplx::kMinOverlapWork;
       if(overlap) {
-        if((r = L.prepare(k, la_cols, rest, U, true, &fast))) return r;
+        // columns of panel k+1 first
+        if((r = L.prepare(k, 0, la_cols, U, false, &fast)) ||
+           (r = L.gemm(k, 0, la_cols, U, fast)) ||
+           (r = L.prepare(k, la_cols, rest, U, true, &fast)))
+          return r;
         int* claim = c.claim + (k & 1) * hplx::kClaimInts;
         int* stop  = c.stop + (k & 1) * 32;
-        HIPCHK(c, hplx::launch_zero_ints(U, claim, hplx::kClaimInts));
-        HIPCHK(c, hplx::launch_zero_ints(U, stop, 1));
+        HIPCHK(c, hplx::launch_zero_ints(U, claim, hplx::kClaimInts, stop));
         hipEvent_t ev_prep, ev_pan;
         if((r = sync_event(c, nev++, &ev_prep)) ||
            (r = sync_event(c, nev++, &ev_pan)))
@@ -622,34 +618,36 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
           };
           if(fast) {
             // the claimed part beside the panel, then the resume part; each
-            // timed by its own event pair
+            // timed by its own pair
             const int pc = pair(2);
-            HIPCHK(c, hipEventRecord(c.ev[2 * pc], U));
+            HIPCHK(c, hplx::launch_stamp(U, {hplx::stamp_at(c, 0, pc), nullptr}));
             HIPCHK(c, hplx::launch_update_claimed(
                           U, m - jb, rest, jb, Pk + jb, lda, L.ws->W, ldu,
                           A12 + jb, lda, lda - j - jb, ldu, claim,
                           c.vacate + 8 * (rR - 1), stop, 2 * c.num_cus));
-            HIPCHK(c, hipEventRecord(c.ev[2 * pc + 1], U));
+            HIPCHK(c, hplx::launch_stamp(U, {hplx::stamp_at(c, 0, pc) + 1, nullptr}));
             const int ns = static_cast<int>(c.splits.size());
             if(ns < hplx::kMaxClaimLog)
               HIPCHK(c, hplx::launch_claim_log(U, claim, m - jb, rest,
                                                c.claim_log + 8 * ns));
             HIPCHK(c, hipStreamWaitEvent(U, ev_pan, 0));
             const int pr = pair(3);
-            HIPCHK(c, hipEventRecord(c.ev[2 * pr], U));
+            HIPCHK(c, hplx::launch_stamp(U, {hplx::stamp_at(c, 0, pr), nullptr}));
             HIPCHK(c, hplx::launch_update_resume(
                           U, m - jb, rest, jb, Pk + jb, lda, L.ws->W, ldu,
                           A12 + jb, lda, lda - j - jb, ldu, claim));
-            HIPCHK(c, hipEventRecord(c.ev[2 * pr + 1], U));
+            L.end        = hplx::stamp_at(c, 0, pr) + 1;
+            L.end_stream = U;
             c.splits.push_back({m - jb, rest, jb, pc, pr});
           } else {
             HIPCHK(c, hipStreamWaitEvent(U, ev_pan, 0));
             const int p1 = pair(1);
-            HIPCHK(c, hipEventRecord(c.ev[2 * p1], U));
             HIPCHK(c, hplx::launch_dgemm(U, m - jb, rest, jb, -1.0, Pk + jb,
                                          lda, A12, lda, 1.0, A12 + jb, lda,
-                                         false, 1));
-            HIPCHK(c, hipEventRecord(c.ev[2 * p1 + 1], U));
+                                         false, 1, false, false,
+                                         {hplx::stamp_at(c, 0, p1), nullptr}));
+            L.end        = hplx::stamp_at(c, 0, p1) + 1;
+            L.end_stream = U;
             c.ev_flops[p1] = flops;
           }
           c.gemm_flops += flops;
@@ -657,9 +655,8 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
           HIPCHK(c, hipStreamWaitEvent(U, ev_pan, 0));
         }
       } else {
-        if(jb1 > 0 && (r = L.panel(k + 1, U))) return r;
-        if(rest > 0 && ((r = L.prepare(k, la_cols, rest, U, false, &fast)) ||
-                        (r = L.gemm(k, la_cols, rest, U, fast))))
+        if((r = L.prepare(k, 0, nt, U, false, &fast)) || (r = L.gemm(k, 0, nt, U, fast)) ||
+           (jb1 > 0 && (r = L.panel(k + 1, U))))
           return r;
       }
     } else if(jb1 > 0) {
@@ -667,6 +664,7 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
     }
     HIPCHK(c, prog.panel_queued(k, U));
   }
+  if(long long* t = L.take_end(U)) HIPCHK(c, hplx::launch_stamp(U, {t, nullptr}));
   if(la) {  // the caller's stream continues after U and P
     hipEvent_t eu, ep;
     if((r = sync_event(c, nev++, &eu)) || (r = sync_event(c, nev++, &ep))) return r;
@@ -920,13 +918,13 @@ int hplx_update_timing(hplx_ctx* ctx, int kind, double* ms, int* launches,
     fl[sp.pair_claimed] = took;
     fl[sp.pair_resume]  = total - took;
   }
+  std::vector<double> t;
+  if((r = hplx::stamp_times(c, 0, c.ev_pairs, &t))) return r;
   double tot = 0.0, f = 0.0;
   int    cnt = 0;
   for(int i = 0; i < c.ev_pairs; ++i) {
     if(kind && c.ev_kind[i] != kind) continue;
-    float t = 0.f;
-    HIPCHK(c, hipEventElapsedTime(&t, c.ev[2 * i], c.ev[2 * i + 1]));
-    tot += t;
+    tot += t[i];
     f += fl[i];
     ++cnt;
   }
@@ -942,13 +940,9 @@ int hplx_swap_timing(hplx_ctx* ctx, double* ms, int* launches,
   if(r) return r;
   Ctx& c = ctx->c;
   HIPCHK(c, hipStreamSynchronize(c.stream));
-  double tot = 0.0;
-  for(int i = 0; i < c.swap_pairs; ++i) {
-    float t = 0.f;
-    HIPCHK(c, hipEventElapsedTime(&t, c.ev_swap[2 * i], c.ev_swap[2 * i + 1]));
-    tot += t;
-  }
-  if(ms) *ms = tot;
+  std::vector<double> t;
+  if((r = hplx::stamp_times(c, 1, c.swap_pairs, &t))) return r;
+  if(ms) *ms = std::accumulate(t.begin(), t.end(), 0.0);
   if(launches) *launches = c.swap_pairs;
   if(bytes) *bytes = c.swap_bytes;
   return HPLX_SUCCESS;
@@ -960,13 +954,9 @@ int hplx_panel_timing(hplx_ctx* ctx, double* ms, int* panels,
   if(r) return r;
   Ctx& c = ctx->c;
   HIPCHK(c, hipStreamSynchronize(c.stream));
-  double tot = 0.0;
-  for(int i = 0; i < c.panel_pairs; ++i) {
-    float t = 0.f;
-    HIPCHK(c, hipEventElapsedTime(&t, c.ev_panel[2 * i], c.ev_panel[2 * i + 1]));
-    tot += t;
-  }
-  if(ms) *ms = tot;
+  std::vector<double> t;
+  if((r = hplx::stamp_times(c, 2, c.panel_pairs, &t))) return r;
+  if(ms) *ms = std::accumulate(t.begin(), t.end(), 0.0);
   if(panels) *panels = c.panel_pairs;
   if(bytes) *bytes = c.panel_bytes;
   return HPLX_SUCCESS;
@@ -978,13 +968,9 @@ int hplx_update_stats(hplx_ctx* ctx, double* gemm_ms, int* launches,
   if(r) return r;
   Ctx& c = ctx->c;
   HIPCHK(c, hipStreamSynchronize(c.stream));
-  double tot = 0.0;
-  for(int i = 0; i < c.ev_pairs; ++i) {
-    float ms = 0.f;
-    HIPCHK(c, hipEventElapsedTime(&ms, c.ev[2 * i], c.ev[2 * i + 1]));
-    tot += ms;
-  }
-  if(gemm_ms) *gemm_ms = tot;
+  std::vector<double> t;
+  if((r = hplx::stamp_times(c, 0, c.ev_pairs, &t))) return r;
+  if(gemm_ms) *gemm_ms = std::accumulate(t.begin(), t.end(), 0.0);
   if(launches) *launches = c.ev_pairs;
   if(gemm_flops) *gemm_flops = c.gemm_flops;
   return HPLX_SUCCESS;

@@ -39,6 +39,12 @@ inline int leaf_rpt(int R) {
 // shader engines (a workgroup waits for a CU of the engine it was handed to,
 // so an engine without a free CU would hold up the panel's kernels).
 constexpr int kMinOverlapCols = 256;
+// Products (m n k) of that rest from which it pays: two streams, their waits
+// and the second preparation cost about 0.1 ms a panel, the update this
+// hides less below (whole solves, from 0 / 2.5e9 / 6e9 / 1.5e10 products on:
+// N = 1000 2.81 / 2.46 / 2.46 / 2.48 ms, N = 4096 14.5 / 14.1 / 14.1 / 14.2,
+// N = 9001 39.1 / 38.1 / 38.4 / 39.9).
+constexpr double kMinOverlapWork = 2.5e9;
 inline int vacate_set_size(int rows) {
   const int g = (rows + kLeafThreads * kLeafRPT - 1) / (kLeafThreads * kLeafRPT);
   return (g + 31) / 32 * 4;
@@ -69,6 +75,15 @@ constexpr int kMaxPanelOps = 512;  // steps of one recorded panel
 // 32768 solves 21 % and 11 % slower with the kernel on every panel; 65536,
 // 98304 and 193280 within run-to-run spread).
 constexpr int kPanelKernelMinRows = 65536;
+
+// Where a kernel notes the time it starts (stamp.hpp); null: nowhere.
+struct Stamps {
+  long long* a = nullptr;
+  long long* b = nullptr;
+};
+// Pairs of times a panel step may take: 3 updates (the next panel's columns,
+// claimed, resumed), 2 interchanges, 1 panel.
+constexpr int kStampPairs = 6;
 
 // Per-context device state.  The small workspace (candidate slots, barrier
 // counter, flags, L11 inverse, composed pivots) lives with the context; the
@@ -138,21 +153,23 @@ struct Ctx {
   // counterpart of the reference's HPL_PROGRESS_REPORT build option)
   int                     progress_every = 0;
   std::vector<hipEvent_t> ev_prog;
-  // timing of the trailing-update GEMM launches of the last solve: one
-  // event pair per launch, its kind (1: a whole update in one launch, 2: the
-  // claimed part of a split update, 3: its resume part) and its flops (for
-  // kinds 2 and 3 filled from the claim log when the stats are read)
-  std::vector<hipEvent_t> ev;
+  // Timing of the last solve: pairs of times in device memory (stamp.hpp), for
+  // kStampPairs pairs per panel: first those of the trailing updates, then of
+  // the interchanges, then of the panels (stamp_at).
+  long long* stamps       = nullptr;
+  int        stamp_panels = 0;  // panels they have room for
+  // the trailing-update GEMM launches: one pair per launch, its kind (1: a
+  // whole update in one launch, 2: the claimed part of a split update, 3: its
+  // resume part) and its flops (for kinds 2 and 3 filled from the claim log
+  // when the stats are read)
   int                     ev_pairs = 0;
-  // the FP64 loop's row interchanges (swap_gather launches): one event pair
-  // per launch and their algorithmic bytes (4 x 8 B per interchanged element)
-  std::vector<hipEvent_t> ev_swap;
+  // the FP64 loop's row interchanges (swap_gather launches): one pair per
+  // launch and their algorithmic bytes (4 x 8 B per interchanged element)
   int                     swap_pairs = 0;
   double                  swap_bytes = 0.0;
-  // the FP64 loop's panel factorisations: one event pair per panel (on the
-  // stream it runs on) and their algorithmic bytes (the m x jb panel read
-  // and written once: 16 B per element)
-  std::vector<hipEvent_t> ev_panel;
+  // the FP64 loop's panel factorisations: one pair per panel (on the stream it
+  // runs on) and their algorithmic bytes (the m x jb panel read and written
+  // once: 16 B per element)
   int                     panel_pairs = 0;
   double                  panel_bytes = 0.0;
   double                  gemm_flops = 0.0;
@@ -262,13 +279,20 @@ hipError_t launch_panel_kernel(Ctx& c, int slot, double* P, int lda, int m,
 
 hipError_t launch_pipid(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
                         int* permU);
+// What follows a panel, in one launch: launch_pipid and launch_linv.
+hipError_t launch_panel_tail(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
+                             int* permU, const double* L, int ldl, double* Linv,
+                             int ldi, Stamps st = Stamps());
+hipError_t launch_panel_tail(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
+                             int* permU, const float* L, int ldl, float* Linv,
+                             int ldi, Stamps st = Stamps());
 // The same for np consecutive panels of nb rows (the last one of what is left
 // of `rows`): panel p's interchanges ipiv + p nb, relative to base + p nb,
 // into permU + 2 p nb.
 hipError_t launch_pipid_panels(hipStream_t s, int np, int nb, int rows,
                                const int* ipiv, int base, int* permU);
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, double* A,
-                              int lda, const int* permU, double* W, int ldw);
+                              int lda, const int* permU, double* W, int ldw, Stamps st = Stamps());
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, float* A, int lda,
                               const int* permU, float* W, int ldw);
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, __half* A,
@@ -279,8 +303,6 @@ hipError_t launch_swap_inverse(hipStream_t s, int jb, int n, double* A,
                                int lda, const int* permU);
 hipError_t launch_linv(hipStream_t s, int jb, const double* L, int ldl,
                        double* Linv, int ldi);
-hipError_t launch_linv(hipStream_t s, int jb, const float* L, int ldl,
-                       float* Linv, int ldi);
 // B (k x n) = L^{-1} B, L unit lower.
 hipError_t launch_trsm_colsweep(hipStream_t s, int k, int n, const double* L,
                                 int ldl, double* B, int ldb);
@@ -295,7 +317,7 @@ hipError_t launch_dgemm(hipStream_t s, int m, int n, int k, double alpha,
                         const double* A, int lda, const double* B, int ldb,
                         double beta, double* C, int ldc, bool lower_a,
                         int kind = 0, bool trans_a = false,
-                        bool trans_b = false);
+                        bool trans_b = false, Stamps st = Stamps());
 // The FP32 MFMA instance (no transposes, no trailing-update kind).
 hipError_t launch_sgemm(hipStream_t s, int m, int n, int k, double alpha,
                         const float* A, int lda, const float* B, int ldb,
@@ -314,7 +336,8 @@ bool       update_fast_ok(int m, int n, int k, const double* A, int lda,
 bool       update_pays(int m, int n);
 hipError_t launch_update(hipStream_t s, int m, int n, int k, const double* A,
                          int lda, const double* Bt, int ldb, double* C,
-                         int ldc, int a_rows, int b_cols, bool panel = false);
+                         int ldc, int a_rows, int b_cols, bool panel = false,
+                         Stamps st = Stamps());
 // The same update split between two launches for the look-ahead:
 // launch_update_claimed runs `grid` persistent workgroups (one per CU) that
 // take tiles through the per-XCD counters claim[0], claim[32], ...,
@@ -334,7 +357,10 @@ hipError_t launch_update_resume(hipStream_t s, int m, int n, int k,
                                 int ldb, double* C, int ldc, int a_rows,
                                 int b_cols, const int* claimed);
 constexpr int kClaimInts = 8 * 32;  // ints of one set of claim counters
-hipError_t launch_zero_ints(hipStream_t s, int* p, int n);
+// p[0:n] = 0 and, if q is not null, q[0] = 0.
+hipError_t launch_zero_ints(hipStream_t s, int* p, int n, int* q = nullptr);
+// The time at which the stream gets here.
+hipError_t launch_stamp(hipStream_t s, Stamps st);
 // *p = 1 with an agent-scope store (read by running kernels on any XCD).
 hipError_t launch_set_flag(hipStream_t s, int* p);
 // out[x] = min(claim[32 x], per) for the 8 XCD shares of a claimed update of

@@ -31,6 +31,7 @@
 //     kGroupM tile rows so that concurrently running tiles on one XCD share
 //     A and B strips in that XCD's L2.
 #include "hplx_internal.hpp"
+#include "stamp.hpp"
 
 namespace hplx {
 namespace {
@@ -269,7 +270,8 @@ template <typename V, bool BETA0, bool NEG, bool LOWER_A, bool TA, bool TB,
 __global__ __launch_bounds__(NT, 2) void dgemm_kernel(
     int M, int N, int K, const V* __restrict__ A, int lda,
     const V* __restrict__ B, int ldb, V* __restrict__ C, int ldc,
-    int tiles_m, int tiles_n) {
+    int tiles_m, int tiles_n, Stamps st) {
+  stamp_now(st);
   __shared__ __attribute__((aligned(16))) V sA[2][BK * LDS_LD];
   __shared__ __attribute__((aligned(16))) V sB[2][BK * LDS_LD];
 
@@ -406,7 +408,8 @@ template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN>
 __global__ __launch_bounds__(NT) void tile_kernel(
     int M, int N, int K, const V* __restrict__ A, int lda,
     const V* __restrict__ B, int ldb, V* __restrict__ C, int ldc, int tiles_m,
-    int tiles_n) {
+    int tiles_n, Stamps st) {
+  stamp_now(st);
   constexpr int BKS = 32, LA = BM + 2, LB = BN + 2;
   constexpr int TM = BM / 32, TN = BN / 32;
   constexpr int QA = BM * BKS / 2 / NT, QB = BN * BKS / 2 / NT;  // pairs per thread
@@ -569,21 +572,21 @@ Tile pick_tile(int m, int n) {
 
 template <bool BETA0, bool NEG, bool LOWER_A, int BM, int BN, typename V>
 hipError_t run_tile(hipStream_t s, int m, int n, int k, const V* A, int lda,
-                    const V* B, int ldb, V* C, int ldc) {
+                    const V* B, int ldb, V* C, int ldc, Stamps st) {
   const int  tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
   const long T    = static_cast<long>(tiles_m) * tiles_n;
   const long grid = (T + kXcds - 1) / kXcds * kXcds;
   if(grid > 0x7fffffffL) return hipErrorInvalidValue;
   hipLaunchKernelGGL((tile_kernel<V, BETA0, NEG, LOWER_A, BM, BN>),
                      dim3(static_cast<unsigned>(grid)), dim3(NT), 0, s, m, n, k, A, lda,
-                     B, ldb, C, ldc, tiles_m, tiles_n);
+                     B, ldb, C, ldc, tiles_m, tiles_n, st);
   return hipGetLastError();
 }
 
 template <bool BETA0, bool NEG, bool LOWER_A, bool TA, bool TB, int KIND,
           typename V>
 hipError_t run(hipStream_t s, int m, int n, int k, const V* A, int lda,
-               const V* B, int ldb, V* C, int ldc) {
+               const V* B, int ldb, V* C, int ldc, Stamps st) {
   const int  tiles_m = (m + BM - 1) / BM;
   const int  tiles_n = (n + BN - 1) / BN;
   const long T       = static_cast<long>(tiles_m) * tiles_n;
@@ -597,31 +600,32 @@ hipError_t run(hipStream_t s, int m, int n, int k, const V* A, int lda,
   if constexpr(!TA && !TB && BETA0 != NEG && !(NEG && LOWER_A))
     if(pair_aligned(A) && lda % 2 == 0 && pair_aligned(B) && ldb % 2 == 0 && k > 0)
       switch(pick_tile(m, n)) {
-        case kTile32: return run_tile<BETA0, NEG, LOWER_A, 32, 32>(s, m, n, k, A, lda, B, ldb, C, ldc);
-        case kTile64x32: return run_tile<BETA0, NEG, LOWER_A, 64, 32>(s, m, n, k, A, lda, B, ldb, C, ldc);
-        case kTile64: return run_tile<BETA0, NEG, LOWER_A, 64, 64>(s, m, n, k, A, lda, B, ldb, C, ldc);
+        case kTile32: return run_tile<BETA0, NEG, LOWER_A, 32, 32>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
+        case kTile64x32: return run_tile<BETA0, NEG, LOWER_A, 64, 32>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
+        case kTile64: return run_tile<BETA0, NEG, LOWER_A, 64, 64>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
         default: break;
       }
   const dim3 g(static_cast<unsigned>(grid)), b(NT);
   if(va && vb)
     hipLaunchKernelGGL((dgemm_kernel<V, BETA0, NEG, LOWER_A, TA, TB, true, true, KIND>),
-                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n);
+                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n, st);
   else if(va)
     hipLaunchKernelGGL((dgemm_kernel<V, BETA0, NEG, LOWER_A, TA, TB, true, false, KIND>),
-                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n);
+                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n, st);
   else if(vb)
     hipLaunchKernelGGL((dgemm_kernel<V, BETA0, NEG, LOWER_A, TA, TB, false, true, KIND>),
-                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n);
+                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n, st);
   else
     hipLaunchKernelGGL((dgemm_kernel<V, BETA0, NEG, LOWER_A, TA, TB, false, false, KIND>),
-                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n);
+                       g, b, 0, s, m, n, k, A, lda, B, ldb, C, ldc, tiles_m, tiles_n, st);
   return hipGetLastError();
 }
 
 template <typename V>
 hipError_t gemm_t(hipStream_t s, int m, int n, int k, double alpha,
                   const V* A, int lda, const V* B, int ldb, double beta, V* C,
-                  int ldc, bool lower_a, int kind, bool trans_a, bool trans_b) {
+                  int ldc, bool lower_a, int kind, bool trans_a, bool trans_b,
+                  Stamps st = Stamps()) {
   if(m <= 0 || n <= 0) return hipSuccess;
   if(!(alpha == 1.0 || alpha == -1.0) || !(beta == 0.0 || beta == 1.0))
     return hipErrorInvalidValue;
@@ -634,29 +638,29 @@ hipError_t gemm_t(hipStream_t s, int m, int n, int k, double alpha,
     if constexpr(sizeof(V) == 8) {
       if(lower_a || !neg) return hipErrorInvalidValue;
       if(trans_a && !trans_b)
-        return beta0 ? run<true, true, false, true, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                     : run<false, true, false, true, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
+        return beta0 ? run<true, true, false, true, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                     : run<false, true, false, true, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
       if(!trans_a && trans_b)
-        return beta0 ? run<true, true, false, false, true, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                     : run<false, true, false, false, true, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
+        return beta0 ? run<true, true, false, false, true, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                     : run<false, true, false, false, true, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
     }
     return hipErrorInvalidValue;
   }
   if(beta0) {
     if(neg)
-      return lower_a ? run<true, true, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                     : run<true, true, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
-    return lower_a ? run<true, false, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                   : run<true, false, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
+      return lower_a ? run<true, true, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                     : run<true, true, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
+    return lower_a ? run<true, false, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                   : run<true, false, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
   }
   if constexpr(sizeof(V) == 8)
     if(neg && !lower_a && kind == 1)
-      return run<false, true, false, false, false, 1>(s, m, n, k, A, lda, B, ldb, C, ldc);
+      return run<false, true, false, false, false, 1>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
   if(neg)
-    return lower_a ? run<false, true, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                   : run<false, true, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
-  return lower_a ? run<false, false, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc)
-                 : run<false, false, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc);
+    return lower_a ? run<false, true, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                   : run<false, true, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
+  return lower_a ? run<false, false, true, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st)
+                 : run<false, false, false, false, false, 0>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
 }
 
 }  // namespace
@@ -664,9 +668,9 @@ hipError_t gemm_t(hipStream_t s, int m, int n, int k, double alpha,
 hipError_t launch_dgemm(hipStream_t s, int m, int n, int k, double alpha,
                         const double* A, int lda, const double* B, int ldb,
                         double beta, double* C, int ldc, bool lower_a,
-                        int kind, bool trans_a, bool trans_b) {
+                        int kind, bool trans_a, bool trans_b, Stamps st) {
   return gemm_t(s, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower_a, kind,
-                trans_a, trans_b);
+                trans_a, trans_b, st);
 }
 
 hipError_t launch_sgemm(hipStream_t s, int m, int n, int k, double alpha,

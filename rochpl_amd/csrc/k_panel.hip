@@ -36,6 +36,8 @@
 #include <climits>
 
 #include "leaf.hpp"
+#include "pipid.hpp"
+#include "stamp.hpp"
 
 namespace hplx {
 namespace {
@@ -50,88 +52,22 @@ __global__ void reset_kernel(int* info, int* err) {
   *err  = 0;
 }
 
-// Device HPL_pipid: compose jb interchanges (row i <-> ipiv[i]-base) into
-// permU[0:jb] (source of each top row) and permU[jb:2jb] (destination of
-// each displaced top row, or -1), without a serial pass:
-//   position i < jb is last written at step i, with what position p_i held
-//   just before step i; a position q is written before step i only by the
-//   latest earlier step i' with p_i' = q, which moved there what position i'
-//   held just before step i'.  With g(i) = content of position i just before
-//   step i:
-//     g(i)       = g(last i' < i with p_i' = i), or i if none
-//     top[i]     = g(i) if p_i == i, else g(last i' < i with p_i' = p_i), or
-//                  p_i if none
-//     a position q >= jb ends with g(last i with p_i = q).
-//   Chains of g only go to smaller indices and are followed per thread.
-// One workgroup per panel (several for the solves with stored factors).
+// HPL_pipid of one panel per workgroup (pipid.hpp), of nb rows or what is left
+// of `rows`.
 __global__ __launch_bounds__(1024) void pipid_kernel(
     int nb, int rows, const int* __restrict__ ipiv, int base,
     int* __restrict__ permU) {
-  __shared__ int sp[kMaxNB];
-  __shared__ int sprev[kMaxNB];   // last i' < i with p_i' == p_i, or -1
-  __shared__ int sto[kMaxNB];     // last i' < i with p_i' == i, or -1
-  __shared__ int slast[kMaxNB];   // 1 if no later step targets p_i
-  __shared__ int sg[kMaxNB];
-  __shared__ int sout[2 * kMaxNB];
-  const int t = threadIdx.x, p0 = blockIdx.x * nb;
-  const int jb = min(nb, rows - p0);
-  ipiv += p0;
-  base += p0;
-  permU += 2 * static_cast<size_t>(p0);
-  // an interchange must target a row at or below its own; anything else is
-  // treated as no interchange so that every LDS index stays in range
-  for(int i = t; i < jb; i += blockDim.x) {
-    const int p = ipiv[i] - base;
-    sp[i]       = p < i ? i : p;
-  }
-  __syncthreads();
-  for(int i = t; i < jb; i += blockDim.x) {
-    int prev = -1, to = -1, last = 1;
-    const int p = sp[i];
-    for(int k2 = 0; k2 < jb; ++k2) {
-      const int q = sp[k2];
-      if(k2 < i) {
-        if(q == p) prev = k2;
-        if(q == i) to = k2;
-      } else if(k2 > i && q == p) {
-        last = 0;
-      }
-    }
-    sprev[i] = prev;
-    sto[i]   = to;
-    slast[i] = last;
-  }
-  __syncthreads();
-  for(int i = t; i < jb; i += blockDim.x) {
-    int j = i;
-    while(sto[j] >= 0) j = sto[j];  // strictly decreasing chain
-    sg[i] = j;
-  }
-  __syncthreads();
-  for(int i = t; i < jb; i += blockDim.x) {
-    const int p = sp[i];
-    int       top;
-    if(p == i)
-      top = sg[i];
-    else
-      top = sprev[i] >= 0 ? sg[sprev[i]] : p;
-    sout[i]      = top;
-    sout[jb + i] = -1;
-  }
-  __syncthreads();
-  for(int i = t; i < jb; i += blockDim.x)
-    if(sp[i] >= jb && slast[i]) sout[jb + sg[i]] = sp[i];
-  __syncthreads();
-  for(int i = t; i < 2 * jb; i += blockDim.x) permU[i] = sout[i];
+  __shared__ PipidShared sh;
+  const int p0 = blockIdx.x * nb;
+  pipid_block(min(nb, rows - p0), ipiv + p0, base + p0,
+              permU + 2 * static_cast<size_t>(p0), sh);
 }
 
-// New top rows -> W (ld ldw); displaced top rows -> their destinations.
-// S: storage type of A; WT: type of W (the FP16-stored factorisation gathers
-// into FP32).
 template <typename S, typename WT>
 __global__ __launch_bounds__(256) void swap_gather_kernel(
     int jb, S* __restrict__ A, int lda, const int* __restrict__ permU,
-    WT* __restrict__ W, int ldw) {
+    WT* __restrict__ W, int ldw, Stamps st) {
+  stamp_now(st);
   constexpr int Q   = kMaxNB / 256;
   const int     col = blockIdx.x;
   S*            ac  = A + static_cast<size_t>(col) * lda;
@@ -570,17 +506,17 @@ hipError_t launch_pipid_panels(hipStream_t s, int np, int nb, int rows,
 
 template <typename S, typename WT>
 hipError_t swap_gather_t(hipStream_t s, int jb, int n, S* A, int lda,
-                         const int* permU, WT* W, int ldw) {
+                         const int* permU, WT* W, int ldw, Stamps st = Stamps()) {
   if(jb <= 0 || n <= 0) return hipSuccess;
   if(jb > kMaxNB) return hipErrorInvalidValue;
   hipLaunchKernelGGL((swap_gather_kernel<S, WT>), dim3(n), dim3(256), 0, s, jb,
-                     A, lda, permU, W, ldw);
+                     A, lda, permU, W, ldw, st);
   return hipGetLastError();
 }
 
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, double* A, int lda,
-                              const int* permU, double* W, int ldw) {
-  return swap_gather_t(s, jb, n, A, lda, permU, W, ldw);
+                              const int* permU, double* W, int ldw, Stamps st) {
+  return swap_gather_t(s, jb, n, A, lda, permU, W, ldw, st);
 }
 
 hipError_t launch_swap_gather(hipStream_t s, int jb, int n, float* A, int lda,

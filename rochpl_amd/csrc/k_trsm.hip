@@ -23,6 +23,8 @@
 // a solve with 32 x 32 and 32 right-hand sides 9.5, 6; all inverses for the
 // correction solves of N = 32768 with FP16 factors 8490, 1460.
 #include "mxp.hpp"
+#include "pipid.hpp"
+#include "stamp.hpp"
 #include "tri_chain.hpp"
 
 namespace hplx {
@@ -54,25 +56,28 @@ constexpr V kLargest = sizeof(V) == 8 ? V(1.7976931348623157e308) : V(3.40282347
 
 constexpr int kTriThreads = 512;
 
-// 16 columns of X per workgroup, of problem blockIdx.y (T and X advance by
-// t_step and x_step).  LOWER: unit lower triangle, forward; else upper,
+// Columns [16 block, 16 block + 16) of X on one workgroup.  LOWER: unit lower triangle, forward; else upper,
 // backward.  IDENTITY: the right-hand sides are the identity's columns (X is
 // only written).  V: element type of X and of the arithmetic; MT: of T.  KM:
 // the largest k.
+template <typename V, int KM>
+struct TriShared {
+  alignas(16) V tri[kTri];
+  V sx[16 * (KM + 1)];
+  V sd[64];
+};
+
 template <typename MT, typename V, bool LOWER, bool IDENTITY, int KM>
-__global__ __launch_bounds__(kTriThreads) void tri_kernel(int k, int n, const MT* __restrict__ T,
-                                                  int ldt, size_t t_step,
-                                                  V* __restrict__ X, int ldx,
-                                                  size_t x_step) {
+__device__ __forceinline__ void tri_block(int k, int n, const MT* __restrict__ T, int ldt,
+                                          V* __restrict__ X, int ldx, int block,
+                                          TriShared<V, KM>& sh) {
   constexpr int LX = KM + 1, NC = 16, NW = kTriThreads / 64;
-  __shared__ __attribute__((aligned(16))) V tri[kTri];
-  __shared__ V sx[NC * LX];
-  __shared__ V sd[64];
-  T += blockIdx.y * t_step;
-  X += blockIdx.y * x_step;
+  V* const tri = sh.tri;
+  V* const sx  = sh.sx;
+  V* const sd  = sh.sd;
   const int t = threadIdx.x, lane = t & 63, m = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int col0 = blockIdx.x * NC, nc = min(NC, n - col0);
+  const int col0 = block * NC, nc = min(NC, n - col0);
   const int nchunk = (k + 63) / 64;
   // with the identity, the rows before its columns in sweep order stay zero
   const int first =
@@ -201,6 +206,52 @@ __global__ __launch_bounds__(kTriThreads) void tri_kernel(int k, int n, const MT
       X[i + static_cast<size_t>(col0 + c) * ldx] = sx[c * LX + i];
 }
 
+// Problem blockIdx.y: T and X advance by t_step and x_step.
+template <typename MT, typename V, bool LOWER, bool IDENTITY, int KM>
+__global__ __launch_bounds__(kTriThreads) void tri_kernel(int k, int n, const MT* T, int ldt,
+                                                          size_t t_step, V* X, int ldx,
+                                                          size_t x_step) {
+  __shared__ TriShared<V, KM> sh;
+  tri_block<MT, V, LOWER, IDENTITY, KM>(k, n, T + blockIdx.y * t_step, ldt,
+                                        X + blockIdx.y * x_step, ldx, blockIdx.x, sh);
+}
+
+// What follows a panel: block 0 composes its interchanges (pipid.hpp), the
+// others form the inverse of L11, 16 columns each.
+template <typename V, int KM>
+__global__ __launch_bounds__(kTriThreads) void panel_tail_kernel(
+    int jb, const int* ipiv, int base, int* permU, const V* L, int ldl, V* Linv, int ldi,
+    Stamps st) {
+  __shared__ union Shared {
+    __device__ Shared() {}
+    TriShared<V, KM> tri;
+    PipidShared      pipid;
+  } sh;
+  stamp_now(st);
+  if(blockIdx.x == 0)
+    pipid_block(jb, ipiv, base, permU, sh.pipid);
+  else
+    tri_block<V, V, true, true, KM>(jb, jb, L, ldl, Linv, ldi, blockIdx.x - 1, sh.tri);
+}
+
+template <typename V>
+hipError_t panel_tail(hipStream_t s, int jb, const int* ipiv, int base, int* permU,
+                      const V* L, int ldl, V* Linv, int ldi, Stamps st) {
+  if(jb <= 0) return hipSuccess;
+  if(jb > kMaxNB) return hipErrorInvalidValue;
+  const dim3 g(1 + (jb + 15) / 16), b(kTriThreads);
+  if(jb <= 128)
+    hipLaunchKernelGGL((panel_tail_kernel<V, 128>), g, b, 0, s, jb, ipiv, base, permU, L,
+                       ldl, Linv, ldi, st);
+  else if(jb <= 512)
+    hipLaunchKernelGGL((panel_tail_kernel<V, 512>), g, b, 0, s, jb, ipiv, base, permU, L,
+                       ldl, Linv, ldi, st);
+  else
+    hipLaunchKernelGGL((panel_tail_kernel<V, 1024>), g, b, 0, s, jb, ipiv, base, permU, L,
+                       ldl, Linv, ldi, st);
+  return hipGetLastError();
+}
+
 // The instance with the least LDS: more workgroups to a CU.
 template <bool LOWER, bool IDENTITY, typename MT, typename V>
 hipError_t tri_solve(hipStream_t s, int k, int n, int blocks, const MT* T, int ldt,
@@ -228,9 +279,16 @@ hipError_t launch_linv(hipStream_t s, int jb, const double* L, int ldl,
   return tri_solve<true, true>(s, jb, jb, 1, L, ldl, 0, Linv, ldi, 0);
 }
 
-hipError_t launch_linv(hipStream_t s, int jb, const float* L, int ldl,
-                       float* Linv, int ldi) {
-  return tri_solve<true, true>(s, jb, jb, 1, L, ldl, 0, Linv, ldi, 0);
+hipError_t launch_panel_tail(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
+                             int* permU, const double* L, int ldl, double* Linv,
+                             int ldi, Stamps st) {
+  return panel_tail(s, jb, ipiv, ipiv_base, permU, L, ldl, Linv, ldi, st);
+}
+
+hipError_t launch_panel_tail(hipStream_t s, int jb, const int* ipiv, int ipiv_base,
+                             int* permU, const float* L, int ldl, float* Linv,
+                             int ldi, Stamps st) {
+  return panel_tail(s, jb, ipiv, ipiv_base, permU, L, ldl, Linv, ldi, st);
 }
 
 // Block J starts at T[J kb, J kb], its inverse (leading dimension kb) at Inv +

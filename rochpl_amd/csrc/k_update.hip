@@ -41,6 +41,7 @@
 // all stage loads are drained before the epilogue.
 #include "claim.hpp"
 #include "hplx_internal.hpp"
+#include "stamp.hpp"
 #include "update_tile.hpp"
 
 namespace hplx {
@@ -56,7 +57,8 @@ template <bool kPanel>
 __global__ __launch_bounds__(512, 2) void update_kernel(
     int M, int N, int K, const double* __restrict__ A, int lda,
     const double* __restrict__ Bt, int ldb, double* __restrict__ C, int ldc,
-    int tiles_m, int tiles_n, int a_rows, int b_cols) {
+    int tiles_m, int tiles_n, int a_rows, int b_cols, Stamps st) {
+  stamp_now(st);
   HPLX_USLOT(0) HPLX_USLOT(1) HPLX_USLOT(2) HPLX_USLOT(3)
   const int T = tiles_m * tiles_n, per = gridDim.x / kUXcds, bid = blockIdx.x;
   const int tile = (bid % kUXcds) * per + bid / kUXcds;
@@ -213,10 +215,14 @@ __global__ void set_flag_kernel(int* p) {
   __hip_atomic_store(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ void zero_ints_kernel(int* p, int n) {
+// p[0:n] = 0, and q[0] if q is not null.
+__global__ void zero_ints_kernel(int* p, int n, int* q) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i < n) p[i] = 0;
+  if(i == 0 && q) *q = 0;
 }
+
+__global__ void stamp_kernel(Stamps st) { stamp_now(st); }
 
 // Each workgroup records the __smid() of the CU it ran on, then waits about
 // `spin` clock ticks so that the grid spreads over every CU.
@@ -231,7 +237,7 @@ __global__ void cu_census_kernel(int* out, long long spin) {
 
 hipError_t launch_update(hipStream_t s, int m, int n, int k, const double* A,
                          int lda, const double* Bt, int ldb, double* C, int ldc,
-                         int a_rows, int b_cols, bool panel) {
+                         int a_rows, int b_cols, bool panel, Stamps st) {
   UpdGrid    g;
   hipError_t e = update_grid(m, n, k, A, lda, Bt, ldb, a_rows, b_cols, &g);
   if(e != hipSuccess) return e;
@@ -239,11 +245,11 @@ hipError_t launch_update(hipStream_t s, int m, int n, int k, const double* A,
   if(panel)
     hipLaunchKernelGGL(update_kernel<true>, dim3(static_cast<unsigned>(grid)),
                        dim3(512), 0, s, m, n, k, A, lda, Bt, ldb, C, ldc,
-                       g.tiles_m, g.tiles_n, a_rows, b_cols);
+                       g.tiles_m, g.tiles_n, a_rows, b_cols, st);
   else
     hipLaunchKernelGGL(update_kernel<false>, dim3(static_cast<unsigned>(grid)),
                        dim3(512), 0, s, m, n, k, A, lda, Bt, ldb, C, ldc,
-                       g.tiles_m, g.tiles_n, a_rows, b_cols);
+                       g.tiles_m, g.tiles_n, a_rows, b_cols, st);
   return hipGetLastError();
 }
 
@@ -338,10 +344,15 @@ hipError_t launch_set_flag(hipStream_t s, int* p) {
   return hipGetLastError();
 }
 
-hipError_t launch_zero_ints(hipStream_t s, int* p, int n) {
+hipError_t launch_stamp(hipStream_t s, Stamps st) {
+  hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(1), 0, s, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_zero_ints(hipStream_t s, int* p, int n, int* q) {
   if(n <= 0) return hipSuccess;
   hipLaunchKernelGGL(zero_ints_kernel, dim3((n + 255) / 256), dim3(256), 0, s,
-                     p, n);
+                     p, n, q);
   return hipGetLastError();
 }
 

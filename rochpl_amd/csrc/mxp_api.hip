@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <numeric>
 #include <vector>
 
 #include "api_common.hpp"
@@ -173,8 +174,8 @@ struct MxpLoop {
     S*        A12 = A + j + static_cast<size_t>(j + jb) * lda;
     float*    P = panel_ptr(k);
     const int ldP = panel_ld();
-    HIPCHK(c, hplx::launch_pipid(s, jb, mat->ipiv + j, j, c.permU));
-    HIPCHK(c, hplx::launch_linv(s, jb, P, ldP, ws->linv, nb));
+    HIPCHK(c, hplx::launch_panel_tail(s, jb, mat->ipiv + j, j, c.permU, P, ldP,
+                                      ws->linv, nb));
     HIPCHK(c, hplx::launch_swap_gather(s, jb, nt, A12, lda, c.permU, ws->W, nb));
     if constexpr(kF16) {
       HIPCHK(c, hplx::launch_sgemm(s, jb, nt, jb, 1.0, ws->linv, nb, ws->W, nb,
@@ -199,7 +200,7 @@ struct MxpLoop {
   }
 
   // C22 columns [c0, c0 + n) of step k -= L21 U12, on stream s, timed by an
-  // event pair of the given kind (1 whole launch, 2 claimed, 3 resume)
+  // pair of the given kind (1 whole launch, 2 claimed, 3 resume)
   // carrying `flops`.
   int gemm(int k, int c0, int n, hipStream_t s, const hplx::MxpPacked& pk,
            const float* U, int ldu, const hplx::MxpLaunch& L, int kind,
@@ -210,7 +211,7 @@ struct MxpLoop {
     const int pi = c.ev_pairs++;
     c.ev_kind[pi]  = kind;
     c.ev_flops[pi] = flops;
-    HIPCHK(c, hipEventRecord(c.ev[2 * pi], s));
+    HIPCHK(c, hplx::launch_stamp(s, {hplx::stamp_at(c, 0, pi), nullptr}));
     if(o->update == HPLX_UPDATE_FP32) {
       if constexpr(!kF16)
         HIPCHK(c, hplx::launch_sgemm(s, m - jb, n, jb, -1.0, panel_ptr(k) + jb,
@@ -221,7 +222,7 @@ struct MxpLoop {
       HIPCHK(c, hplx::launch_mxp_gemm(s, o->update, o->terms, m - jb, n, jb, q,
                                       C, lda, L));
     }
-    HIPCHK(c, hipEventRecord(c.ev[2 * pi + 1], s));
+    HIPCHK(c, hplx::launch_stamp(s, {hplx::stamp_at(c, 0, pi) + 1, nullptr}));
     return HPLX_SUCCESS;
   }
 };
@@ -244,11 +245,7 @@ int factor_loop(Ctx& c, const hplx_palg* palg, const hplx_mxp_opts* o,
   MxpLoop<S> L{c, palg, o, mat, ws, static_cast<S*>(mat->A), N, nb, lda};
 
   const int npanels = (N + nb - 1) / nb;
-  while(static_cast<int>(c.ev.size()) < 6 * npanels) {
-    hipEvent_t e;
-    HIPCHK(c, hipEventCreate(&e));
-    c.ev.push_back(e);
-  }
+  if(const int e = hplx::reserve_stamps(c, npanels)) return e;
   c.ev_pairs   = 0;
   c.gemm_flops = 0.0;
   c.ev_kind.assign(3 * npanels, 1);
@@ -300,8 +297,7 @@ int factor_loop(Ctx& c, const hplx_palg* palg, const hplx_mxp_opts* o,
           return r;
         int* claim = c.claim + (k & 1) * hplx::kClaimInts;
         int* stop  = c.stop + (k & 1) * 32;
-        HIPCHK(c, hplx::launch_zero_ints(U, claim, hplx::kClaimInts));
-        HIPCHK(c, hplx::launch_zero_ints(U, stop, 1));
+        HIPCHK(c, hplx::launch_zero_ints(U, claim, hplx::kClaimInts, stop));
         hipEvent_t ev_prep, ev_pan;
         if((r = hplx::sync_event(c, nev++, &ev_prep)) ||
            (r = hplx::sync_event(c, nev++, &ev_pan)))
@@ -489,13 +485,11 @@ int factor_any(Ctx& c, const hplx_palg* palg, const hplx_mxp_opts* o,
                                          : factor_loop<float>(c, palg, o, mat);
 }
 
-double gemm_ms(Ctx& c) {
-  double t = 0.0;
-  for(int i = 0; i < c.ev_pairs; ++i) {
-    float ms = 0.f;
-    if(hipEventElapsedTime(&ms, c.ev[2 * i], c.ev[2 * i + 1]) == hipSuccess) t += ms;
-  }
-  return t;
+int gemm_ms(Ctx& c, double* ms) {
+  std::vector<double> t;
+  if(const int r = hplx::stamp_times(c, 0, c.ev_pairs, &t)) return r;
+  *ms = std::accumulate(t.begin(), t.end(), 0.0);
+  return HPLX_SUCCESS;
 }
 
 }  // namespace
@@ -654,7 +648,7 @@ int hplx_mxp_pdgesv(hplx_ctx* ctx, const hplx_palg* palg,
   if(r) return r;
   const auto t1 = std::chrono::steady_clock::now();
   R.factor_ms       = std::chrono::duration<double, std::milli>(t1 - t0).count();
-  R.update_ms       = gemm_ms(c);
+  if((r = gemm_ms(c, &R.update_ms))) return r;
   R.update_flops    = c.gemm_flops;
   R.update_launches = c.ev_pairs;
 

@@ -1,0 +1,21 @@
+// Times written by the kernels themselves: block 0 of a kernel notes when it
+// starts, which in stream order is also when what came before it has ended.
+// Two records of an event cost the stream 9 us between two kernels, an event
+// carried by a kernel's own dispatch 7, this nothing.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "hplx_internal.hpp"
+
+namespace hplx {
+
+__device__ inline void stamp_now(const Stamps& s) {
+  if((s.a || s.b) && blockIdx.x == 0 && threadIdx.x == 0) {
+    const long long now = wall_clock64();
+    if(s.a) *s.a = now;
+    if(s.b) *s.b = now;
+  }
+}
+
+}  // namespace hplx

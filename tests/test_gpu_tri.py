@@ -89,3 +89,20 @@ def test_a_column_that_overflows(ctx):
     assert np.array_equal(got[~np.isfinite(U)], U[~np.isfinite(U)], equal_nan=True)
     fin = np.isfinite(U)
     assert np.allclose(got[fin], U[fin], rtol=1e-13, atol=1e-13)
+
+
+@pytest.mark.parametrize("jb", [1, 2, 64, 65, 1000, 1024])
+@pytest.mark.parametrize("kind", ["none", "last", "one below", "few", "far"])
+def test_interchanges_that_share_targets(ctx, jb, kind):
+    """Composed interchanges where many steps have the same target."""
+    from oracle import oracle as o
+    print("[gpu-case] pipid jb=%d %s" % (jb, kind), flush=True)
+    i = np.arange(jb)
+    rng = np.random.default_rng(jb)
+    ipiv = {"none": i, "last": np.full(jb, jb - 1), "one below": np.full(jb, jb),
+            "few": np.maximum(i, rng.choice([jb // 2, jb - 1, jb + 3, 2 * jb], jb)),
+            "far": jb + 2048 * rng.integers(1, 5, jb)}[kind].astype(np.int32)
+    dp, dq = ctx.alloc(4 * jb), ctx.alloc(8 * jb)
+    dp.upload(ipiv)
+    ctx.pipid(jb, dp.ptr, dq.ptr)
+    assert np.array_equal(dq.download(2 * jb, np.int32), o.pipid(ipiv))
