@@ -197,14 +197,16 @@ hipError_t launch_leaf(Ctx& c, V* P, int lda, int m, int JB, int c0, int w,
   // API adds nothing here and refuses to launch while another process holds
   // the device.)
   void* args[] = {&la};
-  return hipLaunchKernel(leaf_kernel_ptr<V>(rpt), dim3(G), dim3(kLeafThreads), args,
+  return hipLaunchKernel(leaf_kernel_ptr<V>(rpt, G == 1), dim3(G), dim3(kLeafThreads), args,
                          0, panel_stream(c));
 }
 
 // C (m x n) -= A (m x k) B (k x n) inside the panel recursion
 // (rocblas_dgemm at src/pfact/HPL_pdrpanrlT.cpp:142-154).  Large FP64
-// products go through the streamed trailing-update kernel with B transposed into the context's L11^{-1} buffer, which is idle
-// while a panel is factored; the others, and FP32, through the generic GEMM.
+// products at least one 128-column tile wide go through the streamed
+// trailing-update kernel with B transposed into the context's L11^{-1} buffer,
+// which is idle while a panel is factored; the others, and FP32, through the
+// generic GEMM.
 inline hipError_t panel_gemm(Ctx& c, int m, int n, int k, const double* A,
                              int lda, const double* B, int ldb, double* C,
                              int ldc) {
@@ -216,7 +218,7 @@ inline hipError_t panel_gemm(Ctx& c, int m, int n, int k, const double* A,
   // of them is followed by a further column of the panel (B's first
   // column), so the extra element lies inside the panel's storage.
   const int a_rows = (m + 1) & ~1;
-  if(update_pays(m, n) && static_cast<size_t>(k) * ldt <= static_cast<size_t>(kMaxNB) * kMaxNB &&
+  if(n >= 128 && update_pays(m, n) && static_cast<size_t>(k) * ldt <= static_cast<size_t>(kMaxNB) * kMaxNB &&
      update_fast_ok(m, n, k, A, lda, Bt, ldt, a_rows, ldt)) {
     hipError_t e = launch_transpose(s, k, n, B, ldb, Bt, ldt);
     if(e != hipSuccess) return e;
@@ -460,8 +462,8 @@ int panel_steps(const PanelAlgo& a0, int jb, int* out, int max_steps) {
 hipError_t leaf_occupancy(int* blocks_per_cu) {
   // the smallest of the leaves' occupancies
   *blocks_per_cu = INT_MAX;
-  for(const void* f : {leaf_kernel_ptr<double>(1), leaf_kernel_ptr<double>(kLeafRPT),
-                       leaf_kernel_ptr<float>(1), leaf_kernel_ptr<float>(kLeafRPT)}) {
+  for(const void* f : {leaf_kernel_ptr<double>(1, false), leaf_kernel_ptr<double>(kLeafRPT, false),
+                       leaf_kernel_ptr<float>(1, false), leaf_kernel_ptr<float>(kLeafRPT, false)}) {
     int        n = 0;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, kLeafThreads, 0);
     if(e != hipSuccess) return e;

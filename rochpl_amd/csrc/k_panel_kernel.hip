@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
       la.seq_base    = (a.leaf_base + leaf_i++) << 6;
       la.err         = a.err;
           la.grid        = gl;
-      if(b < gl) leaf::leaf_run<double, double, kLeafThreads, kLeafRPT>(la, sh);
+      if(b < gl) leaf::leaf_run<double, double, kLeafThreads, kLeafRPT, false>(la, sh);
     } else if(o.kind == kPanelTrsm) {
       const double* T = a.P + o.ar + static_cast<size_t>(o.ac) * a.lda;
       for(int col = b; col < o.n; col += G)

@@ -16,9 +16,12 @@
 //      as its number is seen: no release, no acquire, no separate flag;
 //   3. the waves read all slots, polling the words themselves, into LDS;
 //      after one workgroup barrier every wave picks the pivot row;
-//   4. labels are swapped, the rows left are divided by the pivot and
-//      updated, the pivot row's values broadcast within the FMA (DPP).  The
-//      pivot row is finished: workgroup 0 keeps it in LDS for the end.
+//   4. labels are swapped, the rows left are divided by the pivot, and the
+//      next column is updated;
+//   5. the other columns are updated, the pivot row's values broadcast within
+//      the FMA (DPP), while the next column's candidates are under way (see
+//      leaf_publish).  The pivot row is finished: workgroup 0 keeps it in LDS
+//      for the end.
 // Slots are double-buffered by column parity, so a workgroup that runs ahead
 // never overwrites a slot another workgroup still reads.  A grid of one
 // workgroup passes the row through LDS only.  The reference instead parks
@@ -48,13 +51,19 @@ constexpr uint32_t kSpinLimit = 1u << 22;
 constexpr int      kTurn      = 8;  // columns per turn of the column loop
 // slot layout (8-byte words, sequence number in the upper half): [0..63] the
 // candidate row's 32-bit halves (FP32: [0..31] its values), [64..67] its
-// header: key (upper, lower half), label, the row it was loaded from
-constexpr int kSlotHead = 64;
-static_assert(kSlotHead + 4 <= kSlotStride, "slot too small");
+// header: key (upper, lower half), label, the row it was loaded from, the
+// row's factor in the update it still lacks (lower, upper half)
+constexpr int kSlotHead = 64, kHeadWords = 6;
+static_assert(kSlotHead + kHeadWords <= kSlotStride, "slot too small");
 // Up to kNear workgroups every candidate row is read along with its header
 // (one memory round trip); with more the headers come first and then only
 // the pivot row.
 constexpr int kNear = 32;
+// Time until the first poll of the slots (x 64 cycles): what the candidates
+// take to be seen.  A poll that comes too early costs a whole round trip: 4096
+// / 9001 / 32000 rows, us with 0, 3, 6, 9, 12: 95.7 / 99.7 / 115.5, 89.4 / 95.1
+// / 112.8, 89.3 / 91.8 / 110.9, 91.9 / 92.0 / 110.8, 94.2 / 95.9 / 111.3.
+constexpr int kFirstPoll = 7;
 
 struct LeafArgs {
   void*    P;          // panel top-left (panel row 0), storage type S
@@ -79,9 +88,14 @@ struct LeafShared {
   alignas(16) T cand[kNear][kLeafMax];    // the workgroups' candidate rows
   alignas(16) T row[2][kLeafMax];         // this workgroup's, by column parity
   alignas(16) T fin[kLeafMax][kLeafMax];  // workgroup 0: the finished top rows
-  alignas(16) uint32_t head[kNear][4];    // the candidates' headers
+  // the pivot row, by column parity, as the tile is arranged for its column and
+  // for the next
+  alignas(16) T ucur[2][2][kLeafMax];
+  alignas(16) T nl[2];                    // this workgroup's candidate's factor
+  alignas(16) uint32_t head[kNear][8];    // the candidates' headers
   alignas(16) uint32_t wave[2][16][4];    // the waves' candidates, as headers
-  int sel[2];  // the pivot's label and the row it was loaded from
+  int      sel[2];  // the pivot's label and the row it was loaded from
+  uint32_t sel_nl[2];  // and its factor's halves
   int ok;
 };
 
@@ -163,6 +177,12 @@ __device__ inline uint32_t lo_bits(double x) {
 }
 __device__ inline uint32_t hi_bits(float x) { return __float_as_uint(x); }
 __device__ inline uint32_t lo_bits(float) { return 0; }
+__device__ inline double from_halves(uint32_t lo, uint32_t hi, double) {
+  return __hiloint2double(static_cast<int>(hi), static_cast<int>(lo));
+}
+__device__ inline float from_halves(uint32_t lo, uint32_t, float) {
+  return __uint_as_float(lo);
+}
 template <typename T>
 constexpr uint32_t kInfBits = sizeof(T) == 8 ? 0x7ff00000u : 0x7f800000u;
 
@@ -229,6 +249,11 @@ __device__ inline int word_of(int lane) {
   return sizeof(T) == 8 ? lane : lane & (kLeafMax - 1);
 }
 
+// Word of a header that a lane carries.
+__device__ inline int head_word(int lane) {
+  return (lane & 7) < kHeadWords ? lane & 7 : 0;
+}
+
 // A wait's poll failed: true when the grid has to stop.
 __device__ inline bool give_up(uint32_t& spins, int* err) {
   ++spins;
@@ -244,48 +269,59 @@ __device__ inline bool give_up(uint32_t& spins, int* err) {
 }
 
 // Every workgroup's candidate of sequence `seq` into sh.cand / sh.head: wave
-// w of NW takes slots w, w + NW, ..., up to four at a time in flight.  False
-// on timeout or error.
+// w of NW takes slots w, w + NW, ..., up to four.  (Two polls under way at a
+// time are no faster: the barrier that follows waits for both.)  False on
+// timeout or error.
 template <typename T, int NW>
 __device__ __forceinline__ bool gather_all(const LeafArgs& a,
                                            const unsigned long long* slots,
                                            uint32_t seq, LeafShared<T>& sh) {
-  constexpr int kBatch = 4;
+  constexpr int kBatch = kNear / NW;
   constexpr int kRowWords = kLeafMax * sizeof(T) / 4;
   const int     lane = threadIdx.x & 63;
   const int     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t*     cand = reinterpret_cast<uint32_t*>(&sh.cand[0][0]);
   uint32_t      spins = 0;
-  for(int g0 = wave; g0 < a.grid; g0 += NW * kBatch) {
-    unsigned pending = 0;
+  unsigned      pending = 0;
+#pragma unroll
+  for(int k = 0; k < kBatch; ++k)
+    if(wave + k * NW < a.grid) pending |= 1u << k;
+  if(!pending) return true;
+  struct Poll {
+    unsigned long long rw[kBatch], hw[kBatch];
+  };
+  const unsigned long long* row = slots + wave * kSlotStride + word_of<T>(lane);
+  const unsigned long long* head = slots + wave * kSlotStride + kSlotHead + head_word(lane);
+  auto issue = [&](Poll& p) {
 #pragma unroll
     for(int k = 0; k < kBatch; ++k)
-      if(g0 + k * NW < a.grid) pending |= 1u << k;
-    while(pending) {
-      unsigned long long rw[kBatch], hw[kBatch];
+      if(pending & (1u << k)) {
+        p.rw[k] = ld_word(row + k * NW * kSlotStride);
+        p.hw[k] = ld_word(head + k * NW * kSlotStride);
+      }
+  };
+  auto check = [&](const Poll& p) {
 #pragma unroll
-      for(int k = 0; k < kBatch; ++k)
-        if(pending & (1u << k)) {
-          const unsigned long long* s = slots + (g0 + k * NW) * kSlotStride;
-          rw[k] = ld_word(s + word_of<T>(lane));
-          hw[k] = ld_word(s + kSlotHead + (lane & 3));
+    for(int k = 0; k < kBatch; ++k)
+      if(pending & (1u << k)) {
+        const bool in = static_cast<uint32_t>(p.rw[k] >> 32) == seq &&
+                        static_cast<uint32_t>(p.hw[k] >> 32) == seq;
+        if(__all(in)) {
+          const int g = wave + k * NW;
+          cand[g * kRowWords + word_of<T>(lane)] = static_cast<uint32_t>(p.rw[k]);
+          if(lane < kHeadWords) sh.head[g][lane] = static_cast<uint32_t>(p.hw[k]);
+          pending &= ~(1u << k);
         }
-#pragma unroll
-      for(int k = 0; k < kBatch; ++k)
-        if(pending & (1u << k)) {
-          const bool in = static_cast<uint32_t>(rw[k] >> 32) == seq &&
-                          static_cast<uint32_t>(hw[k] >> 32) == seq;
-          if(__all(in)) {
-            const int g = g0 + k * NW;
-            cand[g * kRowWords + word_of<T>(lane)] = static_cast<uint32_t>(rw[k]);
-            if(lane < 4) sh.head[g][lane] = static_cast<uint32_t>(hw[k]);
-            pending &= ~(1u << k);
-          }
-        }
-      if(pending && give_up(spins, a.err)) return false;
-    }
+      }
+  };
+  __builtin_amdgcn_s_sleep(kFirstPoll);
+  for(;;) {
+    Poll p;
+    issue(p);
+    check(p);
+    if(!pending) return true;
+    if(give_up(spins, a.err)) return false;
   }
-  return true;
 }
 
 // The same for many workgroups, on one wave: lane l waits for the headers of
@@ -347,9 +383,11 @@ __device__ __forceinline__ bool gather_pivot(const LeafArgs& a,
   const unsigned long long* s = slots + g * kSlotStride;
   for(;;) {
     const unsigned long long x = ld_word(s + word_of<T>(lane));
-    if(__all(static_cast<uint32_t>(x >> 32) == seq)) {
+    const unsigned long long y = ld_word(s + kSlotHead + 4 + (lane & 1));
+    if(__all(static_cast<uint32_t>(x >> 32) == seq && static_cast<uint32_t>(y >> 32) == seq)) {
       reinterpret_cast<uint32_t*>(&sh.cand[0][0])[word_of<T>(lane)] =
           static_cast<uint32_t>(x);
+      if(lane < 2) sh.sel_nl[lane] = static_cast<uint32_t>(y);
       return true;
     }
     if(give_up(spins, a.err)) return false;
@@ -576,38 +614,50 @@ __device__ __forceinline__ void fma_turn3(float (&v)[kLeafMax][3], float u,
       : "scc");
 }
 
-// Column jb0 + j of the leaf, held in tile position 0 (every register of the
-// tile is addressed statically).  Positions [0, 8 - j) hold the columns from
-// there on and [8 - j, 8) the j columns finished in this turn; [8, act) hold
-// the unfinished columns of the next turns.  lab: the labels of the thread's
-// rows, -1 for a row that is finished or outside the panel, whose registers
-// may then hold anything; msk: 0x7fffffff, 0 for those rows.  dst: lane
-// i >= 32 the label of the row loaded from row c0 + i - 32 (-1 once it is a
-// pivot row); src: lane i < 32 the row that the pivot row of column i was
-// loaded from; piv: lane i < 32 its label then.  False if the grid has to
-// stop.
 struct LeafMoves {
   int piv, dst, src;
 };
 
-template <typename T, int NT, int RPT>
-__device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RPT],
-                                          int (&lab)[RPT], uint32_t (&msk)[RPT],
-                                          LeafShared<T>& sh, LeafMoves& mv,
-                                          int& zero, int jb0, int j, int act) {
+// A column is two halves.  leaf_publish finds the pivot candidate of column jj
+// (its values x, the column already updated) and sends it; leaf_receive waits
+// for the pivot row, scales the column, and forms the next column's values.
+// Between the two, while the exchange is under way, the rank-1 update of the
+// column before is applied to the tile (leaf_update) -- so a candidate's row is
+// sent without that update and with the row's factor in it, and whoever
+// receives it applies it, with the same FMA.  A workgroup by itself (SINGLE)
+// has nothing to wait for and updates its tile first.
+//
+// Tile positions (every register of the tile is addressed statically): column
+// jb0 + j, jb0 a multiple of 8, is in position 0; positions [0, 8 - j) hold the
+// columns from there on and [8 - j, 8) the j columns finished in this turn;
+// [8, act) hold the unfinished columns of the next turns.  leaf_update leaves
+// the tile arranged for the next column.
+//
+// lab: the labels of the thread's rows, -1 for a row that is finished or
+// outside the panel, whose registers may then hold anything.  nl: minus the rows'
+// factors in the last update.  dst: lane i >= 32 the label of the row loaded
+// from row c0 + i - 32 (-1 once it is a pivot row); src: lane i < 32 the row
+// that the pivot row of column i was loaded from; piv: lane i < 32 its label
+// then.
+template <typename T, int NT, int RPT, bool SINGLE>
+__device__ __forceinline__ void leaf_publish(const LeafArgs& a,
+                                             const T (&v)[kLeafMax][RPT],
+                                             const T (&x)[RPT], const T (&nl)[RPT],
+                                             const int (&lab)[RPT],
+                                             LeafShared<T>& sh, int jj) {
   constexpr int NW   = NT / 64;
   const int     t    = threadIdx.x;
   const int     lane = t & 63;
   const int     wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int     b    = blockIdx.x;
-  const int     jj   = jb0 + j, par = j & 1;
+  const int     par  = jj & 1;
   const int     gc   = a.c0 + jj;  // current top row == current column
   // ---- step 1: candidate max |a(r, gc)| over the labels left, first by the
   // upper halves alone
   uint32_t k[RPT], top = 0;
 #pragma unroll
   for(int q = 0; q < RPT; ++q) {
-    k[q] = hi_bits(v[0][q]) & msk[q];
+    k[q] = lab[q] >= 0 ? hi_bits(x[q]) & 0x7fffffffu : 0u;
     top  = k[q] > top ? k[q] : top;
   }
   top = wave_max(top);
@@ -620,7 +670,7 @@ __device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RP
     const unsigned long long w  = __ballot(is);
     hits += __builtin_popcountll(w);
     at |= w;
-    kl = is ? lo_bits(v[0][q]) : kl;
+    kl = is ? lo_bits(x[q]) : kl;
     kb = is ? lab[q] : kb;
     kq = is ? q : kq;
   }
@@ -636,9 +686,9 @@ __device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RP
     kq          = 0;
 #pragma unroll
     for(int q = 0; q < RPT; ++q) {
-      const T    x   = v[0][q];
-      const bool nan = !(x == x);
-      uint32_t   h   = (hi_bits(x) & 0x7fffffffu) + kKeyBase, l = lo_bits(x);
+      const T    y   = x[q];
+      const bool nan = !(y == y);
+      uint32_t   h   = (hi_bits(y) & 0x7fffffffu) + kKeyBase, l = lo_bits(y);
       if(nan) {
         h = lab[q] == gc ? kKeyTopNan : 0;
         l = 0;
@@ -675,46 +725,80 @@ __device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RP
   int       org = a.c0 + b * CH + kq * NT + wave * 64 + owner;
   // ---- the candidate row, by its wave
   if(wave == ww && lb != INT_MAX && lane == owner) {
+    // as the tile will be arranged for this column
+    const bool turn  = (jj & (kTurn - 1)) == 0;
+    T* const   first = sh.row[par] + (turn ? kLeafMax - kTurn : 0);
+    T* const   rest  = sh.row[par] - (turn ? kTurn : 0);
 #pragma unroll
     for(int q = 0; q < RPT; ++q)
       if(kq == q) {
+        if constexpr(SINGLE) {
 #pragma unroll
-        for(int c = 0; c < kLeafMax; ++c) sh.row[par][c] = v[c][q];
+          for(int c = 0; c < kLeafMax; ++c) sh.row[par][c] = v[c][q];
+        } else {
+#pragma unroll
+          for(int c = 0; c < kTurn; ++c) first[(c - 1) & (kTurn - 1)] = v[c][q];
+#pragma unroll
+          for(int c = kTurn; c < kLeafMax; ++c) rest[c] = v[c][q];
+          sh.nl[par] = nl[q];
+        }
         // keeps the cases apart: merged, they would index the tile by kq
         asm volatile("; row %0" : : "n"(q));
       }
-    if(a.grid == 1) {
+    if constexpr(SINGLE) {
       sh.sel[0] = lb;
       sh.sel[1] = org;
     }
   }
-  int      p, po;  // the pivot's label, the row it was loaded from
-  const T* urow;
-  if(a.grid == 1) {
+  if constexpr(SINGLE) return;
+  // A workgroup without rows left publishes an empty candidate (key 0, label
+  // INT_MAX).
+  if(wave == ww) {
+    const uint32_t      seq  = a.seq_base + jj + 1;
+    unsigned long long* mine = reinterpret_cast<unsigned long long*>(a.slots) +
+                               (static_cast<size_t>(par) * (kMaxGrid + 1) + b) * kSlotStride;
+    // the wave's lanes see its own LDS stores in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t* half = reinterpret_cast<const uint32_t*>(sh.row[par]);
+    const uint32_t* fact = reinterpret_cast<const uint32_t*>(&sh.nl[par]);
+    st_word(mine + word_of<T>(lane), seq, half[word_of<T>(lane)]);
+    if(lane < kHeadWords)
+      st_word(mine + kSlotHead + lane, seq,
+              lane == 0   ? top
+              : lane == 1 ? wlo
+              : lane == 2 ? static_cast<uint32_t>(lb)
+              : lane == 3 ? static_cast<uint32_t>(org)
+                          : fact[sizeof(T) == 8 ? lane - 4 : 0]);
+  }
+}
+
+// False if the grid has to stop.
+template <typename T, int NT, int RPT, bool SINGLE>
+__device__ __forceinline__ bool leaf_receive(const LeafArgs& a, T (&v)[kLeafMax][RPT],
+                                             T (&x)[RPT], T (&nl)[RPT], int (&lab)[RPT],
+                                             LeafShared<T>& sh, LeafMoves& mv, int& zero,
+                                             int jj) {
+  constexpr int NW   = NT / 64;
+  const int     t    = threadIdx.x;
+  const int     lane = t & 63;
+  const int     wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int     b    = blockIdx.x;
+  const int     jb0 = jj & ~(kTurn - 1), j = jj & (kTurn - 1), par = j & 1;
+  const int     gc = a.c0 + jj;
+  int       p, po;  // the pivot's label, the row it was loaded from
+  uint32_t  nlo = 0, nhi = 0;
+  const T*  urow;
+  if constexpr(SINGLE) {
     __syncthreads();
     p    = sh.sel[0];
     po   = sh.sel[1];
     urow = sh.row[par];
   } else {
-    // ---- steps 2-3.  A workgroup without rows left publishes an empty
-    // candidate (key 0, label INT_MAX).
-    const uint32_t      seq  = a.seq_base + jj + 1;
-    unsigned long long* slots =
-        reinterpret_cast<unsigned long long*>(a.slots) +
+    const uint32_t            seq = a.seq_base + jj + 1;
+    const unsigned long long* slots =
+        reinterpret_cast<const unsigned long long*>(a.slots) +
         static_cast<size_t>(par) * (kMaxGrid + 1) * kSlotStride;
-    unsigned long long* mine = slots + b * kSlotStride;
-    if(wave == ww) {
-      // the wave's lanes see its own LDS stores in order
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const uint32_t* half = reinterpret_cast<const uint32_t*>(sh.row[par]);
-      st_word(mine + word_of<T>(lane), seq, half[word_of<T>(lane)]);
-      if(lane < 4)
-        st_word(mine + kSlotHead + lane, seq,
-                lane == 0   ? top
-                : lane == 1 ? wlo
-                            : static_cast<uint32_t>(lane == 2 ? lb : org));
-    }
     const bool near = a.grid <= kNear;
     if(near ? !gather_all<T, NW>(a, slots, seq, sh)
             : wave == 0 && !gather_pivot<T>(a, slots, seq, sh))
@@ -729,49 +813,72 @@ __device__ __forceinline__ bool leaf_step(const LeafArgs& a, T (&v)[kLeafMax][RP
         go = sh.head[lane][1];
         gl = static_cast<int>(sh.head[lane][2]);
       }
-      top         = wave_max(gh);
+      const uint32_t top = wave_max(gh);
       const int g = first_of(__ballot(gh == top) & ((1ull << a.grid) - 1), top, go, gl);
       p           = readlane(gl, g);
       po          = static_cast<int>(sh.head[g][3]);
+      nlo         = sh.head[g][4];
+      nhi         = sh.head[g][5];
       urow        = sh.cand[g];
     } else {
       p    = sh.sel[0];
       po   = sh.sel[1];
+      nlo  = sh.sel_nl[0];
+      nhi  = sh.sel_nl[1];
       urow = sh.cand[0];
     }
   }
   p  = __builtin_amdgcn_readfirstlane(p);
   po = __builtin_amdgcn_readfirstlane(po);
-  // u0 / u1: the pivot row's positions 0..15 / 16..31, in every 16 lanes
-  const T u0 = urow[lane & 15], u1 = urow[16 + (lane & 15)];
+  // the pivot row's positions c and 16 + c
+  const int c  = lane & 15;
+  T         u0 = urow[c], u1 = urow[16 + c];
+  if constexpr(!SINGLE) {
+    // with the update it lacks: that of the column before, which is not
+    // finished in positions [0, 8 - j) of this turn and [8, act)
+    const int act = (a.w + kTurn - 1) / kTurn * kTurn - jb0;
+    const T   pnl = from_halves(nlo, nhi, T(0));
+    const T   c0 = sh.ucur[par ^ 1][1][c], c1 = sh.ucur[par ^ 1][1][16 + c];
+    if(jj > 0) {
+      u0 = c < kTurn - j || (c >= kTurn && c < act) ? fma(c0, pnl, u0) : u0;
+      u1 = 16 + c < act ? fma(c1, pnl, u1) : u1;
+    }
+    // for later, each copy by a wave of its own; read after the next column's
+    // barriers
+    if(lane < 16) {
+      if(wave == 2) {
+        sh.ucur[par][0][c]      = u0;
+        sh.ucur[par][0][16 + c] = u1;
+      }
+      if(wave == 3) {
+        const bool turn = j == kTurn - 1;
+        sh.ucur[par][1][c < kTurn ? ((c - 1) & (kTurn - 1)) + (turn ? kLeafMax - kTurn : 0)
+                                  : c - (turn ? kTurn : 0)] = u0;
+        sh.ucur[par][1][16 + c - (turn ? kTurn : 0)]        = u1;
+      }
+    }
+  }
+  if(b == 0 && wave == 1 && lane < 16) {
+    sh.fin[jj][c < kTurn ? jb0 + ((c + j) & (kTurn - 1)) : (c + jb0) & (kLeafMax - 1)] = u0;
+    sh.fin[jj][(c + 16 + jb0) & (kLeafMax - 1)] = u1;
+  }
   const T piv = readlane(u0, 0);
-  if(b == 0 && t < kLeafMax)
-    sh.fin[jj][t < kTurn ? jb0 + ((t + j) & (kTurn - 1))
-                         : (t + jb0) & (kLeafMax - 1)] = urow[t];
   if(piv == T(0) && zero < 0) zero = jj;
-  // ---- step 4: interchange rows gc and p (the pivot row is finished),
-  // scale, rank-1 update
+  // interchange rows gc and p (the pivot row is finished), scale
   mv.piv = lane == jj ? p : mv.piv;
   mv.src = lane == jj ? po : mv.src;
   mv.dst = mv.dst == p ? -1 : mv.dst == gc ? p : mv.dst;
-  T nl[RPT];
 #pragma unroll
   for(int q = 0; q < RPT; ++q) {
-    if(lab[q] == p) msk[q] = 0;
     lab[q] = lab[q] == p ? -1 : lab[q] == gc ? p : lab[q];
     if(piv != T(0)) v[0][q] = v[0][q] / piv;
     nl[q] = -v[0][q];
   }
-  if constexpr(RPT == 1) {
-    fma_turn1<0>(v, u0, nl, j);
-    if(act > 8) fma_group1<8, 0>(v, u0, nl);
-    if(act > 16) fma_group1<16, 0>(v, u1, nl);
-    if(act > 24) fma_group1<24, 0>(v, u1, nl);
-  } else {
-    fma_turn3<0>(v, u0, nl, j);
-    if(act > 8) fma_group3<8, 0>(v, u0, nl);
-    if(act > 16) fma_group3<16, 0>(v, u1, nl);
-    if(act > 24) fma_group3<24, 0>(v, u1, nl);
+  if constexpr(!SINGLE) {  // the next column, updated
+    const T un = readlane(u0, j < kTurn - 1 ? 1 : kTurn);
+#pragma unroll
+    for(int q = 0; q < RPT; ++q)
+      x[q] = fma(un, nl[q], j < kTurn - 1 ? v[1][q] : v[kTurn][q]);
   }
   // sh.cand / sh.row are rewritten only after later barriers, which every
   // wave reaches after its reads here
@@ -787,11 +894,49 @@ __device__ __forceinline__ void rotate_turn(T (&v)[kLeafMax][RPT]) {
             v[5][q], v[6][q], v[7][q]);
 }
 
+// The next turn's columns come to the front, the finished ones go to the end.
+template <typename T, int RPT>
+__device__ __forceinline__ void rotate_turns(T (&v)[kLeafMax][RPT]) {
+#pragma unroll
+  for(int i = 0; i < kTurn; ++i)
+#pragma unroll
+    for(int q = 0; q < RPT; ++q)
+      rotate4(v[i][q], v[i + 8][q], v[i + 16][q], v[i + 24][q]);
+}
+
+// The rank-1 update of column jj (none before column 0), and the arrangement
+// for the next column.
+template <typename T, int RPT, bool SINGLE>
+__device__ __forceinline__ void leaf_update(T (&v)[kLeafMax][RPT], const T (&nl)[RPT],
+                                            const LeafShared<T>& sh, int w, int jj) {
+  // the pivot row's positions 0..15 / 16..31, in every 16 lanes
+  const int lane = threadIdx.x & 15;
+  const T*  u    = SINGLE ? sh.row[jj & 1] : sh.ucur[jj & 1][0];
+  const T   u0 = u[lane], u1 = u[16 + lane];
+  const int j   = __builtin_amdgcn_readfirstlane(jj & (kTurn - 1));
+  const int act = (w + kTurn - 1) / kTurn * kTurn - (jj & ~(kTurn - 1));
+  if(jj >= 0) {
+    if constexpr(RPT == 1) {
+      fma_turn1<0>(v, u0, nl, j);
+      if(act > 8) fma_group1<8, 0>(v, u0, nl);
+      if(act > 16) fma_group1<16, 0>(v, u1, nl);
+      if(act > 24) fma_group1<24, 0>(v, u1, nl);
+    } else {
+      fma_turn3<0>(v, u0, nl, j);
+      if(act > 8) fma_group3<8, 0>(v, u0, nl);
+      if(act > 16) fma_group3<16, 0>(v, u1, nl);
+      if(act > 24) fma_group3<24, 0>(v, u1, nl);
+    }
+  }
+  rotate_turn(v);
+  if(j == kTurn - 1) rotate_turns(v);
+}
+
 // One leaf on workgroups 0 .. a.grid-1 of NT threads, RPT rows each: the
 // body of leaf_kernel, also run by the persistent panel kernel
 // (k_panel_kernel.hip) once per leaf.  Workgroups whose rows all lie at or
 // below a.m take part in every exchange with an empty candidate.
-template <typename T, typename S, int NT, int RPT>
+template <typename T, typename S, int NT, int RPT, bool SINGLE>
 __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared<T>& sh) {
   constexpr int NW   = NT / 64;
   constexpr int CH   = NT * RPT;  // rows per workgroup
@@ -803,20 +948,21 @@ __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared<T>& sh) {
   S*            P    = static_cast<S*>(a.P);
 
   int          lab[RPT];  // the row each slot stands for; -1: none
-  uint32_t     msk[RPT];
   T            v[kLeafMax][RPT];
 #pragma unroll
   for(int q = 0; q < RPT; ++q) {
     const int row = a.c0 + b * CH + q * NT + t;
     lab[q]        = row < a.m ? row : -1;
-    msk[q]        = row < a.m ? 0x7fffffffu : 0u;
   }
+  // arranged as if the column before the first had ended a turn
 #pragma unroll
   for(int c = 0; c < kLeafMax; ++c) {
-    const S* col = P + static_cast<size_t>(a.c0 + c) * a.lda;
+    const S*  col = P + static_cast<size_t>(a.c0 + c) * a.lda;
+    const int p   = (c + kTurn) & (kLeafMax - 1);
+    const int pos = p < kTurn ? (p + 1) & (kTurn - 1) : p;
 #pragma unroll
     for(int q = 0; q < RPT; ++q)
-      v[c][q] = (c < a.w && lab[q] >= 0)
+      v[pos][q] = (c < a.w && lab[q] >= 0)
                        ? load_s<T, S>(col + static_cast<unsigned>(lab[q]))
                        : T(0);
   }
@@ -830,24 +976,29 @@ __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared<T>& sh) {
   mv.src   = a.c0 + (lane & (kLeafMax - 1));
   mv.dst   = lane < kLeafMax ? -2 : mv.src;
   int zero = -1;  // the first column with a zero pivot
-  int jb0  = 0;
-#pragma unroll 1
-  for(; jb0 < a.w; jb0 += kTurn) {
-    const int act  = (a.w + kTurn - 1) / kTurn * kTurn - jb0;
-    const int turn = a.w - jb0 < kTurn ? a.w - jb0 : kTurn;
-#pragma unroll 1
-    for(int j = 0; j < kTurn; ++j) {
-      if(j < turn && !leaf_step<T, NT, RPT>(a, v, lab, msk, sh, mv, zero, jb0, j, act))
-        return;
-      rotate_turn(v);
-    }
-    // the next columns come to the front, the finished ones go to the end
+  T   x[RPT], nl[RPT];
 #pragma unroll
-    for(int i = 0; i < kTurn; ++i)
-#pragma unroll
-      for(int q = 0; q < RPT; ++q)
-        rotate4(v[i][q], v[i + 8][q], v[i + 16][q], v[i + 24][q]);
+  for(int q = 0; q < RPT; ++q) {
+    x[q]  = v[kTurn][q];  // column 0
+    nl[q] = T(0);
   }
+#pragma unroll 1
+  for(int jj = 0; jj < a.w; ++jj) {
+    if constexpr(SINGLE) {
+      leaf_update<T, RPT, true>(v, nl, sh, a.w, jj - 1);
+      leaf_publish<T, NT, RPT, true>(a, v, v[0], nl, lab, sh, jj);
+      leaf_receive<T, NT, RPT, true>(a, v, x, nl, lab, sh, mv, zero, jj);
+    } else {
+      leaf_publish<T, NT, RPT, false>(a, v, x, nl, lab, sh, jj);
+      leaf_update<T, RPT, false>(v, nl, sh, a.w, jj - 1);
+      if(!leaf_receive<T, NT, RPT, false>(a, v, x, nl, lab, sh, mv, zero, jj)) return;
+    }
+  }
+  // the last turn to its end
+#pragma unroll 1
+  for(int j = (a.w - 1) & (kTurn - 1); j < kTurn; ++j) rotate_turn(v);
+  rotate_turns(v);
+  const int jb0 = (a.w + kTurn - 1) & ~(kTurn - 1);
 
   // ---- write the leaf back: the rows below where their labels say, the
   // finished top rows by workgroup 0
@@ -902,25 +1053,28 @@ __device__ __forceinline__ void leaf_run(const LeafArgs& a, LeafShared<T>& sh) {
 }
 
 // Bound by latency: per column one workgroup-wide and one grid-wide exchange
-// and the issue of about 150 (one row per thread) or 290 instructions; HBM
-// traffic is one read and one write of the leaf.  Time of a 32-column leaf of
-// m rows, FP64 (FP32), before this form and now:
-//   m = 500 131 (128) -> 47 (42) us, 1500 160 (158) -> 70 (62),
-//   4000 222 (216) -> 102 (88), 16000 246 (239) -> 114 (105),
-//   65000 276 (270) -> 134 (127), 131072 318 (320) -> 155 (150).
-template <typename T, typename S, int NT, int RPT>
+// and the issue of about 150 (one row per thread) or 290 instructions, of which
+// the update's and the arrangement's run beside the exchange; HBM traffic is
+// one read and one write of the leaf.  Time of a 32-column leaf of m rows, us,
+// FP64 (FP32): with the leaf unrolled / with the update before the exchange /
+// now:
+//   m = 500 131 (128) / 45 (39) / 43 (41), 1500 160 (158) / 68 (60) / 65 (56),
+//   4000 222 (216) / 99 (87) / 90 (84), 16000 246 (239) / 112 (102) / 100 (91),
+//   65000 276 (270) / 135 (126) / 134 (115),
+//   131072 318 (320) / 154 (148) / 151 (127).
+template <typename T, typename S, int NT, int RPT, bool SINGLE>
 __global__ __launch_bounds__(NT) void leaf_kernel(LeafArgs a) {
   __shared__ LeafShared<T> sh;
   if(__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     return;
-  leaf_run<T, S, NT, RPT>(a, sh);
+  leaf_run<T, S, NT, RPT, SINGLE>(a, sh);
 }
 
 }  // namespace leaf
 
 // Kernel entry of the FP64 or FP32 leaf with rpt (1 or kLeafRPT) rows per
-// thread (defined in k_leaf*.hip).
+// thread, for one workgroup (single) or several (defined in k_leaf*.hip).
 template <typename T>
-const void* leaf_kernel_ptr(int rpt);
+const void* leaf_kernel_ptr(int rpt, bool single);
 
 }  // namespace hplx
