@@ -71,9 +71,11 @@ struct PanelOp {
 };
 constexpr int kMaxPanelOps = 512;  // steps of one recorded panel
 // Panel height from which HPLX_OPT_PANEL_KERNEL = 2 takes the persistent
-// kernel: below it the launch sequence is faster (measured: N = 16384 and
-// 32768 solves 21 % and 11 % slower with the kernel on every panel; 65536,
-// 98304 and 193280 within run-to-run spread).
+// kernel (a fixed contract of that option).  By itself a panel is faster as
+// launches at every height (896 columns, ms, launches / kernel: 32768 rows 4.2
+// / 6.0, 65536 5.4 / 7.1, 131072 7.3 / 9.4, 193280 9.0 / 11.4); beside an
+// update, which hides it, it makes no difference (the factorisation with N =
+// 98304 9.68 / 9.71 s).
 constexpr int kPanelKernelMinRows = 65536;
 
 // Where a kernel notes the time it starts (stamp.hpp); null: nowhere.

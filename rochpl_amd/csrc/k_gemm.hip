@@ -30,11 +30,13 @@
 //     give each XCD a contiguous range of tiles, walked in groups of
 //     kGroupM tile rows so that concurrently running tiles on one XCD share
 //     A and B strips in that XCD's L2.
-#include "hplx_internal.hpp"
+#include "gemm_tile.hpp"
 #include "stamp.hpp"
 
 namespace hplx {
 namespace {
+
+using namespace gemm;
 
 constexpr int BM      = 128;
 constexpr int BN      = 128;
@@ -45,35 +47,8 @@ constexpr int WN      = 64;
 constexpr int TM      = WM / 16;
 constexpr int TN      = WN / 16;
 constexpr int LDS_LD  = BM + 2;  // even (16-byte rows), staggers LDS banks
-constexpr int kGroupM = 8;
 constexpr int kXcds   = 8;
 constexpr int kTileGrid = 1024;
-
-template <typename V>
-using vec4_t = V __attribute__((ext_vector_type(4)));
-template <typename V>
-using vec2_t = V __attribute__((ext_vector_type(2)));
-
-// V_MFMA_F64_16X16X4_F64 / V_MFMA_F32_16X16X4_F32 operand layout (lane l):
-//   a-operand: X[l % 16][l / 16]   (16 x 4)
-//   b-operand: Y[l / 16][l % 16]   (4 x 16)
-//   result:    D[4*r + l / 16][l % 16], r = 0..3         (f64)
-//              D[4*(l / 16) + r][l % 16], r = 0..3       (f32)
-template <typename V>
-__device__ inline int dl_row(int r, int lane) {
-  if constexpr(sizeof(V) == 8)
-    return 4 * r + (lane >> 4);
-  else
-    return 4 * (lane >> 4) + r;
-}
-
-template <typename V>
-__device__ inline vec4_t<V> mfma16x16x4(V a, V b, vec4_t<V> c) {
-  if constexpr(sizeof(V) == 8)
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 // Stages one 128 x 16 tile of an operand (outer index o = row of A or
 // column of B, inner index k) from global memory into LDS as S[k][o].
@@ -392,157 +367,21 @@ __global__ __launch_bounds__(NT, 2) void dgemm_kernel(
   }
 }
 
-// The same product in small tiles (see pick_tile), BM x BN per workgroup of 4
-// waves in 2 x 2, for aligned operands that are not transposed: K in 32-deep
-// stages through one LDS buffer (the next stage's loads are in flight in
-// registers meanwhile), C loaded along with the first stage.  Every element is
-// the sum over the same MFMA steps as in dgemm_kernel, so the two give the
-// same bits (but for zeros of op(A)'s upper triangle times values that are not
-// finite).
-//
-// Bound by latency (a load, a stage's MFMAs and the store, one after the
-// other) or, tall and thin, by C's and A's traffic; 128 x 128 tiles left most
-// CUs idle (256 x 256, K = 256: 4 tiles) or computed 4 columns for each wanted
-// one (n = 32).
+// The product in small tiles (gemm_tile.hpp; see pick_tile).  128 x 128 tiles
+// left most CUs idle (256 x 256, K = 256: 4 tiles) or computed 4 columns for
+// each wanted one (n = 32).
 template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN>
-__global__ __launch_bounds__(NT) void tile_kernel(
+__global__ __launch_bounds__(kTileThreads) void tile_kernel(
     int M, int N, int K, const V* __restrict__ A, int lda,
     const V* __restrict__ B, int ldb, V* __restrict__ C, int ldc, int tiles_m,
     int tiles_n, Stamps st) {
   stamp_now(st);
-  constexpr int BKS = 32, LA = BM + 2, LB = BN + 2;
-  constexpr int TM = BM / 32, TN = BN / 32;
-  constexpr int QA = BM * BKS / 2 / NT, QB = BN * BKS / 2 / NT;  // pairs per thread
-  constexpr int KA = 2 * NT / BM, OB = 2 * NT / BKS;  // k / columns per pass
-  __shared__ __attribute__((aligned(16))) V sA[BKS * LA];
-  __shared__ __attribute__((aligned(16))) V sB[BKS * LB];
-
+  __shared__ TileShared<V, BM, BN> sh;
   const int per  = gridDim.x / kXcds;
   const int tile = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
   if(tile >= tiles_m * tiles_n) return;
-  const int width  = kGroupM * tiles_n;
-  const int group  = tile / width;
-  const int firstm = group * kGroupM;
-  const int gsz    = min(tiles_m - firstm, kGroupM);
-  const int within = tile - group * width;
-  const int m0     = (firstm + within % gsz) * BM;
-  const int n0     = within / gsz * BN;
-  const int kend   = LOWER_A ? min(K, m0 + BM) : K;
-
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int l16 = lane & 15, lk = lane >> 4;
-  const int wm0 = (wave & 1) * (BM / 2), wn0 = (wave >> 1) * (BN / 2);
-
-  // out-of-range elements are read from a clamped address and replaced by
-  // zero at the LDS store
-  const int ao = 2 * (t % (BM / 2)), ak = t / (BM / 2);
-  const int bk = 2 * (t % (BKS / 2)), bo = t / (BKS / 2);
-  vec2_t<V> ra[QA], rb[QB];
-  // pairs that lie inside, one by one at the edge of an odd extent
-  const bool pairs_a = M % 2 == 0 || m0 + BM <= M;
-  const V*   pa0     = A + min(m0 + ao, pairs_a ? M - 2 : M - 1);
-  const V*   pa1     = A + min(m0 + ao + 1, M - 1);
-  auto load_stage = [&](int k0) {
-    if(pairs_a) {
-#pragma unroll
-      for(int q = 0; q < QA; ++q)
-        ra[q] = *reinterpret_cast<const vec2_t<V>*>(
-            pa0 + static_cast<size_t>(min(k0 + ak + KA * q, kend - 1)) * lda);
-    } else {
-#pragma unroll
-      for(int q = 0; q < QA; ++q) {
-        const size_t c = static_cast<size_t>(min(k0 + ak + KA * q, kend - 1)) * lda;
-        ra[q].x        = pa0[c];
-        ra[q].y        = pa1[c];
-      }
-    }
-    if(kend % 2 == 0 || k0 + BKS <= kend) {
-      const V* pb = B + min(k0 + bk, kend - 2);
-#pragma unroll
-      for(int q = 0; q < QB; ++q)
-        rb[q] = *reinterpret_cast<const vec2_t<V>*>(
-            pb + static_cast<size_t>(min(n0 + bo + OB * q, N - 1)) * ldb);
-    } else {
-      const int b0 = min(k0 + bk, kend - 1), b1 = min(k0 + bk + 1, kend - 1);
-#pragma unroll
-      for(int q = 0; q < QB; ++q) {
-        const V* c = B + static_cast<size_t>(min(n0 + bo + OB * q, N - 1)) * ldb;
-        rb[q].x    = c[b0];
-        rb[q].y    = c[b1];
-      }
-    }
-  };
-  auto store_stage = [&](int k0) {
-#pragma unroll
-    for(int q = 0; q < QA; ++q) {
-      const int  k  = ak + KA * q;
-      const bool in = k0 + k < kend;
-      vec2_t<V>  x;
-      x.x = in && m0 + ao < M ? (NEG ? -ra[q].x : ra[q].x) : V(0);
-      x.y = in && m0 + ao + 1 < M ? (NEG ? -ra[q].y : ra[q].y) : V(0);
-      *reinterpret_cast<vec2_t<V>*>(sA + k * LA + ao) = x;
-    }
-#pragma unroll
-    for(int q = 0; q < QB; ++q) {
-      const int  o  = bo + OB * q;
-      const bool in = n0 + o < N;
-      sB[bk * LB + o]       = in && k0 + bk < kend ? rb[q].x : V(0);
-      sB[(bk + 1) * LB + o] = in && k0 + bk + 1 < kend ? rb[q].y : V(0);
-    }
-  };
-
-  load_stage(0);
-  V cv[TM][TN][4];
-  if(!BETA0) {
-#pragma unroll
-    for(int i = 0; i < TM; ++i)
-#pragma unroll
-      for(int j = 0; j < TN; ++j)
-#pragma unroll
-        for(int r = 0; r < 4; ++r)
-          cv[i][j][r] =
-              C[min(m0 + wm0 + i * 16 + l16, M - 1) +
-                static_cast<size_t>(min(n0 + wn0 + j * 16 + dl_row<V>(r, lane), N - 1)) * ldc];
-  }
-  vec4_t<V> acc[TM][TN];
-#pragma unroll
-  for(int i = 0; i < TM; ++i)
-#pragma unroll
-    for(int j = 0; j < TN; ++j) acc[i][j] = vec4_t<V>{0, 0, 0, 0};
-  for(int k0 = 0; k0 < kend; k0 += BKS) {
-    if(k0 > 0) __syncthreads();
-    store_stage(k0);
-    __syncthreads();
-    if(k0 + BKS < kend) load_stage(k0 + BKS);
-    const V* a_s = sA + lk * LA + wm0 + l16;
-    const V* b_s = sB + lk * LB + wn0 + l16;
-#pragma unroll
-    for(int ks = 0; ks < BKS / 4; ++ks) {
-      V fa[TM], fb[TN];
-#pragma unroll
-      for(int i = 0; i < TM; ++i) fa[i] = a_s[ks * 4 * LA + i * 16];
-#pragma unroll
-      for(int j = 0; j < TN; ++j) fb[j] = b_s[ks * 4 * LB + j * 16];
-#pragma unroll
-      for(int i = 0; i < TM; ++i)
-#pragma unroll
-        for(int j = 0; j < TN; ++j) acc[i][j] = mfma16x16x4<V>(fb[j], fa[i], acc[i][j]);
-    }
-  }
-#pragma unroll
-  for(int i = 0; i < TM; ++i) {
-    const int row = m0 + wm0 + i * 16 + l16;
-    if(row >= M) continue;
-#pragma unroll
-    for(int j = 0; j < TN; ++j)
-#pragma unroll
-      for(int r = 0; r < 4; ++r) {
-        const int col = n0 + wn0 + j * 16 + dl_row<V>(r, lane);
-        if(col < N)
-          C[row + static_cast<size_t>(col) * ldc] =
-              BETA0 ? acc[i][j][r] : cv[i][j][r] + acc[i][j][r];
-      }
-  }
+  gemm_tile<V, BETA0, NEG, LOWER_A, BM, BN>(threadIdx.x, tile, true, M, N, K, A, lda, B,
+                                            ldb, C, ldc, tiles_m, tiles_n, sh);
 }
 
 // a pair of elements (the VEC2 load) is naturally aligned
@@ -578,7 +417,7 @@ hipError_t run_tile(hipStream_t s, int m, int n, int k, const V* A, int lda,
   const long grid = (T + kXcds - 1) / kXcds * kXcds;
   if(grid > 0x7fffffffL) return hipErrorInvalidValue;
   hipLaunchKernelGGL((tile_kernel<V, BETA0, NEG, LOWER_A, BM, BN>),
-                     dim3(static_cast<unsigned>(grid)), dim3(NT), 0, s, m, n, k, A, lda,
+                     dim3(static_cast<unsigned>(grid)), dim3(kTileThreads), 0, s, m, n, k, A, lda,
                      B, ldb, C, ldc, tiles_m, tiles_n, st);
   return hipGetLastError();
 }

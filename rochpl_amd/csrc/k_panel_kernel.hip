@@ -10,13 +10,13 @@
 //   - a leaf is the cooperative register leaf (leaf.hpp, leaf_run), its
 //     pivot exchange through the same candidate slots, one sequence number
 //     per leaf;
-//   - a triangular solve gives each workgroup right-hand-side columns
-//     b, b + G, ... (tri_solve.hpp, one at a time, with the order of
-//     operations of k_trsm.hip);
-//   - a product first transposes its U block into the scratch buffer (32 x 32
-//     tiles through LDS), passes a barrier, then runs the streamed update's
-//     128 x 128 tiles b, b + G, ... (update_tile.hpp, the routine of the
-//     trailing update).
+//   - a triangular solve gives each workgroup blocks of 16 right-hand sides
+//     b, b + G, ... (tri_block.hpp);
+//   - a product gives each workgroup a run of consecutive tiles, two at a time,
+//     one on each half of its threads (gemm_tile.hpp: 64 x 32 up to 32 columns,
+//     else 64 x 64).  With U transposed for the streamed update's 128 x 128
+//     tiles, which took a barrier more, a panel of 131072 x 896 took 10.6 ms,
+//     9.4 now (as launches 7.3).
 // The grid is one workgroup of 512 threads on every CU the panel has, all
 // resident at once: with the look-ahead the CUs the claimed update leaves
 // free, else the whole device.  A leaf runs on the workgroups that hold its
@@ -31,15 +31,12 @@
 // before each launch, so barrier i waits for (i + 1) G arrivals.  Waits are
 // bounded: past the limit the workgroup raises the error flag and every
 // workgroup leaves, as the leaf's own waits do.
-#include "hplx_internal.hpp"
+#include "gemm_tile.hpp"
 #include "leaf.hpp"
-#include "tri_solve.hpp"
-#include "update_tile.hpp"
+#include "tri_block.hpp"
 
 namespace hplx {
 namespace {
-
-using namespace upd;
 
 struct PkArgs {
   double*        P;     // panel top-left
@@ -56,7 +53,6 @@ struct PkArgs {
   uint32_t       leaf_base;  // launch number of the first leaf
   int*           err;
   unsigned*      bar;        // grid barrier counter, zero at launch
-  double*        Bt;         // kMaxNB^2 doubles: the products' U^T
 };
 
 constexpr uint32_t kBarSpinLimit = 1u << 22;
@@ -81,7 +77,7 @@ __device__ bool grid_sync(const PkArgs& a, unsigned target, int* ok_sh) {
         ok = 0;
         break;
       }
-      __builtin_amdgcn_s_sleep(1);
+      __builtin_amdgcn_s_sleep(16);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     *ok_sh = ok;
@@ -90,11 +86,36 @@ __device__ bool grid_sync(const PkArgs& a, unsigned target, int* ok_sh) {
   return *ok_sh != 0;
 }
 
+// C -= A B for a product step, 64 x BN tiles.
+template <int BN>
+__device__ __forceinline__ void product(const PkArgs& a, const PanelOp& o, int rows,
+                                        gemm::TileShared<double, 64, BN> (&sh)[2]) {
+  static_assert(kLeafThreads == 2 * gemm::kTileThreads, "two tiles at a time");
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x / gemm::kTileThreads);
+  const int t    = threadIdx.x % gemm::kTileThreads;
+  const int tm = (rows + 63) / 64, tn = (o.n + BN - 1) / BN, T = tm * tn;
+  const int pairs = (T + 1) / 2, G = gridDim.x;
+  const int per = (pairs + G - 1) / G, p0 = blockIdx.x * per, p1 = min(p0 + per, pairs);
+  for(int p = p0; p < p1; ++p) {
+    if(p > p0) __syncthreads();  // sh is free again
+    const int tile = 2 * p + half;
+    gemm::gemm_tile<double, false, true, false, 64, BN>(
+        t, min(tile, T - 1), tile < T, rows, o.n, o.k,
+        a.P + o.ar + static_cast<size_t>(o.ac) * a.lda, a.lda,
+        a.P + o.br + static_cast<size_t>(o.bc) * a.lda, a.lda,
+        a.P + o.cr + static_cast<size_t>(o.cc) * a.lda, a.lda, tm, tn, sh[half]);
+  }
+}
+
 __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
-  __shared__ leaf::LeafShared<double> sh;
-  __shared__ double           tt[32][33];  // transpose tile
-  __shared__ int              ok_sh;
-  HPLX_USLOT(0) HPLX_USLOT(1) HPLX_USLOT(2) HPLX_USLOT(3)
+  __shared__ union Shared {
+    __device__ Shared() {}
+    leaf::LeafShared<double>         leaf;
+    tri::TriShared<double, kMaxNB>   tri;
+    gemm::TileShared<double, 64, 64> wide[2];
+    gemm::TileShared<double, 64, 32> narrow[2];
+  } sh;
+  __shared__ int ok_sh;
 
   if(__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     return;
@@ -130,46 +151,23 @@ __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
       la.slots       = a.slots;
       la.seq_base    = (a.leaf_base + leaf_i++) << 6;
       la.err         = a.err;
-          la.grid        = gl;
-      if(b < gl) leaf::leaf_run<double, double, kLeafThreads, kLeafRPT, false>(la, sh);
+      la.grid        = gl;
+      if(b < gl) leaf::leaf_run<double, double, kLeafThreads, kLeafRPT, false>(la, sh.leaf);
     } else if(o.kind == kPanelTrsm) {
       const double* T = a.P + o.ar + static_cast<size_t>(o.ac) * a.lda;
-      for(int col = b; col < o.n; col += G)
-        trs::tri_solve_col(o.k, T, a.lda,
-                           a.P + o.br + static_cast<size_t>(o.bc + col) * a.lda);
+      for(int blk = b; 16 * blk < o.n; blk += G) {
+        if(blk > b) __syncthreads();  // sh is free again
+        tri::tri_block<double, double, true, false, kMaxNB>(
+            o.k, o.n, T, a.lda, a.P + o.br + static_cast<size_t>(o.bc) * a.lda, a.lda, blk,
+            sh.tri);
+      }
     } else {
       const int rows = o.m_fix >= 0 ? o.m_fix : a.m - o.m_sub;
       if(rows <= 0) continue;  // uniform over the grid: no barrier owed
-      const int ldt = ut_ld(o.n);
-      // U (k x n at br, bc) -> Bt (row kk holds U(kk, 0 .. n-1))
-      const double* B  = a.P + o.br + static_cast<size_t>(o.bc) * a.lda;
-      const int     gx = (o.k + 31) / 32, gy = (o.n + 31) / 32;
-      const int     tx = t & 31, ty = t >> 5;  // 32 x 16
-      for(int tile = b; tile < gx * gy; tile += G) {
-        const int r0 = (tile % gx) * 32, c0 = (tile / gx) * 32;
-#pragma unroll
-        for(int q = 0; q < 2; ++q) {
-          const int c = c0 + ty + 16 * q, r = r0 + tx;
-          if(r < o.k && c < o.n) tt[ty + 16 * q][tx] = B[r + static_cast<size_t>(c) * a.lda];
-        }
-        __syncthreads();
-#pragma unroll
-        for(int q = 0; q < 2; ++q) {
-          const int r = r0 + ty + 16 * q, c = c0 + tx;
-          if(r < o.k && c < o.n) a.Bt[c + static_cast<size_t>(r) * ldt] = tt[tx][ty + 16 * q];
-        }
-        __syncthreads();
-      }
-      if(!grid_sync(a, ++nbar * G, &ok_sh)) return;
-      const double* A  = a.P + o.ar + static_cast<size_t>(o.ac) * a.lda;
-      double*       C  = a.P + o.cr + static_cast<size_t>(o.cc) * a.lda;
-      const int     tm = (rows + 127) / 128, tn = (o.n + 127) / 128;
-      for(int tile = b; tile < tm * tn; tile += G) {
-        if(tile > b) __syncthreads();  // the LDS ring is free again
-        update_tile(tile, rows, o.n, o.k, A, a.lda, a.Bt, ldt, C, a.lda, tn, tm,
-                    (rows + 1) & ~1, ldt, sA0, sB0, sA1, sB1, sA2, sB2, sA3,
-                    sB3);
-      }
+      if(o.n <= 32)
+        product<32>(a, o, rows, sh.narrow);
+      else
+        product<64>(a, o, rows, sh.wide);
     }
     if(!grid_sync(a, ++nbar * G, &ok_sh)) return;
   }
@@ -195,9 +193,10 @@ hipError_t launch_panel_kernel(Ctx& c, int slot, double* P, int lda, int m,
   int G = c.panel_cus > 0 ? c.panel_cus : c.pk_resident;
   G     = G < c.pk_resident ? G : c.pk_resident;
   G     = G > gl ? G : gl;
-  // every product must take the streamed tile (the launch sequence falls
-  // back to the generic GEMM for the others)
-  double* Bt = panel_scratch(c);
+  // every product must be one that the streamed update takes too (aligned
+  // pairs, a multiple of 8 columns of A); the launch sequence falls back to
+  // the generic GEMM for the others
+  const double* Bt = panel_scratch(c);
   for(const PanelOp& o : ops) {
     if(o.kind != kPanelGemm) continue;
     const int rows = o.m_fix >= 0 ? o.m_fix : m - o.m_sub;
@@ -232,7 +231,6 @@ hipError_t launch_panel_kernel(Ctx& c, int slot, double* P, int lda, int m,
   a.leaf_base  = c.leaf_launches + 1;
   a.err        = c.flags + 1;
   a.bar        = c.pbar;
-  a.Bt         = Bt;
   c.leaf_launches += nleaf;
   hipError_t e = launch_zero_ints(s, reinterpret_cast<int*>(c.pbar), 1);
   if(e != hipSuccess) return e;

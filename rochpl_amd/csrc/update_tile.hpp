@@ -1,8 +1,6 @@
 // One 128 x 128 tile of the streamed FP64 update C -= A * Bt^T (the tile
 // routine of update_kernel, update_claimed_kernel and update_resume_kernel
-// in k_update.hip, whose header describes the stage pipeline), shared with
-// the persistent panel kernel (k_panel_kernel.hip), which runs the panel
-// recursion's products with it.
+// in k_update.hip, whose header describes the stage pipeline).
 #pragma once
 
 #include <hip/hip_runtime.h>
