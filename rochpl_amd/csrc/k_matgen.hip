@@ -21,7 +21,10 @@ namespace {
 constexpr int kGenRows = 256;  // rows per block (one per thread)
 constexpr int kGenCols = 256;  // columns per block
 constexpr int kChkCols = 4096; // columns per partial-sum chunk (row pass)
-constexpr int kChkRows = 4096; // rows per partial-sum chunk (column pass)
+constexpr int kChkR    = 4;    // rows per thread of the whole check
+constexpr int kChkRows = 256 * kChkR;  // and of its workgroups
+constexpr int kChkSub  = 256;  // columns whose sums are kept in LDS at once
+constexpr int kChkStep = 8;    // columns between two reductions
 
 // T: stored type.  FP32 storage holds RN_fp32(v); FP16 storage holds
 // RN_fp16(RN_fp32(v)) of the FP64 generator value v.
@@ -76,41 +79,127 @@ __global__ __launch_bounds__(256) void check_rows_kernel(
   __syncthreads();
   const int i = bx * 256 + threadIdx.x;
   if(i >= n) return;
-  uint64_t s = lcg_state(seed, static_cast<uint64_t>(i) +
-                                   static_cast<uint64_t>(j0) *
-                                       static_cast<uint64_t>(n));
+  // four columns' states at a time: the chain of dependent products is a
+  // quarter as long; the sums keep their order
+  uint64_t s[4], a4 = colA, c4 = colC;
+  s[0] = lcg_state(seed, static_cast<uint64_t>(i) +
+                             static_cast<uint64_t>(j0) * static_cast<uint64_t>(n));
+#pragma unroll
+  for(int q = 1; q < 4; ++q) s[q] = colA * s[q - 1] + colC;
+#pragma unroll
+  for(int q = 0; q < 2; ++q) {  // the map of four columns
+    c4 = a4 * c4 + c4;
+    a4 = a4 * a4;
+  }
   double acc = 0.0, aabs = 0.0;
-  for(int t = 0; t < jn; ++t) {
-    double v = lcg_value(s);
-    if(i == j0 + t) v += shift;
-    acc  = fma(v, sx[t], acc);
-    aabs += fabs(v);
-    s = colA * s + colC;
+  for(int t0 = 0; t0 < jn; t0 += 4) {
+#pragma unroll
+    for(int q = 0; q < 4; ++q) {
+      if(t0 + q < jn) {
+        double v = lcg_value(s[q]);
+        if(i == j0 + t0 + q) v += shift;
+        acc = fma(v, sx[t0 + q], acc);
+        aabs += fabs(v);
+      }
+      s[q] = a4 * s[q] + c4;
+    }
   }
   part_r[static_cast<size_t>(c) * n + i] = acc;
   part_a[static_cast<size_t>(c) * n + i] = aabs;
 }
 
-// Column pass: part_c[rc*n + j] = sum_{i in row chunk rc} |a(i,j)|.
-__global__ __launch_bounds__(256) void check_cols_kernel(
-    int n, uint64_t seed, double shift, double* __restrict__ part_c, int gx) {
-  const int bx = blockIdx.x % gx;
-  const int rc = blockIdx.x / gx;
-  const int j  = bx * 256 + threadIdx.x;
-  if(j >= n) return;
-  const int i0 = rc * kChkRows;
-  const int in = min(n, i0 + kChkRows);
-  uint64_t s = lcg_state(seed, static_cast<uint64_t>(i0) +
-                                   static_cast<uint64_t>(j) *
-                                       static_cast<uint64_t>(n));
-  double aabs = 0.0;
-  for(int i = i0; i < in; ++i) {
-    double v = lcg_value(s);
-    if(i == j) v += shift;
-    aabs += fabs(v);
-    s = kLcgMult * s + kLcgAdd;
+// The whole check in one pass: part_r and part_a as above for chunks of `cc`
+// columns, and part_c[rc*n + j] = sum_{i in row chunk rc} |a(i,j)|.  A thread
+// has kChkR rows; a column's sum over them goes to LDS, and every kChkStep
+// columns each wave adds up its 64 lanes' (8 lanes to a column).
+//
+// Bound by the integer units: 3 products, 2 conversions and 6 other operations
+// an element, once instead of once per row and once per column; the diagonal
+// is looked for only where it can be.  N = 20000 540 us in two passes, 335 in
+// this one.
+// EDGE: the step's rows may cross the diagonal or the last row.
+template <bool EDGE>
+__device__ __forceinline__ void check_step(int i, int j, uint64_t (&s)[kChkR],
+                                           double (&acc)[kChkR], double (&aabs)[kChkR],
+                                           double x, double shift, uint64_t colA,
+                                           uint64_t colC, const bool (&in)[kChkR],
+                                           double& sum) {
+  sum = 0.0;
+#pragma unroll
+  for(int q = 0; q < kChkR; ++q) {
+    double v = lcg_value(s[q]);
+    if(EDGE && i + 256 * q == j) v += shift;
+    acc[q] = fma(v, x, acc[q]);
+    aabs[q] += fabs(v);
+    sum += !EDGE || in[q] ? fabs(v) : 0.0;
+    s[q] = colA * s[q] + colC;
   }
-  part_c[static_cast<size_t>(rc) * n + j] = aabs;
+}
+
+__global__ __launch_bounds__(256) void check_kernel(
+    int n, int cc, uint64_t seed, double shift, const double* __restrict__ X,
+    double* __restrict__ part_r, double* __restrict__ part_a,
+    double* __restrict__ part_c, uint64_t colA, uint64_t colC, int gx) {
+  __shared__ double sx[kChkSub];
+  __shared__ double tile[4][kChkStep][64];
+  __shared__ double sums[4][kChkSub];
+  const int bx = blockIdx.x % gx, c = blockIdx.x / gx;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int i = bx * kChkRows + t;
+  const int j0 = c * cc, j1 = min(n, j0 + cc);
+  uint64_t  s[kChkR];
+  double    acc[kChkR], aabs[kChkR];
+  bool      in[kChkR];
+#pragma unroll
+  for(int q = 0; q < kChkR; ++q) {
+    s[q] = lcg_state(seed, static_cast<uint64_t>(i + 256 * q) +
+                               static_cast<uint64_t>(j0) * static_cast<uint64_t>(n));
+    in[q]  = i + 256 * q < n;
+    acc[q] = aabs[q] = 0.0;
+  }
+  for(int js = j0; js < j1; js += kChkSub) {
+    const int jn = min(kChkSub, j1 - js);
+    __syncthreads();  // sx and sums are free again
+    if(t < jn) sx[t] = X[js + t];
+    __syncthreads();
+    const bool edge = (js < (bx + 1) * kChkRows && js + jn > bx * kChkRows) ||
+                      (bx + 1) * kChkRows > n;
+    for(int u0 = 0; u0 < jn; u0 += kChkStep) {
+      const int un = min(kChkStep, jn - u0);
+      for(int u = 0; u < un; ++u) {
+        double sum;
+        if(edge)
+          check_step<true>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
+                           sum);
+        else
+          check_step<false>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
+                            sum);
+        tile[wave][u][lane] = sum;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // lane 8 u + p: an eighth of column u
+      double p = 0.0;
+      if((lane >> 3) < un)
+#pragma unroll
+        for(int k = 0; k < 8; ++k) p += tile[wave][lane >> 3][8 * k + (lane & 7)];
+      p += __shfl_xor(p, 1);
+      p += __shfl_xor(p, 2);
+      p += __shfl_xor(p, 4);
+      if((lane & 7) == 0 && (lane >> 3) < un) sums[wave][u0 + (lane >> 3)] = p;
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    if(t < jn)
+      part_c[static_cast<size_t>(bx) * n + js + t] =
+          (sums[0][t] + sums[1][t]) + (sums[2][t] + sums[3][t]);
+  }
+#pragma unroll
+  for(int q = 0; q < kChkR; ++q)
+    if(in[q]) {
+      part_r[static_cast<size_t>(c) * n + i + 256 * q] = acc[q];
+      part_a[static_cast<size_t>(c) * n + i + 256 * q] = aabs[q];
+    }
 }
 
 __device__ inline double block_max(double v, double* sh) {
@@ -302,9 +391,19 @@ hipError_t launch_matgen(hipStream_t s, int m, int n, __half* A, int lda,
   return matgen_t(s, m, n, A, lda, seed, diag_shift);
 }
 
+// Columns per chunk of the check: as many as leave 4096 workgroups, 4096 at
+// most (the partial sums of the rows are n x 2 per chunk).
+static int check_cols(int n) {
+  const long rows = (n + kChkRows - 1) / kChkRows;
+  int        cc   = 4096;
+  while(cc > kChkSub && rows * ((n + cc - 1) / cc) < 4096) cc /= 2;
+  return cc;
+}
+
 size_t check_part_len(int n) {
   if(n <= 0) return 16;
-  const size_t nch_c = (n + kChkCols - 1) / kChkCols;
+  const int    cc    = check_cols(n);
+  const size_t nch_c = (n + cc - 1) / cc;
   const size_t nch_r = (n + kChkRows - 1) / kChkRows;
   const size_t nblk  = (n + 255) / 256;
   return (2 * nch_c + nch_r) * static_cast<size_t>(n) + 8 + 8 * nblk + 16;
@@ -315,7 +414,8 @@ hipError_t launch_check(hipStream_t s, int n, int seed, double diag_shift,
                         double* out_dev) {
   if(n <= 0) return hipErrorInvalidValue;
   if(part_len < check_part_len(n)) return hipErrorInvalidValue;
-  const int nch_c = (n + kChkCols - 1) / kChkCols;
+  const int cc    = check_cols(n);
+  const int nch_c = (n + cc - 1) / cc;
   const int nch_r = (n + kChkRows - 1) / kChkRows;
   const int nblk  = (n + 255) / 256;
   double* part_r = part;
@@ -324,13 +424,9 @@ hipError_t launch_check(hipStream_t s, int n, int seed, double diag_shift,
   double* bp     = part_c + static_cast<size_t>(nch_r) * n;
   const Affine colj = lcg_jump(static_cast<uint64_t>(n));
   const uint64_t sd = static_cast<uint64_t>(seed);
-  hipLaunchKernelGGL(check_rows_kernel,
-                     dim3(static_cast<unsigned>(nblk) * nch_c), dim3(256), 0, s,
-                     n, sd, diag_shift, X, part_r, part_a, colj.a, colj.c,
-                     nblk);
-  hipLaunchKernelGGL(check_cols_kernel,
-                     dim3(static_cast<unsigned>(nblk) * nch_r), dim3(256), 0, s,
-                     n, sd, diag_shift, part_c, nblk);
+  hipLaunchKernelGGL(check_kernel, dim3(static_cast<unsigned>(nch_r) * nch_c),
+                     dim3(256), 0, s, n, cc, sd, diag_shift, X, part_r, part_a, part_c,
+                     colj.a, colj.c, nch_r);
   hipLaunchKernelGGL(check_finish_kernel, dim3(nblk), dim3(256), 0, s, n,
                      nch_c, nch_r, sd, X, part_r, part_a, part_c, bp);
   hipLaunchKernelGGL(check_reduce_kernel, dim3(1), dim3(256), 0, s, n, nblk,
