@@ -38,8 +38,8 @@
 // rather than 64-row ones: half the trips (that U 1115 us).
 //
 // hplx_pdgetrs, before and now: N = 16384, NB = 512, 64 right-hand sides 9.50
-// -> 2.78 ms (transposed 8.92 -> 3.51), one 9.27 -> 1.69, 512 15.2 -> 9.9;
-// N = 5000, NB = 128, one 2.87 -> 0.77 ms.  The floor is one read of the
+// -> 2.69 ms (transposed 8.92 -> 3.46), one 9.27 -> 1.60, 512 15.2 -> 9.6;
+// N = 5000, NB = 128, one 2.87 -> 0.69 ms.  The floor is one read of the
 // factors (2.1 GB, 0.4 ms).
 #include "hplx_internal.hpp"
 #include "lds_stream.hpp"
@@ -79,17 +79,33 @@ struct FlowArgs {
   int           ns;      // slices of 16 right-hand sides
   unsigned long long* x;      // nd x ns blocks of 2 halves of 16 x 64 values
   int*                flags;  // nd x ns
+  // The interchanges of a panel of L, applied as B is loaded (null: none): perm
+  // as launch_pipid composes it, relative to d0; top: the panel's rows of B as
+  // they were before it (leading dimension d1 - d0), whose places in B the
+  // solved blocks take; next: where the first rows below go for the next panel
+  // (next_rows of them; null: nowhere).
+  const int*    perm;
+  const double* top;
+  double*       next;
+  int           next_rows;
 };
 
 // The exchange buffer's filling: a NaN no computed value has (those that
 // would be published are replaced by the plain quiet NaN).
 constexpr unsigned long long kEmpty = 0x7ff8b10cffffb10cull;
 
+// Also copies the first `rows` rows of B's nrhs columns to top, if it is not
+// null.
 __global__ __launch_bounds__(256) void fill_kernel(unsigned long long* p, int n,
-                                                   int* flags, int nf) {
+                                                   int* flags, int nf,
+                                                   const double* B, int ldb, int nrhs,
+                                                   double* top, int rows) {
   const int i0 = blockIdx.x * 256 + threadIdx.x;
   for(int i = i0; i < n; i += gridDim.x * 256) p[i] = kEmpty;
   if(i0 < nf) flags[i0] = 0;
+  if(top)
+    for(int i = i0; i < rows * nrhs; i += gridDim.x * 256)
+      top[i] = B[i % rows + static_cast<size_t>(i / rows) * ldb];
 }
 
 // A wave's 16 rows x 64 columns of op(T): lane (m, g) holds T(row0 + m,
@@ -268,6 +284,7 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
   __shared__ __attribute__((aligned(16))) double tri[2 * kTri];
   __shared__ double scale[2 * kFH];
   __shared__ int    rare;
+  __shared__ int    from[kFB];  // where the block's rows of B come from
   // the slices of a block on one XCD (they read the same rows of T), blocks
   // in index order
   const int per = 8 * a.ns, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
@@ -292,9 +309,35 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
   double*         Bc = a.B + r0 + static_cast<size_t>(c0 + ac) * a.ldb;
   // the products are summed by themselves and added to B at the end
   typename P::Acc acc = P::zero(), b = P::zero();
+  bool swap = false;
+  if constexpr(!TRANS && !BACK) swap = a.perm != nullptr;
+  if(swap) {
+    // from: a row of top (>= 0) or of B (< 0: minus the row from d0, minus 1)
+    const int jb = a.d1 - a.d0;
+    if(t < kFB) {
+      const int q = r - a.d0 + t;  // the row, from d0
+      const int f = diag ? (t < w ? a.perm[q] : 0) : q;
+      from[t]     = f < jb ? f : -f - 1;
+    }
+    __syncthreads();
+    if(!diag)  // the panel's rows that were moved into this block
+      for(int k = t; k < jb; k += 512) {
+        const int q = a.perm[jb + k] - (r - a.d0);
+        if(q >= 0 && q < w) from[q] = k;
+      }
+    __syncthreads();
 #pragma unroll
-  for(int e = 0; e < E; ++e)
-    if(P::row(e) < nr && ac < nc) b[e] = Bc[P::row(e)];
+    for(int e = 0; e < E; ++e)
+      if(P::row(e) < nr && ac < nc) {
+        const int f = from[16 * wave + P::row(e)];
+        b[e]        = f >= 0 ? a.top[f + static_cast<size_t>(c0 + ac) * jb]
+                             : a.B[a.d0 - f - 1 + static_cast<size_t>(c0 + ac) * a.ldb];
+      }
+  } else {
+#pragma unroll
+    for(int e = 0; e < E; ++e)
+      if(P::row(e) < nr && ac < nc) b[e] = Bc[P::row(e)];
+  }
   double tv[16], tn[16];
   if(diag) {
     if(t == 0) rare = 0;
@@ -366,9 +409,16 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     acc += block_product<WIDE>(tv, x);
   }
   if(!diag) {
+    // (a row that a block on the diagonal takes from here was read before that
+    // block's x appeared)
 #pragma unroll
     for(int e = 0; e < E; ++e)
-      if(P::row(e) < nr && ac < nc) Bc[P::row(e)] = b[e] + acc[e];
+      if(P::row(e) < nr && ac < nc) {
+        const double v = b[e] + acc[e];
+        const int    q = r0 - a.d1 + P::row(e);
+        Bc[P::row(e)]  = v;
+        if(swap && q < a.next_rows) a.next[q + static_cast<size_t>(c0 + ac) * a.next_rows] = v;
+      }
     return;
   }
   for(int h = 0; h < 2; ++h) {
@@ -435,6 +485,14 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A panel's interchanges and where its rows of B are kept (FlowArgs).
+struct FlowSwap {
+  const int*    perm      = nullptr;
+  const double* top       = nullptr;
+  double*       next      = nullptr;
+  int           next_rows = 0;
+};
+
 // The solves of one call on a stream, for at most kFlowCols right-hand sides.
 struct Flow {
   hipStream_t        s;
@@ -459,12 +517,14 @@ struct Flow {
     return static_cast<size_t>(bpp) * slices() * group() * kFB;
   }
 
-  // np panels' (of bpp blocks) x marked as not there yet
-  hipError_t prepare(int np, int bpp) {
+  // np panels' (of bpp blocks) x marked as not there yet, and the first `rows`
+  // rows of B kept in top (if not null)
+  hipError_t prepare(int np, int bpp, double* top = nullptr, int top_rows = 0) {
     if(np * bpp > blocks()) return hipErrorInvalidValue;
     const int n = static_cast<int>(x_panel(bpp)) * np;
     hipLaunchKernelGGL(fill_kernel, dim3(n < 256 * 1024 ? (n + 255) / 256 : 1024),
-                       dim3(256), 0, s, w.x, n, w.flags, np * bpp * slices());
+                       dim3(256), 0, s, w.x, n, w.flags, np * bpp * slices(), B, ldb,
+                       nrhs, top, top_rows);
     return hipGetLastError();
   }
 
@@ -483,14 +543,15 @@ struct Flow {
   // op(T) on rows [d0, d1) solved, then applied to rows [o0, o1); block: the
   // index of the first of these blocks among the prepared ones.
   hipError_t solve(bool trans, bool back, int d0, int d1, int o0, int o1,
-                   int block) {
-    if(!split()) return flow(trans, back, d0, d1, o0, o1, block);
+                   int block, const FlowSwap& sw = FlowSwap()) {
+    if(!split()) return flow(trans, back, d0, d1, o0, o1, block, sw);
     const int n = (d1 - d0 + kSplitRows - 1) / kSplitRows;
     for(int k = 0; k < n; ++k) {
       const int q  = back ? n - 1 - k : k;
       const int s0 = d0 + q * kSplitRows;
       const int s1 = s0 + kSplitRows < d1 ? s0 + kSplitRows : d1;
-      hipError_t e = flow(trans, back, s0, s1, s0, s0, block + q * (kSplitRows / kFB));
+      hipError_t e =
+          flow(trans, back, s0, s1, s0, s0, block + q * (kSplitRows / kFB), FlowSwap());
       // the rows of the diagonal range still to be solved, then the others
       if(e == hipSuccess) e = back ? update(trans, s0, s1, d0, s0) : update(trans, s0, s1, s1, d1);
       if(e == hipSuccess) e = update(trans, s0, s1, o0, o1);
@@ -511,8 +572,13 @@ struct Flow {
                          B + o0, ldb);
   }
 
-  hipError_t flow(bool trans, bool back, int d0, int d1, int o0, int o1, int block) {
+  hipError_t flow(bool trans, bool back, int d0, int d1, int o0, int o1, int block,
+                  const FlowSwap& sw) {
     FlowArgs a;
+    a.perm      = sw.perm;
+    a.top       = sw.top;
+    a.next      = sw.next;
+    a.next_rows = sw.next_rows;
     a.T     = T;
     a.ldt   = ldt;
     a.x     = w.x + x_panel(block);
@@ -584,10 +650,18 @@ static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
   const int np  = (N + nb - 1) / nb;
   const int bpp = (nb + kFB - 1) / kFB;
   const int pc  = f.blocks() / bpp;  // panels prepared at once
+  // Few right-hand sides: a panel's interchanges are applied by the launch that
+  // solves with it, its rows kept in one half of the work buffer while the
+  // first rows below go to the other half for the next panel.  A launch of
+  // their own took 4.6 us a panel (N = 5000, NB = 128, one right-hand side 0.74
+  // ms with it, 0.69 without; N = 1000, NB = 64, five 0.226, 0.200).
+  const size_t half  = static_cast<size_t>(nb) * nrhs;
+  const bool   fused = !f.split() && 2 * half <= w.work_doubles;
   // panels [p0, p0 + pc): their exchange buffers, and the interchanges composed
   auto prepare = [&](int p0) -> hipError_t {
     const int p1 = p0 + pc < np ? p0 + pc : np;
-    HCHK(f.prepare(p1 - p0, bpp));
+    HCHK(f.prepare(p1 - p0, bpp, fused && !trans && p0 == 0 ? w.work : nullptr,
+                   nb < N ? nb : N));
     return launch_pipid_panels(s, p1 - p0, nb, N - p0 * nb, ipiv + p0 * nb,
                                p0 * nb, w.perm);
   };
@@ -597,8 +671,17 @@ static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
     for(int p = 0; p < np; ++p) {
       const int j = p * nb, jb = (N - j) < nb ? (N - j) : nb, pi = p % pc;
       if(pi == 0) HCHK(prepare(p));
-      HCHK(launch_swap_inplace(s, jb, nrhs, B + j, ldb, w.perm + pi * 2 * nb));
-      HCHK(f.solve(false, false, j, j + jb, j + jb, N, pi * bpp));
+      FlowSwap sw;
+      if(fused) {
+        const int left = N - j - jb;
+        sw.perm      = w.perm + pi * 2 * nb;
+        sw.top       = w.work + (p & 1) * half;
+        sw.next      = w.work + (1 - (p & 1)) * half;
+        sw.next_rows = left < nb ? left : nb;
+      } else {
+        HCHK(launch_swap_inplace(s, jb, nrhs, B + j, ldb, w.perm + pi * 2 * nb));
+      }
+      HCHK(f.solve(false, false, j, j + jb, j + jb, N, pi * bpp, sw));
     }
     return f.upper(N);
   }
