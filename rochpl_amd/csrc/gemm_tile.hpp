@@ -39,6 +39,82 @@ __device__ inline vec4_t<V> mfma16x16x4(V a, V b, vec4_t<V> c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
+// One operand of a tile, BO outer indices (rows of C for A, columns for B) by
+// kTileK of k, staged as S[k][o] with pitch BO + 2.  KFAST: k is the contiguous
+// index in memory, else o.  Pairs are loaded whole where they lie inside and
+// one by one at the edge of an odd extent; out-of-range elements are read from
+// a clamped address and replaced by zero at the store.
+template <typename V, int BO, bool KFAST>
+struct TileOperand {
+  static constexpr int Q    = BO * kTileK / 2 / kTileThreads;  // pairs per thread
+  static constexpr int LD   = BO + 2;
+  static constexpr int STEP = 2 * kTileThreads / (KFAST ? kTileK : BO);
+  const V* __restrict__ P;
+  int       ld, o0, O, o, k;
+  vec2_t<V> r[Q];
+
+  __device__ __forceinline__ TileOperand(const V* P_, int ld_, int o0_, int O_, int t)
+      : P(P_), ld(ld_), o0(o0_), O(O_),
+        o(KFAST ? t / (kTileK / 2) : 2 * (t % (BO / 2))),
+        k(KFAST ? 2 * (t % (kTileK / 2)) : t / (BO / 2)) {}
+
+  __device__ __forceinline__ void load(int k0, int kend) {
+    if constexpr(!KFAST) {
+      if(O % 2 == 0 || o0 + BO <= O) {
+        const V* p = P + min(o0 + o, O % 2 == 0 ? O - 2 : O - 1);
+#pragma unroll
+        for(int q = 0; q < Q; ++q)
+          r[q] = *reinterpret_cast<const vec2_t<V>*>(
+              p + static_cast<size_t>(min(k0 + k + STEP * q, kend - 1)) * ld);
+      } else {
+        const V *p0 = P + min(o0 + o, O - 1), *p1 = P + min(o0 + o + 1, O - 1);
+#pragma unroll
+        for(int q = 0; q < Q; ++q) {
+          const size_t c = static_cast<size_t>(min(k0 + k + STEP * q, kend - 1)) * ld;
+          r[q].x         = p0[c];
+          r[q].y         = p1[c];
+        }
+      }
+    } else {
+      if(kend % 2 == 0 || k0 + kTileK <= kend) {
+        const V* p = P + min(k0 + k, kend - 2);
+#pragma unroll
+        for(int q = 0; q < Q; ++q)
+          r[q] = *reinterpret_cast<const vec2_t<V>*>(
+              p + static_cast<size_t>(min(o0 + o + STEP * q, O - 1)) * ld);
+      } else {
+        const int c0 = min(k0 + k, kend - 1), c1 = min(k0 + k + 1, kend - 1);
+#pragma unroll
+        for(int q = 0; q < Q; ++q) {
+          const V* c = P + static_cast<size_t>(min(o0 + o + STEP * q, O - 1)) * ld;
+          r[q].x     = c[c0];
+          r[q].y     = c[c1];
+        }
+      }
+    }
+  }
+
+  template <bool NEG>
+  __device__ __forceinline__ void store(V* S, int k0, int kend) const {
+#pragma unroll
+    for(int q = 0; q < Q; ++q) {
+      const int  kq = KFAST ? k : k + STEP * q, oq = KFAST ? o + STEP * q : o;
+      const bool ix = o0 + oq < O && k0 + kq < kend;
+      const bool iy = KFAST ? o0 + oq < O && k0 + kq + 1 < kend
+                            : o0 + oq + 1 < O && k0 + kq < kend;
+      vec2_t<V>  x;
+      x.x = ix ? (NEG ? -r[q].x : r[q].x) : V(0);
+      x.y = iy ? (NEG ? -r[q].y : r[q].y) : V(0);
+      if constexpr(KFAST) {
+        S[kq * LD + oq]       = x.x;
+        S[(kq + 1) * LD + oq] = x.y;
+      } else {
+        *reinterpret_cast<vec2_t<V>*>(S + kq * LD + oq) = x;
+      }
+    }
+  }
+};
+
 template <typename V, int BM, int BN>
 struct TileShared {
   alignas(16) V a[kTileK * (BM + 2)];
@@ -46,9 +122,9 @@ struct TileShared {
 };
 
 // Tile `tile` (rows first within groups of kGroupM tile rows) of C (M x N) =
-// beta C + alpha A B, BM x BN on 4 waves in 2 x 2 (t: the thread among them),
-// for 16-byte aligned operands with even leading dimensions that are not
-// transposed: K in 32-deep stages through one LDS buffer (the next stage's
+// beta C + alpha op(A) op(B), BM x BN on 4 waves in 2 x 2 (t: the thread among
+// them), for 16-byte aligned operands with even leading dimensions (TA / TB:
+// stored transposed): K in 32-deep stages through one LDS buffer (the next stage's
 // loads are in flight in registers meanwhile), C loaded along with the first
 // stage.  Every element is the sum over the same MFMA steps as in
 // k_gemm.hip's dgemm_kernel, so the two give the same bits (but for zeros of
@@ -57,16 +133,15 @@ struct TileShared {
 //
 // Bound by latency (a load, a stage's MFMAs and the store, one after the
 // other) or, tall and thin, by C's and A's traffic.
-template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN>
+template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN, bool TA = false,
+          bool TB = false>
 __device__ __forceinline__ void gemm_tile(int t, int tile, bool live, int M, int N, int K,
                                           const V* __restrict__ A, int lda,
                                           const V* __restrict__ B, int ldb,
                                           V* __restrict__ C, int ldc, int tiles_m,
                                           int tiles_n, TileShared<V, BM, BN>& sh) {
-  constexpr int NT = kTileThreads, BKS = kTileK, LA = BM + 2, LB = BN + 2;
+  constexpr int BKS = kTileK, LA = BM + 2, LB = BN + 2;
   constexpr int TM = BM / 32, TN = BN / 32;
-  constexpr int QA = BM * BKS / 2 / NT, QB = BN * BKS / 2 / NT;  // pairs per thread
-  constexpr int KA = 2 * NT / BM, OB = 2 * NT / BKS;  // k / columns per pass
   const int width  = kGroupM * tiles_n;
   const int group  = tile / width;
   const int firstm = group * kGroupM;
@@ -80,65 +155,10 @@ __device__ __forceinline__ void gemm_tile(int t, int tile, bool live, int M, int
   const int l16 = lane & 15, lk = lane >> 4;
   const int wm0 = (wave & 1) * (BM / 2), wn0 = (wave >> 1) * (BN / 2);
 
-  // out-of-range elements are read from a clamped address and replaced by
-  // zero at the LDS store
-  const int ao = 2 * (t % (BM / 2)), ak = t / (BM / 2);
-  const int bk = 2 * (t % (BKS / 2)), bo = t / (BKS / 2);
-  vec2_t<V> ra[QA], rb[QB];
-  // pairs that lie inside, one by one at the edge of an odd extent
-  const bool pairs_a = M % 2 == 0 || m0 + BM <= M;
-  const V*   pa0     = A + min(m0 + ao, pairs_a ? M - 2 : M - 1);
-  const V*   pa1     = A + min(m0 + ao + 1, M - 1);
-  auto load_stage = [&](int k0) {
-    if(pairs_a) {
-#pragma unroll
-      for(int q = 0; q < QA; ++q)
-        ra[q] = *reinterpret_cast<const vec2_t<V>*>(
-            pa0 + static_cast<size_t>(min(k0 + ak + KA * q, kend - 1)) * lda);
-    } else {
-#pragma unroll
-      for(int q = 0; q < QA; ++q) {
-        const size_t c = static_cast<size_t>(min(k0 + ak + KA * q, kend - 1)) * lda;
-        ra[q].x        = pa0[c];
-        ra[q].y        = pa1[c];
-      }
-    }
-    if(kend % 2 == 0 || k0 + BKS <= kend) {
-      const V* pb = B + min(k0 + bk, kend - 2);
-#pragma unroll
-      for(int q = 0; q < QB; ++q)
-        rb[q] = *reinterpret_cast<const vec2_t<V>*>(
-            pb + static_cast<size_t>(min(n0 + bo + OB * q, N - 1)) * ldb);
-    } else {
-      const int b0 = min(k0 + bk, kend - 1), b1 = min(k0 + bk + 1, kend - 1);
-#pragma unroll
-      for(int q = 0; q < QB; ++q) {
-        const V* c = B + static_cast<size_t>(min(n0 + bo + OB * q, N - 1)) * ldb;
-        rb[q].x    = c[b0];
-        rb[q].y    = c[b1];
-      }
-    }
-  };
-  auto store_stage = [&](int k0) {
-#pragma unroll
-    for(int q = 0; q < QA; ++q) {
-      const int  k  = ak + KA * q;
-      const bool in = k0 + k < kend;
-      vec2_t<V>  x;
-      x.x = in && m0 + ao < M ? (NEG ? -ra[q].x : ra[q].x) : V(0);
-      x.y = in && m0 + ao + 1 < M ? (NEG ? -ra[q].y : ra[q].y) : V(0);
-      *reinterpret_cast<vec2_t<V>*>(sh.a + k * LA + ao) = x;
-    }
-#pragma unroll
-    for(int q = 0; q < QB; ++q) {
-      const int  o  = bo + OB * q;
-      const bool in = n0 + o < N;
-      sh.b[bk * LB + o]       = in && k0 + bk < kend ? rb[q].x : V(0);
-      sh.b[(bk + 1) * LB + o] = in && k0 + bk + 1 < kend ? rb[q].y : V(0);
-    }
-  };
-
-  load_stage(0);
+  TileOperand<V, BM, TA>  la(A, lda, m0, M, t);
+  TileOperand<V, BN, !TB> lb(B, ldb, n0, N, t);
+  la.load(0, kend);
+  lb.load(0, kend);
   V cv[TM][TN][4];
   if(!BETA0) {
 #pragma unroll
@@ -158,9 +178,13 @@ __device__ __forceinline__ void gemm_tile(int t, int tile, bool live, int M, int
     for(int j = 0; j < TN; ++j) acc[i][j] = vec4_t<V>{0, 0, 0, 0};
   for(int k0 = 0; k0 < kend; k0 += BKS) {
     if(k0 > 0) __syncthreads();
-    store_stage(k0);
+    la.template store<NEG>(sh.a, k0, kend);
+    lb.template store<false>(sh.b, k0, kend);
     __syncthreads();
-    if(k0 + BKS < kend) load_stage(k0 + BKS);
+    if(k0 + BKS < kend) {
+      la.load(k0 + BKS, kend);
+      lb.load(k0 + BKS, kend);
+    }
     const V* a_s = sh.a + lk * LA + wm0 + l16;
     const V* b_s = sh.b + lk * LB + wn0 + l16;
 #pragma unroll

@@ -21,11 +21,11 @@ constexpr int kLeafThreads = 512;   // threads per leaf workgroup
 constexpr int kLeafRPT     = 3;     // rows per thread of the tall leaves
 // Rows per thread of a leaf of R rows: one where at most 512 rows fit one
 // workgroup or 32 workgroups hold them, since the time per column falls with
-// the rows of a thread (500 rows 47 against 67 us, 4000 FP32 88 against 109,
-// 16000 FP64 114 against 119); three for 513 .. 1536 rows, which then need no
-// exchange between workgroups (1500 rows 70 against 78 us), and above 16384
-// rows, where the number of workgroups costs more (48000 rows 131 .. 139 us
-// either way, 131072 155 against 212).
+// the rows of a thread (2048 rows 86 against 100 us, 4096 89 against 102, 9001
+// 92 against 104, 16000 100 against 108); three for 513 .. 1536 rows, which
+// then need no exchange between workgroups (1500 rows 65 us, 1600 with it 86),
+// and above 16384 rows, where the number of workgroups costs more (131072 rows
+// 155 against 212 when that was measured).
 inline int leaf_rpt(int R) {
   return R <= kLeafThreads || (R > kLeafThreads * kLeafRPT && R <= 32 * kLeafThreads)
              ? 1
@@ -400,7 +400,7 @@ hipError_t launch_nn_sub(hipStream_t s, int K, int m, int n, const double* A,
                          int lda, const double* B, int ldb, double* C,
                          int ldc);
 // C (m x n, ldc) = -A B^T for A (m x K, lda) and B (n x K, ldb): the
-// adjoint's gradA = -gradB X^T (write-bound; same kernel as launch_tn_sub).
+// adjoint's gradA = -gradB X^T (launch_dgemm's tiles).
 hipError_t launch_outer_neg(hipStream_t s, int K, int m, int n,
                             const double* A, int lda, const double* B, int ldb,
                             double* C, int ldc);

@@ -65,8 +65,7 @@ constexpr uint32_t kFlowSpinLimit = 1u << 22;
 // against 2.21).
 constexpr int kNarrowGrid = 512;
 // From this many right-hand sides on the rows off the diagonal blocks of
-// kSplitRows rows are updated by the GEMM of k_trsv.hip, which reads T once
-// per 64 of them.
+// kSplitRows rows are updated by a GEMM, which reads T once per 64 of them.
 constexpr int kSplitRhs = 192, kSplitRows = 512;
 struct FlowArgs {
   const double* T;

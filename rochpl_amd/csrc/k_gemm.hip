@@ -370,7 +370,7 @@ __global__ __launch_bounds__(NT, 2) void dgemm_kernel(
 // The product in small tiles (gemm_tile.hpp; see pick_tile).  128 x 128 tiles
 // left most CUs idle (256 x 256, K = 256: 4 tiles) or computed 4 columns for
 // each wanted one (n = 32).
-template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN>
+template <typename V, bool BETA0, bool NEG, bool LOWER_A, int BM, int BN, bool TB>
 __global__ __launch_bounds__(kTileThreads) void tile_kernel(
     int M, int N, int K, const V* __restrict__ A, int lda,
     const V* __restrict__ B, int ldb, V* __restrict__ C, int ldc, int tiles_m,
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(kTileThreads) void tile_kernel(
   const int per  = gridDim.x / kXcds;
   const int tile = (blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
   if(tile >= tiles_m * tiles_n) return;
-  gemm_tile<V, BETA0, NEG, LOWER_A, BM, BN>(threadIdx.x, tile, true, M, N, K, A, lda, B,
+  gemm_tile<V, BETA0, NEG, LOWER_A, BM, BN, false, TB>(threadIdx.x, tile, true, M, N, K, A, lda, B,
                                             ldb, C, ldc, tiles_m, tiles_n, sh);
 }
 
@@ -409,14 +409,14 @@ Tile pick_tile(int m, int n) {
   return big >= kTileGrid / 2 && 16 * 4 * big <= 17 * tiles(64, 64) ? kTile128 : kTile64;
 }
 
-template <bool BETA0, bool NEG, bool LOWER_A, int BM, int BN, typename V>
+template <bool BETA0, bool NEG, bool LOWER_A, int BM, int BN, bool TB = false, typename V>
 hipError_t run_tile(hipStream_t s, int m, int n, int k, const V* A, int lda,
                     const V* B, int ldb, V* C, int ldc, Stamps st) {
   const int  tiles_m = (m + BM - 1) / BM, tiles_n = (n + BN - 1) / BN;
   const long T    = static_cast<long>(tiles_m) * tiles_n;
   const long grid = (T + kXcds - 1) / kXcds * kXcds;
   if(grid > 0x7fffffffL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((tile_kernel<V, BETA0, NEG, LOWER_A, BM, BN>),
+  hipLaunchKernelGGL((tile_kernel<V, BETA0, NEG, LOWER_A, BM, BN, TB>),
                      dim3(static_cast<unsigned>(grid)), dim3(kTileThreads), 0, s, m, n, k, A, lda,
                      B, ldb, C, ldc, tiles_m, tiles_n, st);
   return hipGetLastError();
@@ -444,6 +444,12 @@ hipError_t run(hipStream_t s, int m, int n, int k, const V* A, int lda,
         case kTile64: return run_tile<BETA0, NEG, LOWER_A, 64, 64>(s, m, n, k, A, lda, B, ldb, C, ldc, st);
         default: break;
       }
+  // C = -A B^T (the adjoint's gradA, bound by C's traffic and its MFMAs alike):
+  // N = 16384, K = 64 945 us with loads one by one, 749 with pairs
+  if constexpr(!TA && TB && BETA0 && NEG && KIND == 0)
+    if(pair_aligned(A) && lda % 2 == 0 && pair_aligned(B) && ldb % 2 == 0 && k > 0)
+      return run_tile<BETA0, NEG, LOWER_A, 64, 64, true>(s, m, n, k, A, lda, B, ldb, C, ldc,
+                                                         st);
   const dim3 g(static_cast<unsigned>(grid)), b(NT);
   if(va && vb)
     hipLaunchKernelGGL((dgemm_kernel<V, BETA0, NEG, LOWER_A, TA, TB, true, true, KIND>),

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(kLeafThreads) void panel_kernel(PkArgs a) {
 
   if(__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     return;
-  const int G = gridDim.x, b = blockIdx.x, t = threadIdx.x;
+  const int G = gridDim.x, b = blockIdx.x;
   unsigned  nbar   = 0;
   uint32_t  leaf_i = 0;
   for(int i = 0; i < a.nops; ++i) {
