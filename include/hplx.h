@@ -138,7 +138,7 @@ int         hplx_num_cus(hplx_ctx* ctx);
  * an odd leading dimension, runs as the sequence).  0: every panel as a
  * sequence of kernels, one per leaf, triangular solve and product of the
  * recursion.  2 (default): the persistent kernel for panels of at least
- * 65536 rows, the sequence below (where it is faster).  Pivots and factors
+ * 65536 rows, the sequence below.  Pivots and factors
  * are the same bit for bit in all three.  The environment variable
  * HPLX_PANEL_KERNEL=0|1|2 sets the default of new contexts. */
 #define HPLX_OPT_PANEL_KERNEL 2
@@ -299,7 +299,7 @@ int hplx_pdtrsv(hplx_ctx* ctx, int n, int nb, const double* A, int lda,
                 double* x);
 
 /* Device time in ms of the FP64 trailing-update GEMM kernels queued since
- * the last hplx_pdgesv started (HIP events around each launch), with the
+ * the last hplx_pdgesv started (times the kernels note as they start), with the
  * count of launches and their algorithmic flops. */
 int hplx_update_stats(hplx_ctx* ctx, double* gemm_ms, int* launches,
                       double* gemm_flops);
@@ -316,15 +316,15 @@ int hplx_update_timing(hplx_ctx* ctx, int kind, double* ms, int* launches,
 /* Timing of the row interchanges of the trailing columns (the gather /
  * scatter kernel of HPL_pdlaswp_end / HPL_dlaswp00N at P=1,
  * src/pauxil/HPL_dlaswp00N_device.cpp:22-112) in the last hplx_pdgesv /
- * hplx_pdgetrf: summed launch time (ms, HIP events), launches, and their
+ * hplx_pdgetrf: summed launch time (ms), launches, and their
  * algorithmic bytes (4 x 8 B per interchanged element: the pivot row read,
  * the U buffer written, the displaced top row read and written).  No
  * counterpart in the reference, which times none. */
 int hplx_swap_timing(hplx_ctx* ctx, double* ms, int* launches, double* bytes);
 
 /* Timing of the panel factorisations (HPL_pdfact, src/pfact/HPL_pdfact.cpp)
- * in the last hplx_pdgesv / hplx_pdgetrf: summed time (ms, HIP events
- * around each panel on the stream it runs on, beside the update with the
+ * in the last hplx_pdgesv / hplx_pdgetrf: summed time (ms,
+ * of each panel on the stream it runs on, beside the update with the
  * look-ahead), panels, and their algorithmic bytes (each m x jb panel read
  * and written once, 16 B per element).  No counterpart in the reference. */
 int hplx_panel_timing(hplx_ctx* ctx, double* ms, int* panels, double* bytes);
