@@ -1,6 +1,7 @@
 // Products of the solves: the GEMVs of the mixed-precision solves (rocblas_dgemv
 // at src/pgesv/HPL_pdtrsv_device.cpp:195-332), and the products with many
 // right-hand sides of the FP64 solves and the adjoint.
+#include <type_traits>
 #include "gemm_tile.hpp"
 #include "mxp.hpp"
 
@@ -20,8 +21,11 @@ __device__ inline V to_v(MT x) {
 // y[0:m] -= U[0:m, 0:kb] * xs[0:kb] in the vectors' type V (FP64, or FP32 in
 // the mixed-precision correction solves), U of element type MT (double, or
 // the FP32 / FP16 factors of the mixed forms).  Workgroup = 64 rows; wave w
-// takes a quarter of the columns; partial sums meet in LDS.  xback
-// (optional): workgroup 0 also copies xs[0:kb] there.
+// takes a quarter of the columns, 32 of their loads in flight at a time, since
+// the kernel waits for memory (on average over a solve of N = 16384, kb = 512 in
+// FP32 18.5 us with 4 in flight, 7.8 now; 32768, 1024 in FP16 34.2, 13.5), with
+// the sums in the order of the columns; partial sums meet in LDS.
+// xback (optional): workgroup 0 also copies xs[0:kb] there.
 template <typename MT, typename V>
 __global__ __launch_bounds__(256) void gemv_sub_kernel(
     int m, int kb, const MT* __restrict__ U, int ldu,
@@ -41,18 +45,20 @@ __global__ __launch_bounds__(256) void gemv_sub_kernel(
   V         acc = 0;
   if(row < m) {
     const MT* u = U + row + static_cast<size_t>(c0) * ldu;
-    int c = c0;
-    for(; c + 4 <= c1; c += 4) {
-      const V u0 = to_v<V>(u[0]);
-      const V u1 = to_v<V>(u[static_cast<size_t>(ldu)]);
-      const V u2 = to_v<V>(u[2 * static_cast<size_t>(ldu)]);
-      const V u3 = to_v<V>(u[3 * static_cast<size_t>(ldu)]);
-      acc = fma(u0, sxs[c], acc);
-      acc = fma(u1, sxs[c + 1], acc);
-      acc = fma(u2, sxs[c + 2], acc);
-      acc = fma(u3, sxs[c + 3], acc);
-      u += 4 * static_cast<size_t>(ldu);
-    }
+    int       c = c0;
+    auto      run = [&](auto width) {
+      constexpr int W = decltype(width)::value;
+      for(; c + W <= c1; c += W) {
+        MT v[W];
+#pragma unroll
+        for(int j = 0; j < W; ++j) v[j] = u[static_cast<size_t>(j) * ldu];
+#pragma unroll
+        for(int j = 0; j < W; ++j) acc = fma(to_v<V>(v[j]), sxs[c + j], acc);
+        u += W * static_cast<size_t>(ldu);
+      }
+    };
+    run(std::integral_constant<int, 32>());
+    run(std::integral_constant<int, 4>());
     for(; c < c1; ++c) {
       acc = fma(to_v<V>(u[0]), sxs[c], acc);
       u += ldu;
