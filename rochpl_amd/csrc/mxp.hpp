@@ -63,10 +63,6 @@ hipError_t launch_copy_block(hipStream_t s, int m, int n, const __half* A,
                              int lda, float* B, int ldb);
 hipError_t launch_copy_block(hipStream_t s, int m, int n, const float* A,
                              int lda, __half* B, int ldb);
-hipError_t launch_copy_block(hipStream_t s, int m, int n, const double* A,
-                             int lda, float* B, int ldb);
-hipError_t launch_copy_block(hipStream_t s, int m, int n, const double* A,
-                             int lda, __half* B, int ldb);
 
 // ---- solves with low-precision factors and FP64 vectors
 // The interchanges y[i] <-> y[ipiv[i]] of one panel (i = k0 .. k0+jb-1 in
