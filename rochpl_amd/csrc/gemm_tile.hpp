@@ -121,7 +121,8 @@ struct TileShared {
   alignas(16) V b[kTileK * (BN + 2)];
 };
 
-// Tile `tile` (rows first within groups of kGroupM tile rows) of C (M x N) =
+// Tile `tile` (rows first within groups of kGroupM tile rows; of a LOWER_A product,
+// whose row tiles have K bounds of their own, the longest first) of C (M x N) =
 // beta C + alpha op(A) op(B), BM x BN on 4 waves in 2 x 2 (t: the thread among
 // them), for 16-byte aligned operands with even leading dimensions (TA / TB:
 // stored transposed): K in 32-deep stages through one LDS buffer (the next stage's
@@ -142,13 +143,19 @@ __device__ __forceinline__ void gemm_tile(int t, int tile, bool live, int M, int
                                           int tiles_n, TileShared<V, BM, BN>& sh) {
   constexpr int BKS = kTileK, LA = BM + 2, LB = BN + 2;
   constexpr int TM = BM / 32, TN = BN / 32;
-  const int width  = kGroupM * tiles_n;
-  const int group  = tile / width;
-  const int firstm = group * kGroupM;
-  const int gsz    = min(tiles_m - firstm, kGroupM);
-  const int within = tile - group * width;
-  const int m0     = (firstm + within % gsz) * BM;
-  const int n0     = within / gsz * BN;
+  int m0, n0;
+  if constexpr(LOWER_A) {
+    m0 = (tiles_m - 1 - tile / tiles_n) * BM;
+    n0 = tile % tiles_n * BN;
+  } else {
+    const int width  = kGroupM * tiles_n;
+    const int group  = tile / width;
+    const int firstm = group * kGroupM;
+    const int gsz    = min(tiles_m - firstm, kGroupM);
+    const int within = tile - group * width;
+    m0 = (firstm + within % gsz) * BM;
+    n0 = within / gsz * BN;
+  }
   const int kend   = LOWER_A ? min(K, m0 + BM) : K;
 
   const int lane = t & 63, wave = t >> 6;
