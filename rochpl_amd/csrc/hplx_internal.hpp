@@ -421,6 +421,7 @@ struct FlowScratch {
   size_t              work_doubles;
   int*                perm;   // kFlowPerm
   int*                flags;  // kFlowFlags
+  int                 raised = 0;  // what the flags start as (1: as if all were raised)
 };
 
 // The back-solve U x = b (HPL_pdtrsv), x in place.

@@ -29,8 +29,10 @@
 // through memory and no cache write-back or invalidation.  The blocks
 // further on are not in a hurry: they poll the flag at leisure and then read
 // x_i through their L2 (U of N = 16384 with 64 right-hand sides in 64-row
-// blocks: 2243 us with all of them polling the values, 1220 us so).  Nothing
-// outlives the call, so the launches can be captured and replayed.
+// blocks: 2243 us with all of them polling the values, 1220 us so).  The flag
+// is a hint only: nothing orders it with what a block's L2 may hold, so what
+// they read is checked for that NaN like a poll, and polled for if it is there.
+// Nothing outlives the call, so the launches can be captured and replayed.
 //
 // Bound by latency: a step of the chain is two substitutions of 64 rows (each
 // 64 dependent FMAs on broadcast values), two products of 64 columns and that
@@ -93,15 +95,24 @@ struct FlowArgs {
 // would be published are replaced by the plain quiet NaN).
 constexpr unsigned long long kEmpty = 0x7ff8b10cffffb10cull;
 
+// None of a wave's values is the filling.
+template <int W>
+__device__ __forceinline__ bool all_there(const unsigned long long (&v)[W]) {
+  bool in = true;
+#pragma unroll
+  for(int q = 0; q < W; ++q) in = in && v[q] != kEmpty;
+  return __all(in);
+}
+
 // Also copies the first `rows` rows of B's nrhs columns to top, if it is not
 // null.
 __global__ __launch_bounds__(256) void fill_kernel(unsigned long long* p, int n,
-                                                   int* flags, int nf,
+                                                   int* flags, int nf, int raised,
                                                    const double* B, int ldb, int nrhs,
                                                    double* top, int rows) {
   const int i0 = blockIdx.x * 256 + threadIdx.x;
   for(int i = i0; i < n; i += gridDim.x * 256) p[i] = kEmpty;
-  if(i0 < nf) flags[i0] = 0;
+  if(i0 < nf) flags[i0] = raised;
   if(top)
     for(int i = i0; i < rows * nrhs; i += gridDim.x * 256)
       top[i] = B[i % rows + static_cast<size_t>(i / rows) * ldb];
@@ -363,19 +374,9 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
                                        (R * kFH) + kFH * wave + lane;
     unsigned long long  xv[W];
     if(wave < R) {
+      bool in = false;
       if(diag && j + kNext >= i) {
         __builtin_amdgcn_s_setprio(3);
-        for(;;) {
-          bool in = true;
-#pragma unroll
-          for(int q = 0; q < W; ++q)
-            xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-          for(int q = 0; q < W; ++q) in = in && xv[q] != kEmpty;
-          if(__all(in) || dead) break;
-          dead = ++spins > kFlowSpinLimit;
-        }
       } else {
         const int* flag = a.flags + j * a.ns + sl;
         while(!dead && !__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
@@ -384,7 +385,18 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         }
         asm volatile("" : : : "memory");  // the values are read after the flag
 #pragma unroll
-        for(int q = 0; q < W; ++q) xv[q] = xj[8 * kFH * q];
+        for(int q = 0; q < W; ++q)
+          xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+        in = all_there(xv);
+      }
+      while(!in && !dead) {
+#pragma unroll
+        for(int q = 0; q < W; ++q)
+          xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+        in = all_there(xv);
+        if(!in) dead = ++spins > kFlowSpinLimit;
       }
       if(dead) {
 #pragma unroll
@@ -522,8 +534,8 @@ struct Flow {
     if(np * bpp > blocks()) return hipErrorInvalidValue;
     const int n = static_cast<int>(x_panel(bpp)) * np;
     hipLaunchKernelGGL(fill_kernel, dim3(n < 256 * 1024 ? (n + 255) / 256 : 1024),
-                       dim3(256), 0, s, w.x, n, w.flags, np * bpp * slices(), B, ldb,
-                       nrhs, top, top_rows);
+                       dim3(256), 0, s, w.x, n, w.flags, np * bpp * slices(), w.raised, B,
+                       ldb, nrhs, top, top_rows);
     return hipGetLastError();
   }
 
