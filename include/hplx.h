@@ -202,7 +202,12 @@ int hplx_pdgetrf(hplx_ctx* ctx, const hplx_palg* palg, hplx_pmat* mat);
  * HPL_pdgesv carries b through the factorisation (HPL's L is left unpivoted
  * by later panels).  No allocation: the exchange buffers and
  * partial sums live in the context's own panel buffers, so calls on one
- * context must not overlap. */
+ * context must not overlap.  The solve's kernels wait for each other on the
+ * device (so do the back-solves of hplx_pdgesv and hplx_pdtrsv, and
+ * hplx_pdgesv_adjoint); if other work holds the device for seconds such a wait
+ * gives up, and the call returns HPLX_ERR_HIP with NaNs in B.  The environment
+ * variable HPLX_SOLVE_POLLS sets the failed polls of one wait after which it
+ * does in new contexts (default 4194304). */
 int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
                  double* B, int ldb);
 
@@ -218,7 +223,8 @@ int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
  * one device (on different streams, or from several threads) race.
  * mat->nb above 1024 (what the scratch is laid out for) returns
  * HPLX_ERR_UNSUPPORTED; bad arguments HPLX_ERR_INVALID; a launch failure
- * HPLX_ERR_HIP (no error string: there is no context to hold one). */
+ * HPLX_ERR_HIP (no error string: there is no context to hold one).  A wait that
+ * gives up on the device (see hplx_pdgetrs) shows only as NaNs in B. */
 int hplx_pdgetrs_noalloc(const hplx_pmat* mat, int trans, int nrhs, double* B,
                          int ldb, void* stream);
 

@@ -95,7 +95,20 @@ namespace {
 hplx::FlowScratch flow_scratch(const Ctx& c) {
   return {reinterpret_cast<unsigned long long*>(c.Linv2), c.Linv,
           static_cast<size_t>(hplx::kMaxNB) * hplx::kMaxNB, c.flow_perm,
-          c.flow_flags};
+          c.flow_flags, 0, c.flow_err, c.flow_polls};
+}
+
+// Around a solve: no wait has given up yet; and once the stream has got there,
+// whether one has.
+hplx::FlowScratch begin_solve(Ctx& c) {
+  *static_cast<volatile int*>(c.flow_err) = 0;
+  return flow_scratch(c);
+}
+int end_solve(Ctx& c) {
+  HIPCHK(c, hipStreamSynchronize(c.stream));
+  if(*static_cast<volatile int*>(c.flow_err))
+    return fail(c, HPLX_ERR_HIP, "a wait of the triangular solve timed out");
+  return HPLX_SUCCESS;
 }
 
 }  // namespace
@@ -183,6 +196,7 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   size_t total      = off_pbar + 256;
   auto undo = [&](int code) {
     if(c.small_base) (void)hipFree(c.small_base);
+    if(c.flow_err) (void)hipHostFree(c.flow_err);
     if(c.ustream) (void)hipStreamDestroy(c.ustream);
     if(c.pstream) (void)hipStreamDestroy(c.pstream);
     (void)hipStreamDestroy(c.own_stream);
@@ -192,7 +206,10 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
   if(hipStreamCreateWithFlags(&c.ustream, hipStreamNonBlocking) != hipSuccess ||
      hipStreamCreateWithFlags(&c.pstream, hipStreamNonBlocking) != hipSuccess)
     return undo(HPLX_ERR_HIP);
-  if(hipMalloc(&c.small_base, total) != hipSuccess) return undo(HPLX_ERR_ALLOC);
+  if(hipMalloc(&c.small_base, total) != hipSuccess ||
+     hipHostMalloc(reinterpret_cast<void**>(&c.flow_err), sizeof(int), hipHostMallocDefault) !=
+         hipSuccess)
+    return undo(HPLX_ERR_ALLOC);
   char* b   = static_cast<char*>(c.small_base);
   c.Linv    = reinterpret_cast<double*>(b);
   c.permU   = reinterpret_cast<int*>(b + off_perm);
@@ -218,6 +235,9 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
     const int v = std::atoi(pk);
     c.panel_kernel = v >= 0 && v <= 2 ? v : c.panel_kernel;
   }
+  c.flow_polls = hplx::kFlowPolls;
+  if(const char* sp = std::getenv("HPLX_SOLVE_POLLS"))
+    c.flow_polls = static_cast<uint32_t>(std::strtoul(sp, nullptr, 10));
   if(cu_sets(c, census) != HPLX_SUCCESS) return undo(HPLX_ERR_HIP);
   *out = ctx;
   return HPLX_SUCCESS;
@@ -234,6 +254,7 @@ int hplx_ctx_destroy(hplx_ctx* ctx) {
   for(hipEvent_t e : c.ev_sync) (void)hipEventDestroy(e);
   if(c.stamps) (void)hipFree(c.stamps);
   if(c.small_base) (void)hipFree(c.small_base);
+  if(c.flow_err) (void)hipHostFree(c.flow_err);
   if(c.ustream) (void)hipStreamDestroy(c.ustream);
   if(c.pstream) (void)hipStreamDestroy(c.pstream);
   if(c.own_stream) (void)hipStreamDestroy(c.own_stream);
@@ -703,9 +724,8 @@ int hplx_pdgesv(hplx_ctx* ctx, const hplx_palg* palg, hplx_pmat* mat) {
   HIPCHK(c, hipMemcpyAsync(mat->X, mat->A + static_cast<size_t>(N) * mat->ld,
                            static_cast<size_t>(N) * sizeof(double),
                            hipMemcpyDeviceToDevice, s));
-  HIPCHK(c, hplx::launch_trsv(s, N, mat->A, mat->ld, mat->X, flow_scratch(c)));
-  HIPCHK(c, hipStreamSynchronize(s));
-  return HPLX_SUCCESS;
+  HIPCHK(c, hplx::launch_trsv(s, N, mat->A, mat->ld, mat->X, begin_solve(c)));
+  return end_solve(c);
 }
 
 int hplx_pdgetrf(hplx_ctx* ctx, const hplx_palg* palg, hplx_pmat* mat) {
@@ -724,9 +744,8 @@ int hplx_pdgetrs(hplx_ctx* ctx, const hplx_pmat* mat, int trans, int nrhs,
     return fail(c, HPLX_ERR_INVALID, "pdgetrs: bad arguments");
   if(nrhs == 0) return HPLX_SUCCESS;
   HIPCHK(c, hplx::getrs_enqueue(c.stream, mat->A, mat->n, mat->nb, mat->ld,
-                                mat->ipiv, trans, nrhs, B, ldb, flow_scratch(c)));
-  HIPCHK(c, hipStreamSynchronize(c.stream));
-  return HPLX_SUCCESS;
+                                mat->ipiv, trans, nrhs, B, ldb, begin_solve(c)));
+  return end_solve(c);
 }
 
 int hplx_pdgesv_adjoint(hplx_ctx* ctx, const hplx_pmat* mat, int nrhs,
@@ -891,9 +910,8 @@ int hplx_pdtrsv(hplx_ctx* ctx, int n, int nb, const double* A, int lda,
   HIPCHK(c, hipMemcpyAsync(x, A + static_cast<size_t>(n) * lda,
                            static_cast<size_t>(n) * sizeof(double),
                            hipMemcpyDeviceToDevice, c.stream));
-  HIPCHK(c, hplx::launch_trsv(c.stream, n, A, lda, x, flow_scratch(c)));
-  HIPCHK(c, hipStreamSynchronize(c.stream));
-  return HPLX_SUCCESS;
+  HIPCHK(c, hplx::launch_trsv(c.stream, n, A, lda, x, begin_solve(c)));
+  return end_solve(c);
 }
 
 int hplx_update_timing(hplx_ctx* ctx, int kind, double* ms, int* launches,

@@ -112,6 +112,8 @@ struct Ctx {
   int*      permU2     = nullptr;
   int*      flow_perm  = nullptr;    // kFlowPerm
   int*      flow_flags = nullptr;    // kFlowFlags
+  int*      flow_err   = nullptr;    // pinned host memory (FlowScratch::err)
+  uint32_t  flow_polls = 0;
   int*      claim      = nullptr;    // 2 sets of kClaimInts update-claim counters
   int*      stop       = nullptr;    // 2 flags: claims of update k stop
   unsigned long long* vacate = nullptr;  // kVacateSets x 8 words (see cu_sets)
@@ -415,6 +417,7 @@ constexpr int    kFlowCols   = 1024;  // right-hand sides at once
 constexpr int    kFlowFlags  = kMaxNB * kFlowCols / (128 * 4);
 constexpr size_t kFlowX      = static_cast<size_t>(kMaxNB) * kFlowCols;
 constexpr int    kFlowPerm   = 2 * 128 * kFlowBlocks;  // ints
+constexpr uint32_t kFlowPolls = 1u << 22;  // failed polls of one wait: a few seconds
 struct FlowScratch {
   unsigned long long* x;     // kFlowX
   double*             work;  // work_doubles
@@ -422,6 +425,8 @@ struct FlowScratch {
   int*                perm;   // kFlowPerm
   int*                flags;  // kFlowFlags
   int                 raised = 0;  // what the flags start as (1: as if all were raised)
+  int*                err    = nullptr;  // host memory: set when a wait gives up (null: nowhere)
+  uint32_t            polls  = kFlowPolls;  // after more failed polls than these
 };
 
 // The back-solve U x = b (HPL_pdtrsv), x in place.

@@ -19,8 +19,8 @@
 // Progress.  A workgroup waits only for blocks of smaller index, and the
 // dispatcher hands out workgroups in index order on every XCD, so the
 // unfinished workgroup of the smallest index never waits: the grid need not
-// be resident at once.  The waits are bounded all the same; past the limit a
-// workgroup goes on with NaNs.
+// be resident at once.  The waits are bounded all the same: past the limit of
+// one wait a workgroup raises *err and goes on with NaNs.
 //
 // x_i travels through an exchange buffer that the call fills with a NaN of a
 // payload of its own first (fill_kernel), and then a flag is raised.  The
@@ -60,7 +60,6 @@ constexpr int kFB  = 128;  // rows of a block
 constexpr int kFH  = 64;   // and of its halves
 constexpr int kFLd = 66;   // LDS pitch of a right-hand side of a half
 constexpr int kNext = 1;   // blocks ahead in the chain that poll the values
-constexpr uint32_t kFlowSpinLimit = 1u << 22;
 // Narrow slices (4 right-hand sides) while at most this many workgroups come
 // of it, 2 per CU: a step takes 4.6 instead of 8.7 us, but every slice reads
 // all of T (N = 16384: 16 right-hand sides 2.04 against 2.21 ms, 24 2.31
@@ -80,6 +79,8 @@ struct FlowArgs {
   int           ns;      // slices of 16 right-hand sides
   unsigned long long* x;      // nd x ns blocks of 2 halves of 16 x 64 values
   int*                flags;  // nd x ns
+  int*                err;    // FlowScratch's
+  uint32_t            polls;
   // The interchanges of a panel of L, applied as B is loaded (null: none): perm
   // as launch_pipid composes it, relative to d0; top: the panel's rows of B as
   // they were before it (leading dimension d1 - d0), whose places in B the
@@ -363,8 +364,7 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     const int cj = half_row(0);
     load_block<TRANS>(a.T, a.ldt, r0, nr, cj, min(kFH, a.d1 - cj), tn);
   }
-  uint32_t spins = 0;
-  bool     dead  = false;
+  bool dead = false;
   for(int st = 0; st < steps; ++st) {
 #pragma unroll
     for(int s = 0; s < 16; ++s) tv[s] = tn[s];
@@ -374,13 +374,14 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
                                        (R * kFH) + kFH * wave + lane;
     unsigned long long  xv[W];
     if(wave < R) {
-      bool in = false;
+      bool     in    = false;
+      uint32_t polls = 0;
       if(diag && j + kNext >= i) {
         __builtin_amdgcn_s_setprio(3);
       } else {
         const int* flag = a.flags + j * a.ns + sl;
         while(!dead && !__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-          dead = ++spins > kFlowSpinLimit;
+          dead = ++polls > a.polls;
           __builtin_amdgcn_s_sleep(8);
         }
         asm volatile("" : : : "memory");  // the values are read after the flag
@@ -388,7 +389,8 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         for(int q = 0; q < W; ++q)
           xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-        in = all_there(xv);
+        in    = all_there(xv);
+        polls = 0;
       }
       while(!in && !dead) {
 #pragma unroll
@@ -396,9 +398,11 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
           xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_AGENT);
         in = all_there(xv);
-        if(!in) dead = ++spins > kFlowSpinLimit;
+        if(!in) dead = ++polls > a.polls;
       }
       if(dead) {
+        if(a.err && lane == 0)
+          __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 #pragma unroll
         for(int q = 0; q < W; ++q) xv[q] = 0x7ff8000000000000ull;
       }
@@ -594,6 +598,8 @@ struct Flow {
     a.ldt   = ldt;
     a.x     = w.x + x_panel(block);
     a.flags = w.flags + block * slices();
+    a.err   = w.err;
+    a.polls = w.polls;
     a.B     = B;
     a.ldb   = ldb;
     a.nrhs  = nrhs;
