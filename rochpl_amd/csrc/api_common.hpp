@@ -50,21 +50,30 @@ inline int sync_event(Ctx& c, size_t i, hipEvent_t* e) {
   return HPLX_SUCCESS;
 }
 
-// Room for the times of a factorisation of `panels` panels.
-inline int reserve_stamps(Ctx& c, int panels) {
-  if(panels <= c.stamp_panels) return HPLX_SUCCESS;
-  if(c.stamps) (void)hipFree(c.stamps);
-  c.stamps       = nullptr;
-  c.stamp_panels = 0;
-  HIPCHK(c, hipMalloc(&c.stamps, sizeof(long long) * 2 * kStampPairs * panels));
-  c.stamp_panels = panels;
+// Room for the times of a factorisation of `panels` panels: of its updates
+// (buf 0), or of its interchanges and panels (buf 1).  Nothing is counted in a
+// buffer from here on, whether or not it is replaced.
+inline int reserve_stamps(Ctx& c, int buf, int panels) {
+  if(buf == 0) {
+    c.ev_pairs   = 0;
+    c.gemm_flops = 0.0;
+  } else {
+    c.swap_pairs = c.panel_pairs = 0;
+    c.swap_bytes = c.panel_bytes = 0.0;
+  }
+  StampBuf& b = c.stamps[buf];
+  if(panels <= b.panels) return HPLX_SUCCESS;
+  if(b.t) (void)hipFree(b.t);
+  b = StampBuf();
+  HIPCHK(c, hipMalloc(&b.t, sizeof(long long) * 2 * kStampPairs * panels));
+  b.panels = panels;
   return HPLX_SUCCESS;
 }
 
 // Pair i of the updates (kind 0), the interchanges (1) or the panels (2).
 inline long long* stamp_at(const Ctx& c, int kind, int i) {
-  constexpr int first[3] = {0, 3, 5};
-  return c.stamps + 2 * (static_cast<size_t>(first[kind]) * c.stamp_panels + i);
+  const StampBuf& b = c.stamps[kind > 0];
+  return b.t + 2 * (static_cast<size_t>(kind == 2 ? 2 : 0) * b.panels + i);
 }
 
 // The durations (ms) of the first n pairs of a kind.

@@ -252,7 +252,8 @@ int hplx_ctx_destroy(hplx_ctx* ctx) {
   if(c.pstream) (void)hipStreamSynchronize(c.pstream);
   for(hipEvent_t e : c.ev_prog) (void)hipEventDestroy(e);
   for(hipEvent_t e : c.ev_sync) (void)hipEventDestroy(e);
-  if(c.stamps) (void)hipFree(c.stamps);
+  for(const hplx::StampBuf& b : c.stamps)
+    if(b.t) (void)hipFree(b.t);
   if(c.small_base) (void)hipFree(c.small_base);
   if(c.flow_err) (void)hipHostFree(c.flow_err);
   if(c.ustream) (void)hipStreamDestroy(c.ustream);
@@ -556,13 +557,8 @@ static int factor_loop(Ctx& c, const hplx_palg* palg, hplx_pmat* mat,
   Fp64Loop L{c, mat, static_cast<hplx::MatWs*>(mat->ws), mat->A, N, nb, lda,
              hplx::panel_algo(*palg)};
   const int npanels = (N + nb - 1) / nb;
-  if((r = hplx::reserve_stamps(c, npanels))) return r;
-  c.ev_pairs   = 0;
-  c.gemm_flops = 0.0;
-  c.swap_pairs = 0;
-  c.swap_bytes = 0.0;
-  c.panel_pairs = 0;
-  c.panel_bytes = 0.0;
+  if((r = hplx::reserve_stamps(c, 0, npanels)) || (r = hplx::reserve_stamps(c, 1, npanels)))
+    return r;
   c.ev_kind.assign(3 * npanels, 0);
   c.ev_flops.assign(3 * npanels, 0.0);
   c.splits.clear();

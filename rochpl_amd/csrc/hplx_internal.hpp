@@ -83,9 +83,15 @@ struct Stamps {
   long long* a = nullptr;
   long long* b = nullptr;
 };
-// Pairs of times a panel step may take: 3 updates (the next panel's columns,
-// claimed, resumed), 2 interchanges, 1 panel.
-constexpr int kStampPairs = 6;
+// Pairs of times in device memory (stamp.hpp), with room for those of `panels`
+// panels.
+struct StampBuf {
+  long long* t      = nullptr;
+  int        panels = 0;
+};
+// Pairs a panel step may take: 3 updates (the next panel's columns, claimed,
+// resumed); 2 interchanges and 1 panel.
+constexpr int kStampPairs = 3;
 
 // Per-context device state.  The small workspace (candidate slots, barrier
 // counter, flags, L11 inverse, composed pivots) lives with the context; the
@@ -157,11 +163,10 @@ struct Ctx {
   // counterpart of the reference's HPL_PROGRESS_REPORT build option)
   int                     progress_every = 0;
   std::vector<hipEvent_t> ev_prog;
-  // Timing of the last solve: pairs of times in device memory (stamp.hpp), for
-  // kStampPairs pairs per panel: first those of the trailing updates, then of
-  // the interchanges, then of the panels (stamp_at).
-  long long* stamps       = nullptr;
-  int        stamp_panels = 0;  // panels they have room for
+  // Timing of the last solve, kStampPairs pairs per panel each: the trailing
+  // updates', and in a buffer that the mixed-precision loop leaves alone the
+  // FP64 loop's interchanges', then its panels' (stamp_at).
+  StampBuf stamps[2];
   // the trailing-update GEMM launches: one pair per launch, its kind (1: a
   // whole update in one launch, 2: the claimed part of a split update, 3: its
   // resume part) and its flops (for kinds 2 and 3 filled from the claim log

@@ -245,9 +245,7 @@ int factor_loop(Ctx& c, const hplx_palg* palg, const hplx_mxp_opts* o,
   MxpLoop<S> L{c, palg, o, mat, ws, static_cast<S*>(mat->A), N, nb, lda};
 
   const int npanels = (N + nb - 1) / nb;
-  if(const int e = hplx::reserve_stamps(c, npanels)) return e;
-  c.ev_pairs   = 0;
-  c.gemm_flops = 0.0;
+  if(const int e = hplx::reserve_stamps(c, 0, npanels)) return e;
   c.ev_kind.assign(3 * npanels, 1);
   c.ev_flops.assign(3 * npanels, 0.0);
   c.splits.clear();
