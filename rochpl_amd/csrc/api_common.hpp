@@ -76,15 +76,17 @@ inline long long* stamp_at(const Ctx& c, int kind, int i) {
   return b.t + 2 * (static_cast<size_t>(kind == 2 ? 2 : 0) * b.panels + i);
 }
 
-// The durations (ms) of the first n pairs of a kind.
+// The durations (ms) of the first n pairs of a kind, read on the context's own
+// stream (the null stream would wait for every other blocking stream).
 inline int stamp_times(Ctx& c, int kind, int n, std::vector<double>* ms) {
   ms->assign(n, 0.0);
   if(n == 0) return HPLX_SUCCESS;
   int khz = 0;
   HIPCHK(c, hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device));
   std::vector<long long> t(2 * static_cast<size_t>(n));
-  HIPCHK(c, hipMemcpy(t.data(), stamp_at(c, kind, 0), sizeof(long long) * t.size(),
-                      hipMemcpyDeviceToHost));
+  HIPCHK(c, hipMemcpyAsync(t.data(), stamp_at(c, kind, 0), sizeof(long long) * t.size(),
+                           hipMemcpyDeviceToHost, c.stream));
+  HIPCHK(c, hipStreamSynchronize(c.stream));
   for(int i = 0; i < n; ++i)
     (*ms)[i] = static_cast<double>(t[2 * i + 1] - t[2 * i]) / khz;
   return HPLX_SUCCESS;

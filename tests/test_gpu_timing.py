@@ -1,4 +1,7 @@
-"""The times of the last FP64 solve outlive a mixed-precision solve."""
+"""The times of the last FP64 solve outlive a mixed-precision solve, and reading
+them touches no other stream."""
+import ctypes
+
 import pytest
 
 import rochpl_amd as rp
@@ -25,3 +28,31 @@ def test_fp64_times_outlive_a_mixed_solve(ctx):
         finally:
             c.pmat_free(mat)
             c.mxp_free(mx)
+
+
+def test_reading_times_does_not_wait_for_other_streams(ctx):
+    """The queries work on the context's stream alone: copies that take a tenth
+    of a second on another stream are still under way when they return."""
+    print("[gpu-case] timing queries beside copies on another stream", flush=True)
+    rp.lib()
+    hip, vp, gib = ctypes.CDLL("libamdhip64.so.7"), ctypes.c_void_p, 1 << 30
+    st = vp()
+    with rp.Context(0) as c:
+        mat, d = c.pmat_alloc(500, 100), c.alloc(2 * gib)
+        assert hip.hipStreamCreate(ctypes.byref(st)) == 0
+        try:
+            c.pdrandmat(500, 501, 100, mat.A, mat.ld)
+            assert c.pdgesv(rp.palg_default(), mat) == 0
+            for query in (c.swap_timing, c.panel_timing, c.update_stats,
+                          lambda: c.update_timing(1)):
+                want = query()
+                for _ in range(200):
+                    assert hip.hipMemcpyAsync(vp(d.ptr), vp(d.ptr + gib), ctypes.c_size_t(gib),
+                                              3, st) == 0
+                got, busy = query(), hip.hipStreamQuery(st)
+                assert hip.hipStreamSynchronize(st) == 0
+                assert busy == 600 and got == want  # hipErrorNotReady
+        finally:
+            hip.hipStreamDestroy(st)
+            d.free()
+            c.pmat_free(mat)
