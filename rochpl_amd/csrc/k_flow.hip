@@ -663,6 +663,9 @@ hipError_t launch_trsv(hipStream_t s, int n, const double* A, int lda, double* x
 static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
                                int lda, const int* ipiv, int trans, int nrhs,
                                double* B, int ldb, const FlowScratch& w) {
+  if(N <= 0) return hipSuccess;
+  if(nb > N) nb = N;  // one panel: any wider one is the same
+  if(nb < 1 || nb > kMaxNB) return hipErrorInvalidValue;
   Flow f{s, A, lda, B, ldb, nrhs, N, w};
   const int np  = (N + nb - 1) / nb;
   const int bpp = (nb + kFB - 1) / kFB;
@@ -678,7 +681,7 @@ static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
   auto prepare = [&](int p0) -> hipError_t {
     const int p1 = p0 + pc < np ? p0 + pc : np;
     HCHK(f.prepare(p1 - p0, bpp, fused && !trans && p0 == 0 ? w.work : nullptr,
-                   nb < N ? nb : N));
+                   nb));
     return launch_pipid_panels(s, p1 - p0, nb, N - p0 * nb, ipiv + p0 * nb,
                                p0 * nb, w.perm);
   };
