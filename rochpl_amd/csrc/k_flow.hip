@@ -473,6 +473,13 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
 #pragma unroll
           for(int s = 0; s < 4; ++s) v[s] = u[s];
       }
+      // past the block's rows nothing, whatever infinite values made of their
+      // zeros: the rows further on multiply them by zeros of T
+#pragma unroll
+      for(int s = 0; s < 4; ++s) {
+        const int q = BACK ? kFH - 1 - (16 * s + m) : 16 * s + m;
+        v[s]        = q < left ? v[s] : 0.0;
+      }
       unsigned long long* xi =
           a.x + (static_cast<size_t>(2 * i + h) * a.ns + sl) * (R * kFH) + c * kFH;
 #pragma unroll

@@ -68,3 +68,38 @@ def test_no_rows(ctx):
                                          ctypes.c_void_p(mat.X), 8) == rp.HPLX_SUCCESS
     finally:
         ctx.pmat_free(mat)
+
+
+def upload(mat, A):
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    full = np.zeros((mat.ld, A.shape[1]), order="F")
+    full[:A.shape[0]] = A
+    assert hip.hipMemcpy(ctypes.c_void_p(mat.A), full.ctypes.data_as(ctypes.c_void_p),
+                         ctypes.c_size_t(full.nbytes), 1) == 0
+
+
+@pytest.mark.parametrize("nrhs", [2, 40, 200])
+@pytest.mark.parametrize("n,nb", [(90, 30), (250, 100), (500, 200), (129, 65), (700, 257)])
+def test_infinities_spread_as_in_substitution(ctx, n, nb, nrhs):
+    """Factors whose entries off U's diagonal are all negative turn one infinite
+    right-hand side entry into +inf in every row, and nothing into NaN: the
+    padding of a ragged panel takes no part."""
+    print("[gpu-case] getrs inf n=%d nb=%d nrhs=%d" % (n, nb, nrhs), flush=True)
+    L = np.tril(np.full((n, n), -0.5 / n), -1) + np.eye(n)
+    U = np.triu(np.full((n, n), -0.5 / n), 1) + 4 * np.eye(n)
+    mat = ctx.pmat_alloc(n, nb)
+    try:
+        upload(mat, L @ U)
+        assert ctx.pdgetrf(rp.palg_default(), mat) == 0
+        assert np.array_equal(ctx.download_vec(mat.ipiv, n, np.int32), np.arange(n))
+        B = np.random.default_rng(3).standard_normal((n, nrhs))
+        for trans in (0, 1):
+            X = solve(ctx, mat, B, trans)
+            for k in (0, 10, nb - 1, nb, n - 1):
+                C = B.copy()
+                C[k, 0] = np.inf
+                Y = solve(ctx, mat, C, trans)
+                assert np.all(Y[:, 0] == np.inf), (trans, k)
+                assert np.array_equal(Y[:, 1:], X[:, 1:])
+    finally:
+        ctx.pmat_free(mat)
