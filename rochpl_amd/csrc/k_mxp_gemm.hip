@@ -104,13 +104,14 @@ __device__ inline uint8_t e4m3_bits(float x) {
 }
 
 // Largest e with amax * 2^e <= 448 (0 for an all-zero tile), clamped to the
-// range the scale arithmetic uses.
+// range the scale arithmetic uses (its lower end if amax is infinite).
 __device__ inline int fp8_tile_exp(float amax) {
   if(!(amax > 0.0f)) return 0;
-  int e = static_cast<int>(floorf(log2f(448.0f / amax)));
-  // guard the log2 rounding at exact powers
-  while(ldexpf(amax, e) > 448.0f) --e;
-  while(ldexpf(amax, e + 1) <= 448.0f) ++e;
+  if(amax > 3.40282347e38f) return -100;
+  // amax = f 2^x, 0.5 <= f < 1, against 448 = 0.875 2^9
+  int         x = 0;
+  const float f = frexpf(amax, &x);
+  const int   e = (f <= 0.875f ? 9 : 8) - x;
   return e < -100 ? -100 : (e > 100 ? 100 : e);
 }
 
