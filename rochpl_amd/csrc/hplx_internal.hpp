@@ -418,7 +418,7 @@ hipError_t launch_outer_neg(hipStream_t s, int K, int m, int n,
 // fewer only mean fewer splits) and the composed interchanges of the panels
 // prepared at once.  None needs to start in a particular state.
 constexpr int    kFlowBlocks = 128;
-constexpr int    kFlowCols   = 1024;  // right-hand sides at once
+constexpr int    kFlowCols   = 1024;  // right-hand sides at once (more below 8 blocks)
 constexpr int    kFlowFlags  = kMaxNB * kFlowCols / (128 * 4);
 constexpr size_t kFlowX      = static_cast<size_t>(kMaxNB) * kFlowCols;
 constexpr int    kFlowPerm   = 2 * 128 * kFlowBlocks;  // ints

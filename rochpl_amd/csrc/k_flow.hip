@@ -58,6 +58,7 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 constexpr int kFB  = 128;  // rows of a block
 constexpr int kFH  = 64;   // and of its halves
+constexpr int kXcds = 8;
 constexpr int kFLd = 66;   // LDS pitch of a right-hand side of a half
 constexpr int kNext = 1;   // blocks ahead in the chain that poll the values
 // Narrow slices (4 right-hand sides) while at most this many workgroups come
@@ -296,11 +297,19 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
   __shared__ double scale[2 * kFH];
   __shared__ int    rare;
   __shared__ int    from[kFB];  // where the block's rows of B come from
-  // the slices of a block on one XCD (they read the same rows of T), blocks
-  // in index order
-  const int per = 8 * a.ns, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
-  const int sl = br / 8, i = bg * 8 + (br & 7);
-  if(i >= a.nt) return;
+  // blocks in index order; the slices of a block on one XCD (they read the same
+  // rows of T), unless the blocks are too few for all XCDs (N = 100 with
+  // 1000 right-hand sides, one block: 144 us a call on one XCD, 44 spread)
+  int sl, i;
+  if(a.nt >= kXcds) {
+    const int per = kXcds * a.ns, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
+    sl = br / kXcds;
+    i  = bg * kXcds + br % kXcds;
+    if(i >= a.nt) return;
+  } else {
+    i  = blockIdx.x / a.ns;
+    sl = blockIdx.x - i * a.ns;
+  }
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int ac = P::col();  // this lane's right-hand side
@@ -515,7 +524,8 @@ struct FlowSwap {
   int           next_rows = 0;
 };
 
-// The solves of one call on a stream, for at most kFlowCols right-hand sides.
+// The solves of one call on a stream, for at most as many right-hand sides as
+// getrs_enqueue takes at once.
 struct Flow {
   hipStream_t        s;
   const double*      T;
@@ -617,7 +627,8 @@ struct Flow {
     a.o1    = o1;
     a.nd    = (d1 - d0 + kFB - 1) / kFB;
     a.nt    = a.nd + (o1 - o0 + kFB - 1) / kFB;
-    const long grid = (a.nt + 7L) / 8 * 8 * a.ns;
+    const long grid = static_cast<long>(a.nt < kXcds ? a.nt : (a.nt + kXcds - 1) / kXcds * kXcds) *
+                      a.ns;
     if(block + a.nd > blocks() || grid > 0x7fffffffL) return hipErrorInvalidValue;
     const dim3 g(static_cast<unsigned>(grid)), b(512);
     if(wide())
@@ -666,7 +677,7 @@ hipError_t launch_trsv(hipStream_t s, int n, const double* A, int lda, double* x
     if(e_ != hipSuccess) return e_; \
   } while(0)
 
-// At most kFlowCols right-hand sides.
+// At most as many right-hand sides as getrs_enqueue takes at once.
 static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
                                int lda, const int* ipiv, int trans, int nrhs,
                                double* B, int ldb, const FlowScratch& w) {
@@ -734,9 +745,12 @@ static hipError_t getrs_slices(hipStream_t s, const double* A, int N, int nb,
 hipError_t getrs_enqueue(hipStream_t s, const double* A, int N, int nb, int lda,
                          const int* ipiv, int trans, int nrhs, double* B,
                          int ldb, const FlowScratch& w) {
-  for(int c = 0; c < nrhs; c += kFlowCols)
-    HCHK(getrs_slices(s, A, N, nb, lda, ipiv, trans,
-                      nrhs - c < kFlowCols ? nrhs - c : kFlowCols,
+  // the right-hand sides whose blocks fit the exchange buffer, for a matrix of
+  // up to 8 blocks
+  const int rows = N < kMaxNB ? (N + kFB - 1) / kFB * kFB : kMaxNB;
+  const int cols = rows > 0 ? static_cast<int>(kFlowX / rows) / 16 * 16 : kFlowCols;
+  for(int c = 0; c < nrhs; c += cols)
+    HCHK(getrs_slices(s, A, N, nb, lda, ipiv, trans, nrhs - c < cols ? nrhs - c : cols,
                       B + static_cast<size_t>(c) * ldb, ldb, w));
   return hipSuccess;
 }

@@ -3,8 +3,10 @@ import ctypes
 
 import numpy as np
 import pytest
+import scipy.linalg as sl
 
 import rochpl_amd as rp
+from oracle import oracle as o
 
 pytestmark = pytest.mark.gpu
 
@@ -101,5 +103,26 @@ def test_infinities_spread_as_in_substitution(ctx, n, nb, nrhs):
                 Y = solve(ctx, mat, C, trans)
                 assert np.all(Y[:, 0] == np.inf), (trans, k)
                 assert np.array_equal(Y[:, 1:], X[:, 1:])
+    finally:
+        ctx.pmat_free(mat)
+
+
+@pytest.mark.parametrize("n,nb,cols", [(60, 60, 8192), (128, 50, 8192), (129, 129, 4096),
+                                       (300, 128, 2720), (700, 100, 1360), (1025, 300, 1024)])
+def test_passes_of_right_hand_sides(ctx, n, nb, cols):
+    """Up to the right-hand sides that one pass takes, and past them, against
+    LAPACK with the same matrix (diagonally dominant, so that n eps is kept)."""
+    A = o.matgen(n, n) + n * np.eye(n)
+    lu = sl.lu_factor(A)
+    mat = ctx.pmat_alloc(n, nb)
+    try:
+        ctx.pdrandmat(n, n, nb, mat.A, mat.ld, rp.HPL_ISEED, float(n))
+        assert ctx.pdgetrf(rp.palg_default(), mat) == 0
+        for nrhs in (cols - 15, cols, cols + 5):
+            print("[gpu-case] getrs n=%d nb=%d nrhs=%d" % (n, nb, nrhs), flush=True)
+            B = np.random.default_rng(nrhs).standard_normal((n, nrhs))
+            for trans in (0, 1):
+                X, R = solve(ctx, mat, B, trans), sl.lu_solve(lu, B, trans=trans)
+                assert np.abs(X - R).max() <= 4 * n * 2.0 ** -52 * np.abs(R).max()
     finally:
         ctx.pmat_free(mat)
