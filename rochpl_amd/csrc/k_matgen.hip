@@ -22,7 +22,6 @@ constexpr int kGenRows = 256;  // rows per block (one per thread)
 constexpr int kGenCols = 256;  // columns per block
 constexpr int kChkCols = 4096; // columns per partial-sum chunk (row pass)
 constexpr int kChkR    = 4;    // rows per thread of the whole check
-constexpr int kChkRows = 256 * kChkR;  // and of its workgroups
 constexpr int kChkSub  = 256;  // columns whose sums are kept in LDS at once
 constexpr int kChkStep = 8;    // columns between two reductions
 
@@ -110,7 +109,7 @@ __global__ __launch_bounds__(256) void check_rows_kernel(
 
 // The whole check in one pass: part_r and part_a as above for chunks of `cc`
 // columns, and part_c[rc*n + j] = sum_{i in row chunk rc} |a(i,j)|.  A thread
-// has kChkR rows; a column's sum over them goes to LDS, and every kChkStep
+// has R rows; a column's sum over them goes to LDS, and every kChkStep
 // columns each wave adds up its 64 lanes' (8 lanes to a column).
 //
 // Bound by the integer units: 3 products, 2 conversions and 6 other operations
@@ -118,15 +117,14 @@ __global__ __launch_bounds__(256) void check_rows_kernel(
 // is looked for only where it can be.  N = 20000 540 us in two passes, 335 in
 // this one.
 // EDGE: the step's rows may cross the diagonal or the last row.
-template <bool EDGE>
-__device__ __forceinline__ void check_step(int i, int j, uint64_t (&s)[kChkR],
-                                           double (&acc)[kChkR], double (&aabs)[kChkR],
-                                           double x, double shift, uint64_t colA,
-                                           uint64_t colC, const bool (&in)[kChkR],
+template <bool EDGE, int R>
+__device__ __forceinline__ void check_step(int i, int j, uint64_t (&s)[R], double (&acc)[R],
+                                           double (&aabs)[R], double x, double shift,
+                                           uint64_t colA, uint64_t colC, const bool (&in)[R],
                                            double& sum) {
   sum = 0.0;
 #pragma unroll
-  for(int q = 0; q < kChkR; ++q) {
+  for(int q = 0; q < R; ++q) {
     double v = lcg_value(s[q]);
     if(EDGE && i + 256 * q == j) v += shift;
     acc[q] = fma(v, x, acc[q]);
@@ -136,6 +134,7 @@ __device__ __forceinline__ void check_step(int i, int j, uint64_t (&s)[kChkR],
   }
 }
 
+template <int R>
 __global__ __launch_bounds__(256) void check_kernel(
     int n, int cc, uint64_t seed, double shift, const double* __restrict__ X,
     double* __restrict__ part_r, double* __restrict__ part_a,
@@ -145,13 +144,14 @@ __global__ __launch_bounds__(256) void check_kernel(
   __shared__ double sums[4][kChkSub];
   const int bx = blockIdx.x % gx, c = blockIdx.x / gx;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int i = bx * kChkRows + t;
+  constexpr int kRows = 256 * R;  // of a workgroup
+  const int i = bx * kRows + t;
   const int j0 = c * cc, j1 = min(n, j0 + cc);
-  uint64_t  s[kChkR];
-  double    acc[kChkR], aabs[kChkR];
-  bool      in[kChkR];
+  uint64_t  s[R];
+  double    acc[R], aabs[R];
+  bool      in[R];
 #pragma unroll
-  for(int q = 0; q < kChkR; ++q) {
+  for(int q = 0; q < R; ++q) {
     s[q] = lcg_state(seed, static_cast<uint64_t>(i + 256 * q) +
                                static_cast<uint64_t>(j0) * static_cast<uint64_t>(n));
     in[q]  = i + 256 * q < n;
@@ -162,17 +162,16 @@ __global__ __launch_bounds__(256) void check_kernel(
     __syncthreads();  // sx and sums are free again
     if(t < jn) sx[t] = X[js + t];
     __syncthreads();
-    const bool edge = (js < (bx + 1) * kChkRows && js + jn > bx * kChkRows) ||
-                      (bx + 1) * kChkRows > n;
+    const bool edge = (js < (bx + 1) * kRows && js + jn > bx * kRows) || (bx + 1) * kRows > n;
     for(int u0 = 0; u0 < jn; u0 += kChkStep) {
       const int un = min(kChkStep, jn - u0);
       for(int u = 0; u < un; ++u) {
         double sum;
         if(edge)
-          check_step<true>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
+          check_step<true, R>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
                            sum);
         else
-          check_step<false>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
+          check_step<false, R>(i, js + u0 + u, s, acc, aabs, sx[u0 + u], shift, colA, colC, in,
                             sum);
         tile[wave][u][lane] = sum;
       }
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(256) void check_kernel(
           (sums[0][t] + sums[1][t]) + (sums[2][t] + sums[3][t]);
   }
 #pragma unroll
-  for(int q = 0; q < kChkR; ++q)
+  for(int q = 0; q < R; ++q)
     if(in[q]) {
       part_r[static_cast<size_t>(c) * n + i + 256 * q] = acc[q];
       part_a[static_cast<size_t>(c) * n + i + 256 * q] = aabs[q];
@@ -391,20 +390,30 @@ hipError_t launch_matgen(hipStream_t s, int m, int n, __half* A, int lda,
   return matgen_t(s, m, n, A, lda, seed, diag_shift);
 }
 
-// Columns per chunk of the check: as many as leave 4096 workgroups, 4096 at
-// most (the partial sums of the rows are n x 2 per chunk).
-static int check_cols(int n) {
-  const long rows = (n + kChkRows - 1) / kChkRows;
-  int        cc   = 4096;
-  while(cc > kChkSub && rows * ((n + cc - 1) / cc) < 4096) cc /= 2;
-  return cc;
+// Rows of a workgroup and columns per chunk of the check: of the columns as many
+// as leave 4096 workgroups, 4096 at most (the partial sums of the rows are n x 2
+// per chunk).  Small matrices leave CUs idle all the same, and what counts is the
+// time of one workgroup: a row a thread and 32 columns (us for N = 64 / 100 / 500 /
+// 1000 / 2000: 4 rows and 256 columns 51 / 60 / 98 / 102 / 106, a row and 64 columns
+// 42 / 42 / 46 / 50 / 53, and 32 38 / 39 / 44 / 50 / 53; rows and columns summed by a
+// kernel each 39 / 43 / 73 / 109 / 180).
+struct CheckSplit {
+  int rows, cols;
+};
+static CheckSplit check_split(int n) {
+  const bool small = n <= 2048;
+  const int  r     = small ? 256 : 256 * kChkR;
+  const long rows  = (n + r - 1) / r;
+  int        cc    = 4096;
+  while(cc > (small ? 32 : kChkSub) && rows * ((n + cc - 1) / cc) < 4096) cc /= 2;
+  return {r, cc};
 }
 
 size_t check_part_len(int n) {
   if(n <= 0) return 16;
-  const int    cc    = check_cols(n);
-  const size_t nch_c = (n + cc - 1) / cc;
-  const size_t nch_r = (n + kChkRows - 1) / kChkRows;
+  const CheckSplit c = check_split(n);
+  const size_t nch_c = (n + c.cols - 1) / c.cols;
+  const size_t nch_r = (n + c.rows - 1) / c.rows;
   const size_t nblk  = (n + 255) / 256;
   return (2 * nch_c + nch_r) * static_cast<size_t>(n) + 8 + 8 * nblk + 16;
 }
@@ -414,9 +423,9 @@ hipError_t launch_check(hipStream_t s, int n, int seed, double diag_shift,
                         double* out_dev) {
   if(n <= 0) return hipErrorInvalidValue;
   if(part_len < check_part_len(n)) return hipErrorInvalidValue;
-  const int cc    = check_cols(n);
-  const int nch_c = (n + cc - 1) / cc;
-  const int nch_r = (n + kChkRows - 1) / kChkRows;
+  const CheckSplit c = check_split(n);
+  const int nch_c = (n + c.cols - 1) / c.cols;
+  const int nch_r = (n + c.rows - 1) / c.rows;
   const int nblk  = (n + 255) / 256;
   double* part_r = part;
   double* part_a = part_r + static_cast<size_t>(nch_c) * n;
@@ -424,9 +433,13 @@ hipError_t launch_check(hipStream_t s, int n, int seed, double diag_shift,
   double* bp     = part_c + static_cast<size_t>(nch_r) * n;
   const Affine colj = lcg_jump(static_cast<uint64_t>(n));
   const uint64_t sd = static_cast<uint64_t>(seed);
-  hipLaunchKernelGGL(check_kernel, dim3(static_cast<unsigned>(nch_r) * nch_c),
-                     dim3(256), 0, s, n, cc, sd, diag_shift, X, part_r, part_a, part_c,
-                     colj.a, colj.c, nch_r);
+  const dim3 g(static_cast<unsigned>(nch_r) * nch_c), b(256);
+  if(c.rows == 256)
+    hipLaunchKernelGGL(check_kernel<1>, g, b, 0, s, n, c.cols, sd, diag_shift, X, part_r,
+                       part_a, part_c, colj.a, colj.c, nch_r);
+  else
+    hipLaunchKernelGGL(check_kernel<kChkR>, g, b, 0, s, n, c.cols, sd, diag_shift, X, part_r,
+                       part_a, part_c, colj.a, colj.c, nch_r);
   hipLaunchKernelGGL(check_finish_kernel, dim3(nblk), dim3(256), 0, s, n,
                      nch_c, nch_r, sd, X, part_r, part_a, part_c, bp);
   hipLaunchKernelGGL(check_reduce_kernel, dim3(1), dim3(256), 0, s, n, nblk,
