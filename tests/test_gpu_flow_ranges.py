@@ -126,3 +126,30 @@ def test_passes_of_right_hand_sides(ctx, n, nb, cols):
                 assert np.abs(X - R).max() <= 4 * n * 2.0 ** -52 * np.abs(R).max()
     finally:
         ctx.pmat_free(mat)
+
+
+@pytest.mark.parametrize("n,nb,counts", [(4300, 32, (1, 9)), (8300, 64, (2,)),
+                                         (16500, 512, (1, 64)), (11000, 256, (88,))])
+def test_panels_and_chunks_prepared_more_than_once(ctx, n, nb, counts):
+    """More than 128 panels of at most 128 rows are prepared in several runs, and U
+    of more blocks than the exchange buffer holds (128 with few right-hand sides,
+    85 with 84 to 96) is solved in several chunks: the residual stays within n eps
+    of |A| |x| + |b| per row (A diagonally dominant)."""
+    shift = float(n)
+    A = o.matgen(n, n)
+    A[np.arange(n), np.arange(n)] += shift
+    norms = [np.abs(A).sum(1).max(), np.abs(A).sum(0).max()]
+    mat = ctx.pmat_alloc(n, nb)
+    try:
+        ctx.pdrandmat(n, n, nb, mat.A, mat.ld, rp.HPL_ISEED, shift)
+        assert ctx.pdgetrf(rp.palg_default(), mat) == 0
+        for nrhs in counts:
+            print("[gpu-case] getrs n=%d nb=%d nrhs=%d" % (n, nb, nrhs), flush=True)
+            B = np.random.default_rng(nrhs).standard_normal((n, nrhs))
+            for trans in (0, 1):
+                X = solve(ctx, mat, B, trans)
+                res = np.abs((A.T if trans else A) @ X - B).max()
+                assert res <= n * 2.0 ** -52 * (norms[trans] * np.abs(X).max() +
+                                                np.abs(B).max())
+    finally:
+        ctx.pmat_free(mat)
