@@ -236,7 +236,7 @@ int hplx_ctx_create(int device, hplx_ctx** out) {
     c.panel_kernel = v >= 0 && v <= 2 ? v : c.panel_kernel;
   }
   c.flow_polls = hplx::kFlowPolls;
-  if(const char* sp = std::getenv("HPLX_SOLVE_POLLS"))
+  if(const char* sp = std::getenv("HPLX_SOLVE_POLLS"); sp && *sp >= '0' && *sp <= '9')
     c.flow_polls = static_cast<uint32_t>(std::strtoul(sp, nullptr, 10));
   if(cu_sets(c, census) != HPLX_SUCCESS) return undo(HPLX_ERR_HIP);
   *out = ctx;
