@@ -58,7 +58,7 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 constexpr int kFB  = 128;  // rows of a block
 constexpr int kFH  = 64;   // and of its halves
-constexpr int kXcds = 8;
+constexpr int kXcdBits = 3;
 constexpr int kFLd = 66;   // LDS pitch of a right-hand side of a half
 constexpr int kNext = 1;   // blocks ahead in the chain that poll the values
 // Narrow slices (4 right-hand sides) while at most this many workgroups come
@@ -78,6 +78,7 @@ struct FlowArgs {
   int           o0, o1;  // rows of the others, updated only
   int           nd, nt;  // blocks on the diagonal, in all
   int           ns;      // slices of 16 right-hand sides
+  int           xcd_bits;  // 2^these XCDs take turns at the blocks
   unsigned long long* x;      // nd x ns blocks of 2 halves of 16 x 64 values
   int*                flags;  // nd x ns
   int*                err;    // FlowScratch's
@@ -300,16 +301,10 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
   // blocks in index order; the slices of a block on one XCD (they read the same
   // rows of T), unless the blocks are too few for all XCDs (N = 100 with
   // 1000 right-hand sides, one block: 144 us a call on one XCD, 44 spread)
-  int sl, i;
-  if(a.nt >= kXcds) {
-    const int per = kXcds * a.ns, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
-    sl = br / kXcds;
-    i  = bg * kXcds + br % kXcds;
-    if(i >= a.nt) return;
-  } else {
-    i  = blockIdx.x / a.ns;
-    sl = blockIdx.x - i * a.ns;
-  }
+  const int xb  = a.xcd_bits;
+  const int per = a.ns << xb, bg = blockIdx.x / per, br = blockIdx.x - bg * per;
+  const int sl = br >> xb, i = (bg << xb) + (br & ((1 << xb) - 1));
+  if(i >= a.nt) return;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int ac = P::col();  // this lane's right-hand side
@@ -382,13 +377,25 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     unsigned long long* xj = a.x + (static_cast<size_t>(2 * j + (st & 1)) * a.ns + sl) *
                                        (R * kFH) + kFH * wave + lane;
     unsigned long long  xv[W];
+    const bool          next = diag && j + kNext >= i;
+    // polls the values until all are there
+    auto poll = [&](bool in) {
+      for(uint32_t polls = 0; !in && !dead;) {
+#pragma unroll
+        for(int q = 0; q < W; ++q)
+          xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
+                                    __HIP_MEMORY_SCOPE_AGENT);
+        in = all_there(xv);
+        if(!in) dead = ++polls > a.polls;
+      }
+    };
     if(wave < R) {
-      bool     in    = false;
-      uint32_t polls = 0;
-      if(diag && j + kNext >= i) {
+      if(next) {
         __builtin_amdgcn_s_setprio(3);
+        poll(false);
       } else {
         const int* flag = a.flags + j * a.ns + sl;
+        uint32_t   polls = 0;
         while(!dead && !__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
           dead = ++polls > a.polls;
           __builtin_amdgcn_s_sleep(8);
@@ -398,22 +405,7 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         for(int q = 0; q < W; ++q)
           xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-        in    = all_there(xv);
-        polls = 0;
-      }
-      while(!in && !dead) {
-#pragma unroll
-        for(int q = 0; q < W; ++q)
-          xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT);
-        in = all_there(xv);
-        if(!in) dead = ++polls > a.polls;
-      }
-      if(dead) {
-        if(a.err && lane == 0)
-          __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-#pragma unroll
-        for(int q = 0; q < W; ++q) xv[q] = 0x7ff8000000000000ull;
+        if(WIDE) poll(all_there(xv));
       }
     }
     if(st + 1 < mine) {
@@ -422,6 +414,15 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     }
     double* x = xs[st & 1];
     if(wave < R) {
+      // narrow: checked only here, T's loads under way meanwhile (N = 16384, one
+      // right-hand side 1.58 against 1.60 ms; wide, 64 of them 2.74 against 2.72)
+      if(!WIDE && !next) poll(all_there(xv));
+      if(dead) {
+        if(a.err && lane == 0)
+          __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+        for(int q = 0; q < W; ++q) xv[q] = 0x7ff8000000000000ull;
+      }
 #pragma unroll
       for(int q = 0; q < W; ++q)
         x[(wave + 8 * q) * kFLd + lane] =
@@ -478,16 +479,12 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         double u[4];
         solve_half<TRANS, BACK>(a.T + r + static_cast<size_t>(r) * a.ldt, a.ldt, kFH * half,
                                 left, xc, u);
+        // past the block's rows nothing, whatever infinite values made of their
+        // zeros: the rows further on multiply them by zeros of T
         if((bad >> (lane & 48)) & 0xffff)
 #pragma unroll
-          for(int s = 0; s < 4; ++s) v[s] = u[s];
-      }
-      // past the block's rows nothing, whatever infinite values made of their
-      // zeros: the rows further on multiply them by zeros of T
-#pragma unroll
-      for(int s = 0; s < 4; ++s) {
-        const int q = BACK ? kFH - 1 - (16 * s + m) : 16 * s + m;
-        v[s]        = q < left ? v[s] : 0.0;
+          for(int s = 0; s < 4; ++s)
+            v[s] = (BACK ? kFH - 1 - (16 * s + m) : 16 * s + m) < left ? u[s] : 0.0;
       }
       unsigned long long* xi =
           a.x + (static_cast<size_t>(2 * i + h) * a.ns + sl) * (R * kFH) + c * kFH;
@@ -627,8 +624,8 @@ struct Flow {
     a.o1    = o1;
     a.nd    = (d1 - d0 + kFB - 1) / kFB;
     a.nt    = a.nd + (o1 - o0 + kFB - 1) / kFB;
-    const long grid = static_cast<long>(a.nt < kXcds ? a.nt : (a.nt + kXcds - 1) / kXcds * kXcds) *
-                      a.ns;
+    a.xcd_bits      = a.nt >> kXcdBits ? kXcdBits : 0;
+    const long grid = ((a.nt + (1L << a.xcd_bits) - 1) >> a.xcd_bits << a.xcd_bits) * a.ns;
     if(block + a.nd > blocks() || grid > 0x7fffffffL) return hipErrorInvalidValue;
     const dim3 g(static_cast<unsigned>(grid)), b(512);
     if(wide())
