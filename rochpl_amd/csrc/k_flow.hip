@@ -40,8 +40,8 @@
 // rather than 64-row ones: half the trips (that U 1115 us).
 //
 // hplx_pdgetrs, before and now: N = 16384, NB = 512, 64 right-hand sides 9.50
-// -> 2.69 ms (transposed 8.92 -> 3.46), one 9.27 -> 1.60, 512 15.2 -> 9.6;
-// N = 5000, NB = 128, one 2.87 -> 0.69 ms.  The floor is one read of the
+// -> 2.72 ms (transposed 8.92 -> 3.45), one 9.27 -> 1.58, 512 15.2 -> 8.0;
+// N = 5000, NB = 128, one 2.87 -> 0.70 ms.  The floor is one read of the
 // factors (2.1 GB, 0.4 ms).
 #include "hplx_internal.hpp"
 #include "lds_stream.hpp"
@@ -77,7 +77,7 @@ struct FlowArgs {
   int           d0, d1;  // rows of the diagonal blocks
   int           o0, o1;  // rows of the others, updated only
   int           nd, nt;  // blocks on the diagonal, in all
-  int           ns;      // slices of 16 right-hand sides
+  int           ns;      // slices of 16 or 4 right-hand sides
   int           xcd_bits;  // 2^these XCDs take turns at the blocks
   unsigned long long* x;      // nd x ns blocks of 2 halves of 16 x 64 values
   int*                flags;  // nd x ns

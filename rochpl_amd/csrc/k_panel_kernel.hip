@@ -193,9 +193,10 @@ hipError_t launch_panel_kernel(Ctx& c, int slot, double* P, int lda, int m,
   int G = c.panel_cus > 0 ? c.panel_cus : c.pk_resident;
   G     = G < c.pk_resident ? G : c.pk_resident;
   G     = G > gl ? G : gl;
-  // every product must be one that the streamed update takes too (aligned
-  // pairs, a multiple of 8 columns of A); the launch sequence falls back to
-  // the generic GEMM for the others
+  // every product must be one that the streamed update takes too.  gemm_tile
+  // itself needs only the aligned pairs of that; the rest (K a multiple of 8, U^T
+  // within the scratch buffer) decides, as HPLX_OPT_PANEL_KERNEL states it, which
+  // panels run as the launch sequence, which is the faster of the two
   const double* Bt = panel_scratch(c);
   for(const PanelOp& o : ops) {
     if(o.kind != kPanelGemm) continue;

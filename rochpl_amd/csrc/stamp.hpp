@@ -1,7 +1,8 @@
 // Times written by the kernels themselves: block 0 of a kernel notes when it
 // starts, which in stream order is also when what came before it has ended.
 // Two records of an event cost the stream 9 us between two kernels, an event
-// carried by a kernel's own dispatch 7, this nothing.
+// carried by a kernel's own dispatch 7, this nothing; where no kernel carries a
+// time, launch_stamp's one thread does (2.3 us).
 #pragma once
 
 #include <hip/hip_runtime.h>

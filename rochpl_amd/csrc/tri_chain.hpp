@@ -9,6 +9,9 @@
 // 0.7 us; with the broadcasts as lane shuffles and one right-hand side a wave
 // it was four times that for each.
 //
+// The triangle's zeros take part: a solved value that is exactly -0 may become +0
+// (no other value changes, and what is not finite is solved again without them).
+//
 // "Positions" are rows in the order they are solved (from the last row for a
 // backward solve).
 #pragma once

@@ -1,5 +1,5 @@
 """The residual check's one pass at the edges of its row blocks (1024), column
-chunks (256) and steps (16), against NumPy on the same matrix."""
+chunks (256) and steps (8), against NumPy on the same matrix."""
 import numpy as np
 import pytest
 
