@@ -78,30 +78,15 @@ __global__ __launch_bounds__(256) void check_rows_kernel(
   __syncthreads();
   const int i = bx * 256 + threadIdx.x;
   if(i >= n) return;
-  // four columns' states at a time: the chain of dependent products is a
-  // quarter as long; the sums keep their order
-  uint64_t s[4], a4 = colA, c4 = colC;
-  s[0] = lcg_state(seed, static_cast<uint64_t>(i) +
-                             static_cast<uint64_t>(j0) * static_cast<uint64_t>(n));
-#pragma unroll
-  for(int q = 1; q < 4; ++q) s[q] = colA * s[q - 1] + colC;
-#pragma unroll
-  for(int q = 0; q < 2; ++q) {  // the map of four columns
-    c4 = a4 * c4 + c4;
-    a4 = a4 * a4;
-  }
+  uint64_t s = lcg_state(seed, static_cast<uint64_t>(i) +
+                                   static_cast<uint64_t>(j0) * static_cast<uint64_t>(n));
   double acc = 0.0, aabs = 0.0;
-  for(int t0 = 0; t0 < jn; t0 += 4) {
-#pragma unroll
-    for(int q = 0; q < 4; ++q) {
-      if(t0 + q < jn) {
-        double v = lcg_value(s[q]);
-        if(i == j0 + t0 + q) v += shift;
-        acc = fma(v, sx[t0 + q], acc);
-        aabs += fabs(v);
-      }
-      s[q] = a4 * s[q] + c4;
-    }
+  for(int t = 0; t < jn; ++t) {
+    double v = lcg_value(s);
+    if(i == j0 + t) v += shift;
+    acc  = fma(v, sx[t], acc);
+    aabs += fabs(v);
+    s = colA * s + colC;
   }
   part_r[static_cast<size_t>(c) * n + i] = acc;
   part_a[static_cast<size_t>(c) * n + i] = aabs;
