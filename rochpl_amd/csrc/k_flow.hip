@@ -40,7 +40,7 @@
 // rather than 64-row ones: half the trips (that U 1115 us).
 //
 // hplx_pdgetrs, before and now: N = 16384, NB = 512, 64 right-hand sides 9.50
-// -> 2.72 ms (transposed 8.92 -> 3.45), one 9.27 -> 1.58, 512 15.2 -> 8.0;
+// -> 2.70 ms (transposed 8.92 -> 3.45), one 9.27 -> 1.58, 512 15.2 -> 8.0;
 // N = 5000, NB = 128, one 2.87 -> 0.70 ms.  The floor is one read of the
 // factors (2.1 GB, 0.4 ms).
 #include "hplx_internal.hpp"
@@ -379,7 +379,8 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     unsigned long long  xv[W];
     const bool          next = diag && j + kNext >= i;
     // polls the values until all are there
-    auto poll = [&](bool in) {
+    auto poll = [&]() {
+      bool in = false;
       for(uint32_t polls = 0; !in && !dead;) {
 #pragma unroll
         for(int q = 0; q < W; ++q)
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     if(wave < R) {
       if(next) {
         __builtin_amdgcn_s_setprio(3);
-        poll(false);
+        poll();
       } else {
         const int* flag = a.flags + j * a.ns + sl;
         uint32_t   polls = 0;
@@ -405,7 +406,6 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
         for(int q = 0; q < W; ++q)
           xv[q] = __hip_atomic_load(xj + 8 * kFH * q, __ATOMIC_RELAXED,
                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-        if(WIDE) poll(all_there(xv));
       }
     }
     if(st + 1 < mine) {
@@ -414,19 +414,26 @@ __global__ __launch_bounds__(512) void flow_kernel(FlowArgs a) {
     }
     double* x = xs[st & 1];
     if(wave < R) {
-      // narrow: checked only here, T's loads under way meanwhile (N = 16384, one
-      // right-hand side 1.58 against 1.60 ms; wide, 64 of them 2.74 against 2.72)
-      if(!WIDE && !next) poll(all_there(xv));
+      auto put = [&]() {
+#pragma unroll
+        for(int q = 0; q < W; ++q)
+          x[(wave + 8 * q) * kFLd + lane] =
+              -__longlong_as_double(static_cast<long long>(xv[q]));
+      };
+      put();
+      // what was read after a flag is checked only now, out of the loads' way (N =
+      // 16384, 64 right-hand sides 2.73 ms checked before T's loads, 2.71 so)
+      if(!next && !all_there(xv)) {
+        poll();
+        put();
+      }
       if(dead) {
         if(a.err && lane == 0)
           __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 #pragma unroll
         for(int q = 0; q < W; ++q) xv[q] = 0x7ff8000000000000ull;
+        put();
       }
-#pragma unroll
-      for(int q = 0; q < W; ++q)
-        x[(wave + 8 * q) * kFLd + lane] =
-            -__longlong_as_double(static_cast<long long>(xv[q]));
     }
     __syncthreads();  // this buffer is written again two barriers on
     // a half's sum is formed by itself: N / 64 roundings at the magnitude of
